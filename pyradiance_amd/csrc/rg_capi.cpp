@@ -445,8 +445,8 @@ static void run(rg_ctx* c, const double* rays, long long nrays, int accum, int f
     sc_ctx.push_back(c);
     sc_dev.push_back(&Sd);
   }
-  // The call block, cleared once and read back once: rays traced (u64),
-  // error flags (u32), then per scene with a shadow cache the closest-hit
+  // The call block, cleared once and read back once: error flags (u32, at
+  // byte 8), then per scene with a shadow cache the closest-hit
   // queries of its cast rays per source (u64, when this call fills the
   // cache: the first call after a commit, as the reference fills a source's
   // cache at its first shadow test) and its tested-source flags (u32).
@@ -503,7 +503,6 @@ static void run(rg_ctx* c, const double* rays, long long nrays, int accum, int f
   // rcontrib coefficients (not -V values, nor rtrace radiances, whose range
   // the host cannot bound) accumulate in fixed point
   cfg.fix = (mode == 1 && !c->params.contrib && !adj) ? fixed_scale(accum) : 0.0;
-  cfg.nrays = (unsigned long long*)d_blk;
   cfg.err = (uint32_t*)(d_blk + 8);
   cfg.accum = accum;
   cfg.child_order = c->tuning.child_order;
@@ -584,7 +583,7 @@ static void run(rg_ctx* c, const double* rays, long long nrays, int accum, int f
           "grad");
   hipck(hipStreamSynchronize(c->st), "render");
   uint32_t herr = 0;
-  memcpy(&c->last_nrays, h, 8);
+  c->last_nrays = c->last_stats.rays;
   memcpy(&herr, h + 8, 4);
   for (size_t i = 0; i < nsc; ++i) {
     rg_ctx* bc = sc_ctx[i];

@@ -1,12 +1,21 @@
 // Wavefront renderer for the rtrace / rcontrib ray tree on CDNA4 (gfx950).
 //
-// One fused kernel per generation of the tree: each thread takes one child of
-// a spawn record (binary search over the exclusive scan of child counts),
-// applies the spawn rules of rayorigin() (rt/raytrace.c:40-135), walks the BVH
-// for the closest hit, shades the hit and appends the spawn records of the
-// next generation.  Spawn records are allocated with one atomic per wavefront
-// (ballot + mbcnt), emission is added into the sensor's output with FP64
-// atomics.  The BVH stack lives in LDS, column-major per lane.
+// The tree is walked breadth-first in windows.  A window's rays are traced to
+// their closest hits (k_trace_pf) and shaded (k_shade); shading appends the
+// next generation: single rays, already built and admitted by the rules of
+// rayorigin() (rt/raytrace.c:40-135), and hemisphere records, whose children
+// k_hemi_rays builds when their turn comes.  Emission is added into the
+// sensor's output with integer or FP64 atomics.  The walk's stack lives in
+// LDS, column-major per lane.
+//
+// Appending: atomics on one address complete one after the other, 11.4 ns
+// each over the whole chip (measured; 0.08 ns over 256 addresses), so a
+// counter that every wavefront bumps once costs more than the work of the
+// wavefront: with one spawn counter k_shade took 14.3 ms for the 1.3 M
+// wavefronts of a 2,500-sensor pass, 14.9 ms of it queueing there.  Rays are
+// therefore appended to kRaySegs segments with a counter each (a block's
+// segment is its index modulo their number), and every other per-wavefront
+// counter is kept in registers or taken in large bites.
 #include <hip/hip_runtime.h>
 #include "rg_shade.hpp"
 #include "rg_render.hpp"
@@ -36,35 +45,114 @@ __device__ __forceinline__ uint32_t wave_alloc(uint32_t* ctr) {
   base = __shfl(base, leader);
   return base + lane_rank(m);
 }
-__device__ __forceinline__ void wave_count(unsigned long long* ctr) {
-  unsigned long long m = __ballot(1);
-  uint32_t leader = __ffsll((long long)m) - 1;
-  if (__lane_id() == leader) atomicAdd(ctr, (unsigned long long)__popcll(m));
-}
-
-struct Sink {
-  Spawn* buf;
-  uint32_t* count;
-  uint32_t cap;
-  uint32_t* err;
-  PathRec* pbuf;       // adjoint replay: path record of each spawn (else null)
-  uint32_t* counts;    // child count of each spawn, compact (the scan's input)
+// Rays of a batch live in segments of `segcap` records (a power of two of
+// segments, at most kRaySegs).  They are handed out in chunks of kChunk
+// consecutive rays of one segment: chunk q is tile q / nseg of segment
+// q % nseg, so consecutive chunks cover the segments evenly.  Rays of chunk
+// chunk0 + k have window indices [kChunk k, kChunk k + count).
+constexpr uint32_t kRaySegs = 64;
+constexpr uint32_t kChunkLog = 8;
+constexpr uint32_t kChunk = 1u << kChunkLog;
+struct RayMap {
+  const uint32_t* cnt;   // rays in each segment
+  uint32_t seg_log;      // log2 of the segment count
+  uint32_t segcap;
+  uint32_t chunk0;       // first chunk of this window
+  uint32_t nchunk;       // chunks in this window
+  // chunk k of the window: its first ray's record index and its ray count
+  __device__ __forceinline__ uint32_t chunk(uint32_t k, uint32_t& n) const {
+    const uint32_t q = chunk0 + k, seg = q & ((1u << seg_log) - 1u), at = (q >> seg_log) << kChunkLog;
+    const uint32_t have = cnt[seg];
+    n = have > at ? min(have - at, kChunk) : 0u;
+    return seg * segcap + at;
+  }
 };
 
-// Append a spawn; in adjoint replay also its path: the parent's plus `entry`
-// (none: the parent's vertex is not a differentiated one).
-__device__ __forceinline__ void emit(const Sink& sk, const Spawn& s, const RayS& r, const PathAdd& entry) {
-  uint32_t i = wave_alloc(sk.count);
-  if (i < sk.cap) {
-    sk.buf[i] = s;
-    sk.counts[i] = s.count;
-    if (sk.pbuf) sk.pbuf[i] = path_push(r.path, entry);
-  } else {
-    atomicOr(sk.err, ERR_CAPACITY);
-  }
+// Counters of a launch under way, each on its own 128-byte line: the fill of
+// every output segment, the hemisphere records and their children, and the
+// walk's next unit of work.  k_window_done copies them out and clears them.
+constexpr uint32_t kCtrStride = 32;     // 32-bit words
+enum : uint32_t { CTR_HEMI = kRaySegs, CTR_KIDS = kRaySegs + 1, CTR_WORK = kRaySegs + 2, CTR_COUNT = kRaySegs + 3 };
+constexpr uint32_t kCtrWords = CTR_COUNT * kCtrStride;
+
+// Where a launch appends.  pbuf / hpath: path records (adjoint replay, else null).
+struct Sink {
+  RayGeo* geo;
+  RaySt* st;
+  PathRec* pbuf;
+  uint32_t seg_log;    // log2 of the output segments
+  uint32_t segcap;
+  const uint32_t* have;   // rays the segments already hold (null: none)
+  Spawn* hemi;
+  uint32_t* hcount;    // children of each hemisphere record (the scan's input)
+  PathRec* hpath;
+  uint32_t hcap;
+  uint32_t* ctr;       // kCtrWords
+  uint32_t* err;
+};
+
+__device__ __forceinline__ void put_ray_at(const Sink& sk, const RayS& r, size_t at) {
+  RayGeo g;
+  g.o[0] = r.o.x; g.o[1] = r.o.y; g.o[2] = r.o.z;
+  g.d[0] = r.d.x; g.d[1] = r.d.y; g.d[2] = r.d.z;
+  RaySt q;
+  q.key = r.key;
+  q.coef[0] = r.coef.r; q.coef[1] = r.coef.g; q.coef[2] = r.coef.b;
+  q.w = r.w;
+  q.crc = r.crc;
+  q.sensor = r.sensor;
+  q.crtype = r.crtype;
+  q.rsrc = (int16_t)r.rsrc;
+  q.rlvl = (uint8_t)r.rlvl;
+  q.adepth = (uint8_t)r.adepth;
+  q.scene = (uint16_t)r.scene;
+  q.pad[0] = q.pad[1] = 0u;
+  sk.geo[at] = g;
+  sk.st[at] = q;
+  if (sk.pbuf) sk.pbuf[at] = r.path;
 }
 
-__device__ __forceinline__ void emit(const Sink& sk, const Spawn& s, const RayS& r) { emit(sk, s, r, path_none()); }
+// Appends one ray to this block's segment.
+__device__ __forceinline__ void put_ray(const Sink& sk, const RayS& r) {
+  const uint32_t seg = blockIdx.x & ((1u << sk.seg_log) - 1u);
+  const uint32_t i = wave_alloc(sk.ctr + seg * kCtrStride) + (sk.have ? sk.have[seg] : 0u);
+  if (i >= sk.segcap) { atomicOr(sk.err, ERR_CAPACITY); return; }
+  put_ray_at(sk, r, (size_t)seg * sk.segcap + i);
+}
+
+// Appends a hemisphere of several children.
+__device__ __forceinline__ void put_hemi(const Sink& sk, const Spawn& s, const RayS& r, const PathAdd& entry) {
+  unsigned long long kids = s.count;
+  const unsigned long long m = __ballot(1);
+  // children of the wavefront's active lanes, summed by the first of them
+  const uint32_t leader = __ffsll((long long)m) - 1;
+  unsigned long long sum = 0;
+  for (unsigned long long q = m; q; q &= q - 1) sum += __shfl(kids, __ffsll((long long)q) - 1);
+  if (__lane_id() == leader) atomicAdd((unsigned long long*)(sk.ctr + CTR_KIDS * kCtrStride), sum);
+  const uint32_t i = wave_alloc(sk.ctr + CTR_HEMI * kCtrStride);
+  if (i >= sk.hcap) { atomicOr(sk.err, ERR_CAPACITY); return; }
+  sk.hemi[i] = s;
+  sk.hcount[i] = s.count;
+  if (sk.hpath) sk.hpath[i] = path_push(r.path, entry);
+}
+
+__device__ __forceinline__ bool build_ray(const RunCfg& c, const Spawn& sp, uint32_t ci, RayS& r,
+                                          const PathRec* pp = nullptr);
+
+// The single child of spawn s (an explicit ray, or a hemisphere of one
+// stratum), built and, when admitted, appended; in adjoint replay with its
+// path: the parent's plus `entry` (none: the parent's vertex is not a
+// differentiated one).
+__device__ __forceinline__ void emit(const Sink& sk, const RunCfg& c, const Spawn& s, const RayS& r,
+                                     const PathAdd& entry) {
+  RayS ch;
+  PathRec path;
+  if (c.adj) path = path_push(r.path, entry);
+  if (build_ray(c, s, 0u, ch, &path)) put_ray(sk, ch);
+}
+__device__ __forceinline__ void emit(const Sink& sk, const RunCfg& c, const Spawn& s, const RayS& r) {
+  emit(sk, c, s, r, path_none());
+}
 
 // Bin accumulation.  With c.fix > 0 each channel is rounded to a multiple
 // of 1 / c.fix and added as a 64-bit integer: integer sums do not depend on
@@ -835,9 +923,9 @@ __device__ __forceinline__ void direct_light(const DevScene& S, const RunCfg& c,
       e.w[1] = __float_as_uint((float)parts.a);
       e.w[2] = __float_as_uint((float)parts.b);
       e.w[3] = __float_as_uint((float)parts.g);
-      emit(sk, s, r, e);
+      emit(sk, c, s, r, e);
     } else {
-      emit(sk, s, r);
+      emit(sk, c, s, r);
     }
   }
 }
@@ -872,7 +960,8 @@ __device__ __forceinline__ void ambient(const DevScene& S, const RunCfg& c, cons
       s.ns = (uint16_t)n;
       s.count = (uint32_t)n * (uint32_t)n;
       s.adepth = (uint8_t)(r.adepth + 1);
-      emit(sk, s, r, entry);
+      if (n == 1) emit(sk, c, s, r, entry);
+      else put_hemi(sk, s, r, entry);
       return;
     }
   }
@@ -920,9 +1009,9 @@ __device__ __forceinline__ void gauss_sample(const DevScene& S, const RunCfg& c,
       if (mi >= 0) {
         PathAdd e = path_entry(mi, PV_GSPEC, 0.0);
         e.w[1] = __float_as_uint((float)score);
-        emit(sk, s, r, e);
+        emit(sk, c, s, r, e);
       } else {
-        emit(sk, s, r);
+        emit(sk, c, s, r);
       }
     }
   }
@@ -950,9 +1039,9 @@ __device__ __forceinline__ void gauss_sample(const DevScene& S, const RunCfg& c,
       if (mi >= 0) {
         PathAdd e = path_entry(mi, PV_GTRANS, 0.0);
         e.w[1] = __float_as_uint((float)score);
-        emit(sk, s, r, e);
+        emit(sk, c, s, r, e);
       } else {
-        emit(sk, s, r);
+        emit(sk, c, s, r);
       }
     }
   }
@@ -967,7 +1056,7 @@ __device__ __forceinline__ void shade_normal(const DevScene& S, const RunCfg& c,
     if (!c.p.backvis) {
       Spawn s = make_child(r, hs.rop, TRANS, nullptr, SLOT_PASS, SPF_FORCE);
       set_dir(s, r.d);
-      emit(sk, s, r);
+      emit(sk, c, s, r);
       return;
     }
     flip_surface(hs);
@@ -1019,7 +1108,7 @@ __device__ __forceinline__ void shade_normal(const DevScene& S, const RunCfg& c,
     C3 tc = nd.mcolor * nd.tspec;
     Spawn s = make_child(r, hs.rop, TRANS, &tc, SLOT_TRANS, 0);
     set_dir(s, nd.prdir);
-    emit(sk, s, r, dv ? path_entry(mi, PV_TSPEC, fest) : path_none());
+    emit(sk, c, s, r, dv ? path_entry(mi, PV_TSPEC, fest) : path_none());
   }
   if (r.crtype & SHADOW) return;
   nd.scolor = c3(0, 0, 0);
@@ -1042,10 +1131,11 @@ __device__ __forceinline__ void shade_normal(const DevScene& S, const RunCfg& c,
     if (hastexture && dot(dir, hs.ron) <= FTINY) dir = r.d + hs.ron * (2. * hs.rod);   // penetration
     normalize(dir);
     set_dir(s, dir);
-    emit(sk, s, r, dv ? path_entry(mi, PV_SPEC, fest) : path_none());
+    emit(sk, c, s, r, dv ? path_entry(mi, PV_SPEC, fest) : path_none());
   }
   if ((nd.specfl & SP_PURE) && nd.rdiff <= FTINY && nd.tdiff <= FTINY) return;
   if (!(nd.specfl & SP_PURE)) gauss_sample(S, c, r, hs, nd, sk, dv ? mi : -1);
+  direct_light(S, c, r, hs, nd, sk, dv ? mi : -1, fest);
   if (nd.rdiff > FTINY) {
     C3 a = nd.mcolor * nd.rdiff;
     if (nd.specfl & SP_RBLT) a = a + nd.scolor;
@@ -1057,7 +1147,6 @@ __device__ __forceinline__ void shade_normal(const DevScene& S, const RunCfg& c,
     ambient(S, c, r, hs, a, -nd.pnorm, sk,
             dv ? path_entry(mi, (nd.specfl & SP_TBLT) ? PV_AMB_BACK_TBLT : PV_AMB_BACK, fest) : path_none());
   }
-  direct_light(S, c, r, hs, nd, sk, dv ? mi : -1, fest);
 }
 
 // m_glass() of rt/glass.c:46-165
@@ -1066,7 +1155,7 @@ __device__ __forceinline__ void shade_glass(const RunCfg& c, const RayS& r, HitS
   if (!c.p.backvis && hs.rod <= 0.0) {
     Spawn s = make_child(r, hs.rop, TRANS, nullptr, SLOT_PASS, SPF_FORCE);
     set_dir(s, r.d);
-    emit(sk, s, r);
+    emit(sk, c, s, r);
     return;
   }
   double mc[3] = {m.f[0], m.f[1], m.f[2]};
@@ -1102,7 +1191,7 @@ __device__ __forceinline__ void shade_glass(const RunCfg& c, const RayS& r, HitS
       if (dot(pd, pd) > 0.0) { normalize(pd); td = pd; }
     }
     set_dir(s, td);
-    emit(sk, s, r);
+    emit(sk, c, s, r);
   }
   if (r.crtype & SHADOW) return;
   double cr[3];
@@ -1117,7 +1206,7 @@ __device__ __forceinline__ void shade_glass(const RunCfg& c, const RayS& r, HitS
   V3 dir = r.d + pnorm * (2. * pdot);
   normalize(dir);
   set_dir(s, dir);
-  emit(sk, s, r);
+  emit(sk, c, s, r);
 }
 
 // rayshade() for a surface hit, followed by rcontrib's trace callback.
@@ -1133,52 +1222,51 @@ __device__ __forceinline__ void shade_hit(const DevScene& S, const RunCfg& c, co
   hs.flat = P.flat & PF_FLAT;
   hs.phong = prim_phong_k(S, P.kind, P.goff);
   if (P.mat < 0) { atomicOr(c.err, ERR_NOMAT); return; }
+  // What the surface does is settled first, so that each material function
+  // has one call site (three copies of them took 234 registers).
+  enum { NOTHING, PASS, NORMAL, GLASS } act = NOTHING;
+  int mi = P.mat;                  // material that shades, and its index when it may be differentiated
+  int dmi = -1;
   const Material& m = S.mats[P.mat];
   bool zeroed = false;
   C3 rcol = c3(0, 0, 0);
   // -i: Lambertian replacement at the first qualifying surface (raytirrad)
-  bool tst_irrad = c.irrad && !(r.crtype & ~(PRIMARY | TRANS));
+  const bool tst_irrad = c.irrad && !(r.crtype & ~(PRIMARY | TRANS));
   if (tst_irrad && m.kind != MK_LIGHT && m.kind != MK_GLOW && m.kind != MK_ILLUM) {
-    if (m.transp) {
-      Spawn s = make_child(r, hs.rop, TRANS, nullptr, SLOT_PASS, SPF_FORCE);
-      set_dir(s, r.d);
-      emit(sk, s, r);
-    } else {
-      shade_normal(S, c, r, hs, S.mats[S.lamb], -1, sk);
-    }
-  } else {
-    switch (m.kind) {
-      case MK_PLASTIC:
-      case MK_METAL:
-      case MK_TRANS:
-        shade_normal(S, c, r, hs, m, P.mat, sk);
-        break;
-      case MK_GLASS:
-        shade_glass(c, r, hs, m, sk);
-        break;
-      default: {   // light, glow, illum
-        C3 em = c3(0, 0, 0);
-        bool pass;
-        if (!light_rules(S, c, r, m, h.prim, hs.rot, hs.rod, &em, &pass)) {
-          zeroed = true;
-        } else if (pass) {
-          if (m.kind == MK_ILLUM && m.illum_alt >= 0) {
-            const Material& alt = S.mats[m.illum_alt];
-            if (alt.kind == MK_GLASS) shade_glass(c, r, hs, alt, sk);
-            else if (alt.kind <= MK_TRANS) shade_normal(S, c, r, hs, alt, -1, sk);
-          } else {
-            Spawn s = make_child(r, hs.rop, TRANS, nullptr, SLOT_PASS, SPF_FORCE);
-            set_dir(s, r.d);
-            emit(sk, s, r);
-          }
-        } else {
-          rcol = em;
-          if (c.mode == 0) deposit(c, r.sensor, 0, r.coef * em);
-        }
+    act = m.transp ? PASS : NORMAL;
+    mi = S.lamb;
+  } else if (m.kind <= MK_TRANS) {
+    act = NORMAL;
+    dmi = P.mat;
+  } else if (m.kind == MK_GLASS) {
+    act = GLASS;
+  } else {   // light, glow, illum
+    C3 em = c3(0, 0, 0);
+    bool pass;
+    if (!light_rules(S, c, r, m, h.prim, hs.rot, hs.rod, &em, &pass)) {
+      zeroed = true;
+    } else if (pass) {
+      act = PASS;
+      if (m.kind == MK_ILLUM && m.illum_alt >= 0) {
+        mi = m.illum_alt;
+        const int ak = S.mats[mi].kind;
+        act = ak == MK_GLASS ? GLASS : (ak <= MK_TRANS ? NORMAL : NOTHING);
       }
+    } else {
+      rcol = em;
+      if (c.mode == 0) deposit(c, r.sensor, 0, r.coef * em);
     }
   }
   trace_contrib(S, c, r, P.modslot, h.prim, zeroed, rcol);
+  if (act == NORMAL) {
+    shade_normal(S, c, r, hs, S.mats[mi], dmi, sk);
+  } else if (act == GLASS) {
+    shade_glass(c, r, hs, S.mats[mi], sk);
+  } else if (act == PASS) {
+    Spawn s = make_child(r, hs.rop, TRANS, nullptr, SLOT_PASS, SPF_FORCE);
+    set_dir(s, r.d);
+    emit(sk, c, s, r);
+  }
 }
 
 // A ray that hit nothing: distant sources (sourcehit + m_light).
@@ -1223,7 +1311,7 @@ __global__ void __launch_bounds__(BLOCK) k_irrad_seed(DevScene Sarg, RunCfg c, c
   uint32_t i = blockIdx.x * BLOCK + threadIdx.x;
   if (i >= nsens) return;
   c.adj = ADJ;
-  if (!ADJ) sk.pbuf = nullptr;
+  if (!ADJ) { sk.pbuf = nullptr; sk.hpath = nullptr; }
   const int scene = scene_of_ray(c, s0 + i);
   const DevScene& S = scene_of(Sarg, c, scene);
   const double* ry = rays + 6 * (size_t)i;
@@ -1263,11 +1351,15 @@ __global__ void __launch_bounds__(BLOCK) k_irrad_seed(DevScene Sarg, RunCfg c, c
   shade_normal(S, c, r, hs, S.mats[S.lamb], -1, sk);
 }
 
-// Generation 0 for radiance rays: primary rays as explicit spawns.
+// Generation 0 for radiance rays: the primary rays, one segment in input order.
+template <bool ADJ>
 __global__ void __launch_bounds__(BLOCK) k_primary_seed(RunCfg c, const double* rays, uint32_t nsens, uint32_t s0,
-                                                        Spawn* out, uint32_t* counts) {
+                                                        Sink sk) {
   uint32_t i = blockIdx.x * BLOCK + threadIdx.x;
   if (i >= nsens) return;
+  c.adj = ADJ;
+  if (!ADJ) { sk.pbuf = nullptr; sk.hpath = nullptr; }
+  if (i == 0) sk.ctr[0] = nsens;
   const double* ry = rays + 6 * (size_t)i;
   V3 dir = load3(ry + 3);
   normalize(dir);
@@ -1289,19 +1381,14 @@ __global__ void __launch_bounds__(BLOCK) k_primary_seed(RunCfg c, const double* 
   const int scene = scene_of_ray(c, s0 + i);
   s.scene = (uint16_t)scene;
   s.key = sensor_key(c.p.seed + scene, s0 + i - (c.nscenes ? c.scene_start[scene] : 0));
-  out[i] = s;
-  counts[i] = 1u;
-}
-
-__global__ void __launch_bounds__(BLOCK) k_counts(const Spawn* sp, uint32_t n, uint32_t* counts) {
-  uint32_t i = blockIdx.x * BLOCK + threadIdx.x;
-  if (i < n) counts[i] = sp[i].count;
+  RayS r;
+  build_ray(c, s, 0u, r);          // a primary ray is always admitted
+  put_ray_at(sk, r, i);
 }
 
 // Child ci of spawn record sp: origin, direction and rayorigin() admission.
 // pp: the spawn's path record in adjoint replay (null otherwise).
-__device__ __forceinline__ bool build_ray(const RunCfg& c, const Spawn& sp, uint32_t ci, RayS& r,
-                                          const PathRec* pp = nullptr) {
+__device__ __forceinline__ bool build_ray(const RunCfg& c, const Spawn& sp, uint32_t ci, RayS& r, const PathRec* pp) {
   if (c.adj) r.path = pp ? *pp : PathRec{};
   r.o = v3(sp.org[0], sp.org[1], sp.org[2]);
   r.coef = c3(sp.coef[0], sp.coef[1], sp.coef[2]);
@@ -1360,67 +1447,22 @@ __device__ __forceinline__ uint32_t find_spawn(const uint64_t* offs, uint32_t ns
   return lo;
 }
 
-// Spawn record si and its first child index, requested together and waited
-// for together (the empty asm statement takes the loaded vectors as inputs,
-// which keeps the compiler from splitting the record's fields over several
-// round trips at their first uses).
-__device__ __forceinline__ void load_spawn(const Spawn* in, const uint64_t* offs, uint32_t si, Spawn& sp,
-                                           uint64_t& off) {
-  static_assert(sizeof(Spawn) == 6 * sizeof(u32x4), "Spawn layout");
-  const u32x4* spp = reinterpret_cast<const u32x4*>(in + si);
-  const u32x4 s0 = spp[0], s1 = spp[1], s2 = spp[2], s3 = spp[3], s4 = spp[4], s5 = spp[5];
-  off = offs[si];
-  asm volatile("" :: "v"(s0), "v"(s1), "v"(s2), "v"(s3), "v"(s4), "v"(s5), "v"(off));
-  const u32x4 sv[6] = {s0, s1, s2, s3, s4, s5};
-  __builtin_memcpy(&sp, sv, sizeof sp);
-}
-
-// Spawn of the first child of every 64-child chunk of a window [c0, c0 +
-// nth), and at index nchunk the spawn of the window's last child: one search
-// per chunk, all in parallel, ahead of the walk.  The walk's refill then
-// finds a child's spawn between its chunk's two entries (usually the same
-// record) instead of searching the whole scan from a single lane, a chain of
-// about log2(nspawn) dependent loads that every lane of the wavefront waited
-// for.
-constexpr uint32_t CHUNK_LOG = 6;
-__global__ void __launch_bounds__(BLOCK) k_chunk_spawn(const uint64_t* offs, uint32_t nspawn, uint64_t c0, uint32_t nth,
-                                                       uint32_t* first) {
-  const uint32_t k = blockIdx.x * BLOCK + threadIdx.x;
-  const uint32_t nch = (nth + (1u << CHUNK_LOG) - 1) >> CHUNK_LOG;
-  if (k > nch) return;
-  const uint64_t gid = c0 + (k < nch ? (uint64_t)k << CHUNK_LOG : (uint64_t)nth - 1);
-  first[k] = find_spawn(offs, nspawn, gid);
-}
-
-// Traversal result of one child ray (prim -2: not traced).
-struct alignas(16) TraceOut {
-  double t;
-  int32_t prim;
-  float dx, dy, dz;
-  uint32_t spawn;
-  uint32_t pad;
-};
-
-// One generation, part 1: children [c0, c0+nthreads) of `in` -> closest hits.
-#ifndef RG_TRACE_WAVES
-#define RG_TRACE_WAVES 4     // waves per SIMD the register budget of k_trace targets
-#endif
-__global__ void __launch_bounds__(TBLOCK) __attribute__((amdgpu_waves_per_eu(RG_TRACE_WAVES)))
-k_trace(DevScene Sarg, RunCfg c, const Spawn* in, const uint64_t* offs, uint32_t nspawn, uint64_t c0,
-        uint32_t nthreads, TraceOut* outp) {
-  __shared__ int32_t stk[LSTACK * TBLOCK];
-  __shared__ float stn[LSTACK * TBLOCK];
-  __shared__ float tes[NBIG_ORDER * TBLOCK];
-  uint32_t t = blockIdx.x * TBLOCK + threadIdx.x;
-  if (t >= nthreads) return;
-  c.adj = 0;      // admission does not depend on the path record
-  uint64_t gid = c0 + t;
-  // The wavefront's children are consecutive: one lane searches the whole
-  // table for the first child, the others only the few records after it
-  // (every record has at least one child).
-  unsigned long long act = __ballot(1);
-  uint32_t leader = __ffsll((long long)act) - 1;
-  uint64_t gid0 = __shfl(gid, leader);
+// Children [c0, c0 + nth) of a batch of hemisphere records, built and, when
+// admitted, appended as rays.  A wavefront's children are consecutive: one
+// lane searches the whole scan for the first child's record, the others only
+// the few records after it (every record has at least one child).
+template <bool ADJ>
+__global__ void __launch_bounds__(BLOCK) k_hemi_rays(RunCfg c, const Spawn* in, const PathRec* pin,
+                                                     const uint64_t* offs, uint32_t nspawn, uint64_t c0, uint32_t nth,
+                                                     Sink sk) {
+  const uint32_t t = blockIdx.x * BLOCK + threadIdx.x;
+  if (t >= nth) return;
+  c.adj = ADJ;
+  if (!ADJ) sk.pbuf = nullptr;
+  const uint64_t gid = c0 + t;
+  const unsigned long long act = __ballot(1);
+  const uint32_t leader = __ffsll((long long)act) - 1;
+  const uint64_t gid0 = __shfl(gid, leader);
   uint32_t base = 0;
   if (__lane_id() == leader) base = find_spawn(offs, nspawn, gid0);
   base = __shfl(base, leader);
@@ -1429,129 +1471,130 @@ k_trace(DevScene Sarg, RunCfg c, const Spawn* in, const uint64_t* offs, uint32_t
     uint32_t mid = (lo + hi) >> 1;
     if (offs[mid] <= gid) lo = mid; else hi = mid;
   }
-  uint32_t si = lo;
   RayS r;
+  if (build_ray(c, in[lo], (uint32_t)(gid - offs[lo]), r, ADJ ? pin + lo : nullptr)) put_ray(sk, r);
+}
+
+// Traversal result of one ray, at its window index.
+struct alignas(16) TraceOut {
+  double t;
+  int32_t prim;
+  int32_t pad;
+};
+
+// One generation, part 1: the rays of a window -> closest hits, one ray per thread.
+#ifndef RG_TRACE_WAVES
+#define RG_TRACE_WAVES 4     // waves per SIMD the register budget of k_trace targets
+#endif
+__global__ void __launch_bounds__(TBLOCK) __attribute__((amdgpu_waves_per_eu(RG_TRACE_WAVES)))
+k_trace(DevScene Sarg, RunCfg c, const RayGeo* geo, const RaySt* st, RayMap map, TraceOut* outp) {
+  __shared__ int32_t stk[LSTACK * TBLOCK];
+  __shared__ float stn[LSTACK * TBLOCK];
+  __shared__ float tes[NBIG_ORDER * TBLOCK];
+  static_assert(TBLOCK == kChunk, "one block per chunk");
+  uint32_t n;
+  const uint32_t at = map.chunk(blockIdx.x, n) + threadIdx.x;
+  if (threadIdx.x >= n) return;
+  const RayGeo g = geo[at];
   TraceOut o;
-  o.spawn = si;
   o.pad = 0;
-  if (!build_ray(c, in[si], (uint32_t)(gid - offs[si]), r)) {
-    o.prim = -2;
-    o.t = 0;
-    o.dx = o.dy = o.dz = 0.f;
-    outp[t] = o;
-    return;
-  }
-  wave_count(c.nrays);
   HitRec h;
-  closest_hit<TBLOCK>(scene_of(Sarg, c, r.scene), r.o, r.d, h, stk, stn, tes, c.err, c.visits);
+  closest_hit<TBLOCK>(scene_of(Sarg, c, c.nscenes ? st[at].scene : 0), v3(g.o[0], g.o[1], g.o[2]),
+                      v3(g.d[0], g.d[1], g.d[2]), h, stk, stn, tes, c.err, c.visits);
   o.t = h.t;
   o.prim = h.prim;
-  o.dx = (float)r.d.x; o.dy = (float)r.d.y; o.dz = (float)r.d.z;
-  outp[t] = o;
+  outp[blockIdx.x * kChunk + threadIdx.x] = o;
 }
 
 // Persistent form of k_trace with dynamic ray fetch.  A fixed grid of
 // wavefronts loops; when at least `refill` lanes of a wavefront have finished
-// their ray (or all have), the wavefront takes the next batch of child
-// indices from `work` with one atomic and the idle lanes start new rays,
-// while the others carry on.  Lanes therefore do not idle until the longest
-// ray of their wavefront ends, which is what bounds the one-ray-per-thread
-// kernel (its VALU lane utilisation is about a third).  A child's spawn lies
-// between the entries of its 64-child chunk in `first` (k_chunk_spawn).  Same
-// admission, closest-hit walk and output record as k_trace.  BATCH: rays of several
-// scenes (each lane keeps its ray's scene tables); otherwise the kernel
-// argument's scene, held in scalar registers.  WIDE: the walk fetches the
-// four-wide tree (four child boxes per node; the children hit are taken
-// nearest first, the others pushed farthest first).
+// their ray (or all have), the idle lanes start the next rays of the
+// wavefront's range, while the others carry on.  Lanes therefore do not idle
+// until the longest ray of their wavefront ends, which is what bounds the
+// one-ray-per-thread kernel (its VALU lane utilisation is about a third).  A
+// wavefront takes `grab` units of 64 rays from `work` at a time: the counter
+// is one address for the whole chip, 11.4 ns per increment (with one
+// increment per refill, and one per ray count, the walk of a 2,500-sensor
+// pass waited for 4.2 M of them).  Same closest-hit walk and output record as
+// k_trace.  BATCH: rays of several scenes (each lane keeps its ray's scene
+// tables); otherwise the kernel argument's scene, held in scalar registers.
+// WIDE: the walk fetches the four-wide tree (four child boxes per node; the
+// children hit are taken nearest first, the others pushed farthest first).
 template <int BS, bool BATCH, bool WIDE>
 __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(RG_TRACE_WAVES)))
-k_trace_pf(DevScene Sarg, RunCfg c, const Spawn* in, const uint64_t* offs, const uint32_t* first, uint64_t c0,
-           uint32_t nthreads, TraceOut* outp, uint32_t* work, uint32_t refill) {
+k_trace_pf(DevScene Sarg, RunCfg c, const RayGeo* geo, const RaySt* st, RayMap map, TraceOut* outp, uint32_t* work,
+           uint32_t refill, uint32_t grab) {
   __shared__ int32_t stk[LSTACK * BS];
   __shared__ float stn[LSTACK * BS];
   __shared__ float tes[NBIG_ORDER * BS];
   constexpr int32_t DONE = INT32_MIN;
-  c.adj = 0;
+  constexpr uint32_t kUnits = kChunk / 64;      // units of 64 rays per chunk
   const int lane = threadIdx.x;
-  const uint32_t wl = __lane_id();
+  const uint32_t nunit = map.nchunk * kUnits;
   uint64_t deep[PSTACK];
   int32_t tcur = -1;              // window index of this lane's ray, -1: idle
-  bool exhausted = false;         // no child left to take (wave-uniform)
+  // wave-uniform: units [u0, u1) still to open, rays [rpos, rend) of the open
+  // range, record index minus window index there, no unit left to take
+  uint32_t u0 = 0, u1 = 0, rpos = 0, rend = 0, rdelta = 0;
+  bool exhausted = false;
   DevScene S = Sarg;
   V3 o = v3(0, 0, 0), d = v3(0, 0, 1);
   HitRec h;
   h.t = FHUGE; h.rod = 1.0; h.prim = -1;
   int32_t node = DONE, leaf = -1;
   int sp = 0, iter = 0;
-  uint32_t si = 0;
   float ox = 0, oy = 0, oz = 0, ix = 0, iy = 0, iz = 0;
   uint32_t nvis = 0, nprim = 0;
   for (;;) {
     // ---- refill idle lanes ----
-    unsigned long long idle = __ballot(tcur < 0);
+    const unsigned long long idle = __ballot(tcur < 0);
     const uint32_t nidle = (uint32_t)__popcll(idle);
-    if (!exhausted && nidle && (nidle >= refill || nidle == (uint32_t)__popcll(__ballot(1)))) {
-      const uint32_t leader = __ffsll((long long)idle) - 1;
-      uint32_t base = 0;
-      if (wl == leader) base = atomicAdd(work, nidle);
-      base = __shfl(base, leader);
-      if ((uint64_t)base + nidle >= nthreads) exhausted = true;
-      if (tcur < 0) {
-        const uint32_t my = base + lane_rank(idle);
-        if (my < nthreads) {
-          const uint64_t gid = c0 + my;
-          // last spawn with offs <= gid, between the spawn of this chunk's
-          // first child and that of the next chunk's (or the window's last child)
-          const uint32_t ck = my >> CHUNK_LOG;
-          uint32_t lo = first[ck], hi = first[ck + 1] + 1;
-          if (hi - lo > 2) {
-            // a run of one-child spawns (the later generations) puts child
-            // gid at spawn lo + (gid - offs[lo]): try that spawn first, two
-            // dependent loads instead of a search of six or seven
-            const uint64_t o0 = offs[lo];
-            const uint32_t g = (uint32_t)min((uint64_t)(hi - 2), (uint64_t)lo + (gid - o0));
-            const uint64_t og = offs[g], og1 = offs[g + 1];
-            if (og <= gid && gid < og1) { lo = g; hi = g + 1; }
-          }
-          while (hi - lo > 1) {
-            uint32_t mid = (lo + hi) >> 1;
-            if (offs[mid] <= gid) lo = mid; else hi = mid;
-          }
-          si = lo;
-          RayS r;
-          Spawn srec;
-          uint64_t soff;
-          load_spawn(in, offs, si, srec, soff);
-          if (!build_ray(c, srec, (uint32_t)(gid - soff), r)) {
-            TraceOut to;
-            to.spawn = si; to.pad = 0; to.prim = -2; to.t = 0;
-            to.dx = to.dy = to.dz = 0.f;
-            outp[my] = to;
-          } else {
-            wave_count(c.nrays);
-            tcur = (int32_t)my;
-            if (BATCH) S = scene_of(Sarg, c, r.scene);
-            o = r.o;
-            d = r.d;
-            h.t = FHUGE; h.rod = 1.0; h.prim = -1;
-            big_hits<BS>(S, o, d, h, nprim, tes + lane);
-            node = DONE;
-            leaf = -1;
-            sp = 0;
-            iter = 0;
-            if (S.nbvh > 0) {
-              if (S.root < 0) { hit_prim(S, S.leaf_prim[~S.root], o, d, h); ++nprim; }
-              else node = S.root;
-            }
-            auto inv = [](double v) -> float {
-              float f = (float)v;
-              if (fabsf(f) < 1e-20f) f = f < 0 ? -1e-20f : 1e-20f;
-              return 1.0f / f;
-            };
-            ix = inv(d.x); iy = inv(d.y); iz = inv(d.z);
-            ox = (float)o.x * ix; oy = (float)o.y * iy; oz = (float)o.z * iz;   // origin x inverse direction
-          }
+    if (!exhausted && nidle && (nidle >= refill || nidle == 64u)) {
+      while (rpos >= rend) {
+        if (u0 >= u1) {
+          uint32_t b = 0;
+          if (__lane_id() == 0) b = atomicAdd(work, grab);
+          u0 = __builtin_amdgcn_readfirstlane(b);
+          if (u0 >= nunit) { exhausted = true; break; }
+          u1 = min(u0 + grab, nunit);
         }
+        const uint32_t ck = u0 / kUnits, ue = min(u1, (ck + 1) * kUnits);
+        uint32_t n;
+        const uint32_t base = map.chunk(ck, n);
+        rdelta = base - ck * kChunk;
+        rpos = u0 * 64u;
+        rend = min(ue * 64u, ck * kChunk + n);
+        u0 = ue;
+      }
+      if (rpos < rend) {
+        const uint32_t take = min(nidle, rend - rpos);
+        const uint32_t rank = lane_rank(idle);
+        if (tcur < 0 && rank < take) {
+          tcur = (int32_t)(rpos + rank);
+          const uint32_t at = rpos + rank + rdelta;
+          const RayGeo g = geo[at];
+          if (BATCH) S = scene_of(Sarg, c, st[at].scene);
+          o = v3(g.o[0], g.o[1], g.o[2]);
+          d = v3(g.d[0], g.d[1], g.d[2]);
+          h.t = FHUGE; h.rod = 1.0; h.prim = -1;
+          big_hits<BS>(S, o, d, h, nprim, tes + lane);
+          node = DONE;
+          leaf = -1;
+          sp = 0;
+          iter = 0;
+          if (S.nbvh > 0) {
+            if (S.root < 0) { hit_prim(S, S.leaf_prim[~S.root], o, d, h); ++nprim; }
+            else node = S.root;
+          }
+          auto inv = [](double v) -> float {
+            float f = (float)v;
+            if (fabsf(f) < 1e-20f) f = f < 0 ? -1e-20f : 1e-20f;
+            return 1.0f / f;
+          };
+          ix = inv(d.x); iy = inv(d.y); iz = inv(d.z);
+          ox = (float)o.x * ix; oy = (float)o.y * iy; oz = (float)o.z * iz;   // origin x inverse direction
+        }
+        rpos += take;
       }
     }
     if (__ballot(tcur >= 0) == 0ull) {
@@ -1680,10 +1723,9 @@ k_trace_pf(DevScene Sarg, RunCfg c, const Spawn* in, const uint64_t* offs, const
     // ---- finished rays: write the record, free the lane ----
     if ((tcur >= 0) & (node == DONE) & (leaf < 0)) {
       TraceOut to;
-      to.spawn = si; to.pad = 0;
       to.t = h.t;
       to.prim = h.prim;
-      to.dx = (float)d.x; to.dy = (float)d.y; to.dz = (float)d.z;
+      to.pad = 0;
       outp[tcur] = to;
       tcur = -1;
     }
@@ -1778,151 +1820,92 @@ void shadow_cast(const DevScene& S, const double* d_rays, const int32_t* d_src, 
   check(hipGetLastError(), "k_shadow_cast launch");
 }
 
-// One generation, part 2: shade the hits and append the next spawn records.
-// pin: path records of `in` (adjoint replay only).
+// One generation, part 2: shade the hits and append the next generation.
+// pin: path records of the rays (adjoint replay only).
 #ifndef RG_SHADE_WAVES
 #define RG_SHADE_WAVES 2     // waves per SIMD the register budget of k_shade targets
 #endif
 template <bool ADJ>
-__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(RG_SHADE_WAVES))) k_shade(DevScene Sarg, RunCfg c, const Spawn* in, const PathRec* pin,
-                                                 const uint64_t* offs, uint64_t c0, uint32_t nthreads,
-                                                 const TraceOut* tr, Sink sk) {
-  uint32_t t = blockIdx.x * BLOCK + threadIdx.x;
-  if (t >= nthreads) return;
+__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(RG_SHADE_WAVES)))
+k_shade(DevScene Sarg, RunCfg c, const RayGeo* geo, const RaySt* st, const PathRec* pin, RayMap map,
+        const TraceOut* tr, Sink sk) {
+  const uint32_t t = blockIdx.x * BLOCK + threadIdx.x;
+  uint32_t n;
+  const uint32_t at = map.chunk(t >> kChunkLog, n) + (t & (kChunk - 1u));
+  if ((t & (kChunk - 1u)) >= n) return;
   c.adj = ADJ;
-  if (!ADJ) sk.pbuf = nullptr;
-  // The loads a shaded ray starts with are issued together and waited for
-  // together: the 32-byte trace record (two 16-byte loads), then its spawn
-  // record, the spawn's first child index and, with one scene, the hit
-  // primitive's record.  The empty asm statements take the loaded vectors as
-  // inputs, which keeps the compiler from sinking a load below the early exit
-  // or to its first use, where each would cost a round trip of its own.
-  TraceOut o;
-  {
-    static_assert(sizeof(TraceOut) == 2 * sizeof(u32x4), "TraceOut layout");
-    const u32x4* tp = reinterpret_cast<const u32x4*>(tr + t);
-    const u32x4 a = tp[0], b = tp[1];
-    asm volatile("" :: "v"(a), "v"(b));
-    __builtin_memcpy(&o, &a, sizeof a);
-    __builtin_memcpy(reinterpret_cast<char*>(&o) + sizeof a, &b, sizeof b);
-  }
-  if (o.prim == -2) return;
-  const uint32_t si = o.spawn;
-  Spawn sp;
-  uint64_t off;
-  Prim P{};
-  const bool early = !c.nscenes && o.prim >= 0;
-  {
-    static_assert(sizeof(Spawn) == 6 * sizeof(u32x4), "Spawn layout");
-    const u32x4* spp = reinterpret_cast<const u32x4*>(in + si);
-    const u32x4 s0 = spp[0], s1 = spp[1], s2 = spp[2], s3 = spp[3], s4 = spp[4], s5 = spp[5];
-    off = offs[si];
-    u32x4 p0 = {0u, 0u, 0u, 0u}, p1 = {0u, 0u, 0u, 0u};
-    if (early) {
-      const u32x4* pp = reinterpret_cast<const u32x4*>(Sarg.prims + o.prim);
-      p0 = pp[0];
-      p1 = pp[1];
-    }
-    asm volatile("" :: "v"(s0), "v"(s1), "v"(s2), "v"(s3), "v"(s4), "v"(s5), "v"(off), "v"(p0), "v"(p1));
-    const u32x4 sv[6] = {s0, s1, s2, s3, s4, s5};
-    __builtin_memcpy(&sp, sv, sizeof sp);
-    static_assert(sizeof(Prim) == 2 * sizeof(u32x4), "Prim layout");
-    const u32x4 pv[2] = {p0, p1};
-    __builtin_memcpy(&P, pv, sizeof P);
-  }
+  if (!ADJ) { sk.pbuf = nullptr; sk.hpath = nullptr; }
+  const TraceOut o = tr[t];
+  const RaySt q = st[at];
+  const RayGeo g = geo[at];
+  const DevScene& S = scene_of(Sarg, c, q.scene);
   RayS r;
-  build_ray(c, sp, (uint32_t)(c0 + t - off), r, ADJ ? pin + si : nullptr);
+  r.o = v3(g.o[0], g.o[1], g.o[2]);
+  r.d = v3(g.d[0], g.d[1], g.d[2]);
+  r.coef = c3(q.coef[0], q.coef[1], q.coef[2]);
+  r.w = q.w;
+  r.crc = q.crc;
+  r.sensor = q.sensor;
+  r.crtype = q.crtype;
+  r.rtype = 0;
+  r.rsrc = q.rsrc;
+  r.rlvl = q.rlvl;
+  r.adepth = q.adepth;
+  r.scene = q.scene;
+  r.key = q.key;
+  if (ADJ) r.path = pin[at];
   HitRec h;
   h.t = o.t;
   h.prim = o.prim;
   h.rod = 1.0;
-  const DevScene& S = scene_of(Sarg, c, r.scene);
   if (h.prim >= 0) {
-    if (!early) P = S.prims[h.prim];
+    const Prim P = S.prims[h.prim];
     shade_hit(S, c, r, h, sk, P);
   } else {
     shade_miss(S, c, r);
   }
 }
 
-// ---- grouping a batched generation by scene ----------------------------------
-// Between generations of a batched launch the spawn records are regrouped by
-// scene (counting sort on Spawn.scene), so that the next windows trace one
-// scene at a time instead of interleaving every scene's tables in the caches.
-constexpr int SORT_BLOCK = 256;
-constexpr int SORT_ITEMS = 4;
-
-constexpr int NSC = kMaxBatchScenes;        // histogram bins (scenes)
-constexpr int SC_PER_T = NSC / SORT_BLOCK;   // bins per thread
-
-__global__ void __launch_bounds__(SORT_BLOCK) k_scene_hist(const Spawn* in, uint32_t n, uint32_t* hist) {
-  __shared__ uint32_t h[NSC];
-  for (int q = 0; q < SC_PER_T; ++q) h[threadIdx.x + q * SORT_BLOCK] = 0;
-  __syncthreads();
-  const size_t base = (size_t)blockIdx.x * SORT_BLOCK * SORT_ITEMS + threadIdx.x;
-  for (int k = 0; k < SORT_ITEMS; ++k) {
-    size_t i = base + (size_t)k * SORT_BLOCK;
-    if (i < n) atomicAdd(&h[in[i].scene], 1u);
+// After a window: its counts to the host and to the batch it wrote, and the
+// counters cleared for the next launch.  in: the window's own ray counts
+// when the host does not know them (rays built by k_hemi_rays), else null.
+// host: [0] rays out, [1] fullest segment, [2] hemisphere records, [3] rays
+// in, [4..5] children of the hemispheres.
+__global__ void __launch_bounds__(kRaySegs) k_window_done(uint32_t* ctr, uint32_t segcap, uint32_t* seg_out,
+                                                          uint32_t* in, uint32_t* host) {
+  const uint32_t t = threadIdx.x;
+  const uint32_t v = min(ctr[t * kCtrStride], segcap), vi = in ? in[t] : 0u;
+  ctr[t * kCtrStride] = 0u;
+  seg_out[t] = v;
+  uint32_t sum = v, mx = v, si = vi;
+#pragma unroll
+  for (int off = 32; off; off >>= 1) {
+    sum += __shfl_xor(sum, off);
+    mx = max(mx, (uint32_t)__shfl_xor(mx, off));
+    si += __shfl_xor(si, off);
   }
-  __syncthreads();
-  for (int q = 0; q < SC_PER_T; ++q) {
-    const int b = threadIdx.x + q * SORT_BLOCK;
-    if (h[b]) atomicAdd(&hist[b], h[b]);
+  if (t == 0) {
+    unsigned long long* kids = (unsigned long long*)(ctr + CTR_KIDS * kCtrStride);
+    host[0] = sum;
+    host[1] = mx;
+    host[2] = ctr[CTR_HEMI * kCtrStride];
+    host[3] = si;
+    host[4] = (uint32_t)*kids;
+    host[5] = (uint32_t)(*kids >> 32);
+    *kids = 0ull;
+    ctr[CTR_HEMI * kCtrStride] = 0u;
+    ctr[CTR_WORK * kCtrStride] = 0u;
+    __threadfence_system();
   }
 }
 
-// exclusive scan of the NSC scene counts (one block of 1024, 4 each)
-__global__ void __launch_bounds__(1024) k_scene_start(const uint32_t* hist, uint32_t* start) {
-  static_assert(NSC == 4 * 1024, "scan shape");
-  __shared__ uint32_t sh[1024];
-  const int t = threadIdx.x;
-  const uint32_t v0 = hist[4 * t], v1 = hist[4 * t + 1], v2 = hist[4 * t + 2], v3 = hist[4 * t + 3];
-  const uint32_t tot = v0 + v1 + v2 + v3;
-  sh[t] = tot;
-  __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {
-    uint32_t a = t >= off ? sh[t - off] : 0;
-    __syncthreads();
-    sh[t] += a;
-    __syncthreads();
-  }
-  const uint32_t ex = sh[t] - tot;
-  start[4 * t] = ex;
-  start[4 * t + 1] = ex + v0;
-  start[4 * t + 2] = ex + v0 + v1;
-  start[4 * t + 3] = ex + v0 + v1 + v2;
-}
-
-// Each block reserves one range per scene it holds, then places its records
-// (and their adjoint path records) at LDS-ranked positions in that range.
-__global__ void __launch_bounds__(SORT_BLOCK) k_scene_scatter(const Spawn* in, const PathRec* pin, uint32_t n,
-                                                              const uint32_t* start, uint32_t* fill, Spawn* out,
-                                                              PathRec* pout) {
-  __shared__ uint32_t h[NSC];
-  __shared__ uint32_t b[NSC];
-  for (int q = 0; q < SC_PER_T; ++q) h[threadIdx.x + q * SORT_BLOCK] = 0;
-  __syncthreads();
-  const size_t base = (size_t)blockIdx.x * SORT_BLOCK * SORT_ITEMS + threadIdx.x;
-  uint32_t sc[SORT_ITEMS], rank[SORT_ITEMS];
-  for (int k = 0; k < SORT_ITEMS; ++k) {
-    size_t i = base + (size_t)k * SORT_BLOCK;
-    sc[k] = i < n ? in[i].scene : 0u;
-    rank[k] = i < n ? atomicAdd(&h[sc[k]], 1u) : 0u;
-  }
-  __syncthreads();
-  for (int q = 0; q < SC_PER_T; ++q) {
-    const int c = threadIdx.x + q * SORT_BLOCK;
-    if (h[c]) b[c] = start[c] + atomicAdd(&fill[c], h[c]);
-  }
-  __syncthreads();
-  for (int k = 0; k < SORT_ITEMS; ++k) {
-    size_t i = base + (size_t)k * SORT_BLOCK;
-    if (i < n) {
-      uint32_t pos = b[sc[k]] + rank[k];
-      out[pos] = in[i];
-      if (pin) pout[pos] = pin[i];
-    }
-  }
+// After k_hemi_rays: the segment counts where the walk and shading read them
+// (added to those already there with `more`), and the segment counters
+// cleared for shading's own output.
+__global__ void __launch_bounds__(kRaySegs) k_hemi_done(uint32_t* ctr, uint32_t segcap, uint32_t* seg_out, bool more) {
+  const uint32_t t = threadIdx.x;
+  seg_out[t] = min(ctr[t * kCtrStride] + (more ? seg_out[t] : 0u), segcap);
+  ctr[t * kCtrStride] = 0u;
 }
 
 // ---- exclusive scan of uint32 counts (three-phase, LDS per block) ----------
@@ -1994,29 +1977,6 @@ __device__ __forceinline__ uint64_t block_excl_scan64(uint64_t v, uint64_t* sh, 
   return pre + incl - v;
 }
 
-template <class TI>
-__global__ void __launch_bounds__(SCAN_BLOCK) k_scan_tiles64(const TI* in, uint64_t* out, uint32_t n,
-                                                             uint64_t* tile_sums) {
-  __shared__ uint64_t sh[SCAN_BLOCK];
-  size_t base = (size_t)blockIdx.x * SCAN_TILE + threadIdx.x * SCAN_ITEMS;
-  uint64_t v[SCAN_ITEMS], s = 0;
-  for (int k = 0; k < SCAN_ITEMS; ++k) { v[k] = base + k < n ? (uint64_t)in[base + k] : 0; s += v[k]; }
-  uint64_t total;
-  uint64_t ex = block_excl_scan64(s, sh, total);
-  for (int k = 0; k < SCAN_ITEMS; ++k) {
-    if (base + k < n) out[base + k] = ex;
-    ex += v[k];
-  }
-  if (threadIdx.x == 0) tile_sums[blockIdx.x] = total;
-}
-
-__global__ void __launch_bounds__(SCAN_BLOCK) k_scan_add64(uint64_t* out, uint32_t n, const uint64_t* tile_offs) {
-  size_t base = (size_t)blockIdx.x * SCAN_TILE + threadIdx.x * SCAN_ITEMS;
-  uint64_t a = tile_offs[blockIdx.x];
-  for (int k = 0; k < SCAN_ITEMS; ++k)
-    if (base + k < n) out[base + k] += a;
-}
-
 }  // namespace rg
 
 // ---- host side -----------------------------------------------------------------
@@ -2042,15 +2002,12 @@ void exclusive_scan(const uint32_t* in, uint32_t* out, uint32_t n, DevArena& are
   }
 }
 
-// The same scan with its length n = min(*d_n, cap) read on the device, so
-// that it follows the kernel that produced the counts without a host round
-// trip: persistent blocks walk the tiles, one block scans the tile sums (and
-// writes the total to *d_total and out[n]), persistent blocks add the tile
-// offsets.
-__global__ void __launch_bounds__(SCAN_BLOCK) k_scan_tiles_dev(const uint32_t* in, uint64_t* out, const uint32_t* d_n,
-                                                               uint32_t cap, uint64_t* tile_sums) {
+// The same scan in 64 bits for the hemispheres' child counts: persistent
+// blocks walk the tiles, one block scans the tile sums (and writes the total
+// to out[n]), persistent blocks add the tile offsets.
+__global__ void __launch_bounds__(SCAN_BLOCK) k_scan_tiles64(const uint32_t* in, uint64_t* out, uint32_t n,
+                                                               uint64_t* tile_sums) {
   __shared__ uint64_t sh[SCAN_BLOCK];
-  const uint32_t n = min(*d_n, cap);
   const uint32_t ntiles = (n + SCAN_TILE - 1) / SCAN_TILE;
   for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
     const size_t base = (size_t)tile * SCAN_TILE + threadIdx.x * SCAN_ITEMS;
@@ -2067,10 +2024,8 @@ __global__ void __launch_bounds__(SCAN_BLOCK) k_scan_tiles_dev(const uint32_t* i
 }
 
 constexpr int SUMS_BLOCK = 1024;
-__global__ void __launch_bounds__(SUMS_BLOCK) k_scan_sums_dev(const uint32_t* d_n, uint32_t cap, uint64_t* tile_sums,
-                                                              uint64_t* out, uint64_t* d_total) {
+__global__ void __launch_bounds__(SUMS_BLOCK) k_scan_sums64(uint32_t n, uint64_t* tile_sums, uint64_t* out) {
   __shared__ uint64_t sh[SUMS_BLOCK / 64];
-  const uint32_t n = min(*d_n, cap);
   const uint32_t ntiles = (n + SCAN_TILE - 1) / SCAN_TILE;
   const uint32_t per = (ntiles + SUMS_BLOCK - 1) / SUMS_BLOCK;
   const uint32_t t = threadIdx.x, b0 = min(t * per, ntiles), b1 = min(b0 + per, ntiles);
@@ -2100,15 +2055,10 @@ __global__ void __launch_bounds__(SUMS_BLOCK) k_scan_sums_dev(const uint32_t* d_
     tile_sums[k] = ex;
     ex += v;
   }
-  if (t == SUMS_BLOCK - 1) {
-    out[n] = total;
-    *d_total = total;
-  }
+  if (t == SUMS_BLOCK - 1) out[n] = total;
 }
 
-__global__ void __launch_bounds__(SCAN_BLOCK) k_scan_add_dev(uint64_t* out, const uint32_t* d_n, uint32_t cap,
-                                                             const uint64_t* tile_offs) {
-  const uint32_t n = min(*d_n, cap);
+__global__ void __launch_bounds__(SCAN_BLOCK) k_scan_add64(uint64_t* out, uint32_t n, const uint64_t* tile_offs) {
   const uint32_t ntiles = (n + SCAN_TILE - 1) / SCAN_TILE;
   for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
     const size_t base = (size_t)tile * SCAN_TILE + threadIdx.x * SCAN_ITEMS;
@@ -2118,67 +2068,98 @@ __global__ void __launch_bounds__(SCAN_BLOCK) k_scan_add_dev(uint64_t* out, cons
   }
 }
 
-// out[i] = sum(in[0..i)) in 64 bits, out[n] = total.  `out` holds n+1 entries.
-template <class TI>
-static void exclusive_scan64(const TI* in, uint64_t* out, uint32_t n, DevArena& arena, hipStream_t st, int level) {
-  if (n == 0) {
-    check(hipMemsetAsync(out, 0, sizeof(uint64_t), st), "scan memset");
-    return;
-  }
-  uint32_t ntiles = (n + SCAN_TILE - 1) / SCAN_TILE;
-  uint64_t* sums = (uint64_t*)arena.get("scan64_sums" + std::to_string(level), sizeof(uint64_t) * (ntiles + 1), st, true);
-  hipLaunchKernelGGL(k_scan_tiles64<TI>, dim3(ntiles), dim3(SCAN_BLOCK), 0, st, in, out, n, sums);
-  if (ntiles > 1) {
-    uint64_t* soffs = (uint64_t*)arena.get("scan64_offs" + std::to_string(level), sizeof(uint64_t) * (ntiles + 1), st, true);
-    exclusive_scan64<uint64_t>(sums, soffs, ntiles, arena, st, level + 1);
-    hipLaunchKernelGGL(k_scan_add64, dim3(ntiles), dim3(SCAN_BLOCK), 0, st, out, n, soffs);
-    check(hipMemcpyAsync(out + n, soffs + ntiles, sizeof(uint64_t), hipMemcpyDeviceToDevice, st), "scan total");
-  } else {
-    check(hipMemcpyAsync(out + n, sums, sizeof(uint64_t), hipMemcpyDeviceToDevice, st), "scan total");
-  }
+// out[i] = sum(in[0..i)), out[n] = total.  `out` holds n+1 entries.
+static void scan_children(const uint32_t* in, uint64_t* out, uint32_t n, int ncu, DevArena& arena, hipStream_t st) {
+  const uint32_t ntiles = (n + SCAN_TILE - 1) / SCAN_TILE;
+  const uint32_t grid = std::min(ntiles, 2u * (uint32_t)ncu);
+  uint64_t* sums = (uint64_t*)arena.get("scan_sums64", sizeof(uint64_t) * (ntiles + 1), st, false);
+  hipLaunchKernelGGL(k_scan_tiles64, dim3(grid), dim3(SCAN_BLOCK), 0, st, in, out, n, sums);
+  hipLaunchKernelGGL(k_scan_sums64, dim3(1), dim3(SUMS_BLOCK), 0, st, n, sums, out);
+  if (ntiles > 1) hipLaunchKernelGGL(k_scan_add64, dim3(grid), dim3(SCAN_BLOCK), 0, st, out, n, sums);
+  check(hipGetLastError(), "scan launch");
 }
 
 void render(const DevScene& S, RunCfg cfg, const double* d_rays, uint32_t nsens, bool imm_irrad, int max_srcs,
             const Tuning& tn, DevArena& arena, hipStream_t st, RenderStats* stats) {
-  // Work proceeds in waves of at most `window` children; each child appends
-  // at most `per_child` spawn records, so a wave never overflows its buffer.
-  const uint32_t per_child = 6u + (uint32_t)std::max(max_srcs, S.nsrcs);
+  // Work proceeds in windows of at most `window` rays or hemisphere children;
+  // each ray appends at most `per_ray` rays and two hemispheres, so a window
+  // never overflows its buffers.
+  const uint32_t per_ray = 6u + (uint32_t)std::max(max_srcs, S.nsrcs);
   const uint32_t window = std::max<uint32_t>(tn.window, 1024u);
+  const bool adj = cfg.adj != 0;
   int dev = 0, ncu = 256;
   check(hipGetDevice(&dev), "device");
   check(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev), "device attribute");
-  const uint32_t pf_blocks = (uint32_t)std::max(1, ncu) * std::max<uint32_t>(tn.blocks_per_cu, 1u);
+  ncu = std::max(1, ncu);
+  const uint32_t pf_blocks = (uint32_t)ncu * std::max<uint32_t>(tn.blocks_per_cu, 1u);
   const long max_batches = 1L << 22;
-  uint32_t* d_cnt = (uint32_t*)arena.get("ctr", 64, st, true);
-  uint32_t* h_cnt = arena.host_u32(16);   // [0, 8): frame totals and seeds; [8, 16): windows in flight
+  constexpr int kInFlight = 2;
+  constexpr uint32_t kHostWords = 8;       // per window: k_window_done's report
+  uint32_t* d_ctr = (uint32_t*)arena.get("ctr", sizeof(uint32_t) * kCtrWords * kInFlight, st, true);
+  uint32_t* h_win = arena.host_u32(kHostWords * kInFlight);
 
-  const bool adj = cfg.adj != 0;
-  struct Batch { Spawn* buf; PathRec* pbuf; uint32_t n; int slot; };
-  int nslots = 0;
+  // Output buffers of one window ("slot"): rays in segments, hemispheres.
+  // Both are opened later as frames; the slot is free again when both are
+  // walked.  A slot is held to 1/24 of the device's memory (about six are
+  // live at the deepest point of a ray tree) and to 16 GiB, so capacities fit
+  // 32 bits and scenes with many light sources shrink their windows instead
+  // of failing to allocate.
+  struct Slot {
+    RayGeo* geo; RaySt* rst; PathRec* path; uint32_t* cnt;
+    Spawn* hemi; uint32_t* hcount; PathRec* hpath; uint64_t* hoffs;
+    uint32_t seg_log, segcap, hcap;
+    int frames;
+  };
+  std::vector<Slot> slots;
   std::vector<int> free_slots;
-  auto new_slot = [&]() -> int {
-    if (!free_slots.empty()) { int s = free_slots.back(); free_slots.pop_back(); return s; }
-    return nslots++;
-  };
-  auto slot_buf = [&](int s, size_t cap) -> Spawn* {
-    return (Spawn*)arena.get("spawn" + std::to_string(s), sizeof(Spawn) * cap, st, false);
-  };
-  // adjoint replay: one path record beside every spawn record
-  auto slot_path = [&](int s, size_t cap) -> PathRec* {
-    return adj ? (PathRec*)arena.get("path" + std::to_string(s), sizeof(PathRec) * cap, st, false) : nullptr;
-  };
-  // Spawn buffers: at most slot_bytes each (a window's children each append
-  // at most per_child records), so capacities fit 32 bits and scenes with
-  // many light sources shrink their windows instead of failing to allocate.
-  // A slot is held to 1/24 of the device's memory (about six slots are live
-  // at the deepest point of a ray tree, each with its scan and trace
-  // records), and to 16 GiB.
   size_t dev_mem = 0;
   check(hipDeviceTotalMem(&dev_mem, dev), "device memory");
   const size_t slot_bytes = std::max<size_t>(size_t(64) << 20, std::min<size_t>(size_t(16) << 30, dev_mem / 24));
-  const uint32_t slot_children = (uint32_t)std::max<size_t>(64, slot_bytes / (sizeof(Spawn) * per_child));
-  const uint32_t win = std::min(window, slot_children);
+  const size_t ray_bytes = sizeof(RayGeo) + sizeof(RaySt) + (adj ? sizeof(PathRec) : 0);
+  const size_t hemi_bytes = sizeof(Spawn) + sizeof(uint32_t) + sizeof(uint64_t) + (adj ? sizeof(PathRec) : 0);
+  const uint32_t slot_rays = (uint32_t)std::max<size_t>(kChunk, slot_bytes / (ray_bytes * per_ray + 2 * hemi_bytes));
+  const uint32_t win = std::min(window, slot_rays);
+  auto buf = [&](const char* what, int s, size_t bytes) -> void* {
+    return arena.get(what + std::to_string(s), bytes, st, false);
+  };
+  // Segments for rays appended by nblk blocks: one per 32 blocks (64
+  // wavefronts, 0.7 us of queueing on one counter), up to kRaySegs; fewer
+  // blocks keep their rays together, so that chunks stay full.
+  auto seg_log_for = [](uint32_t nblk) {
+    uint32_t l = 0;
+    while ((2u << l) <= kRaySegs && (nblk >> 5) >= (2u << l)) ++l;
+    return l;
+  };
+  // a slot for the output of nblk blocks of BLOCK threads, each appending at
+  // most `per` rays and two hemispheres
+  auto new_slot = [&](uint32_t nblk, uint32_t per, uint32_t seg_log) -> int {
+    int s;
+    if (!free_slots.empty()) { s = free_slots.back(); free_slots.pop_back(); }
+    else { s = (int)slots.size(); slots.push_back(Slot{}); }
+    const uint32_t nseg = 1u << seg_log;
+    const uint32_t segcap = (nblk + nseg - 1) / nseg * BLOCK * per;
+    const size_t cap = (size_t)segcap * nseg, hcap = (size_t)nblk * BLOCK * 2;
+    Slot& o = slots[s];
+    o.seg_log = seg_log;
+    o.segcap = segcap;
+    o.hcap = (uint32_t)hcap;
+    o.geo = (RayGeo*)buf("geo", s, sizeof(RayGeo) * cap);
+    o.rst = (RaySt*)buf("rst", s, sizeof(RaySt) * cap);
+    o.path = adj ? (PathRec*)buf("path", s, sizeof(PathRec) * cap) : nullptr;
+    o.cnt = (uint32_t*)buf("segcnt", s, sizeof(uint32_t) * kRaySegs);
+    o.hemi = (Spawn*)buf("hemi", s, sizeof(Spawn) * hcap);
+    o.hcount = (uint32_t*)buf("hcount", s, sizeof(uint32_t) * hcap);
+    o.hpath = adj ? (PathRec*)buf("hpath", s, sizeof(PathRec) * hcap) : nullptr;
+    o.hoffs = (uint64_t*)buf("hoffs", s, sizeof(uint64_t) * (hcap + 1));
+    o.frames = 0;
+    return s;
+  };
+  auto sink_of = [&](int s, uint32_t* ctr) {
+    const Slot& o = slots[s];
+    return Sink{o.geo, o.rst, o.path, o.seg_log, o.segcap, nullptr, o.hemi, o.hcount, o.hpath, o.hcap, ctr, cfg.err};
+  };
   long gens = 0;
+  unsigned long long traced = 0;
   // Events: two per window in flight (its read-back, and the trace / shade
   // timing when asked for), reused in turn.
   struct Events {
@@ -2186,7 +2167,6 @@ void render(const DevScene& S, RunCfg cfg, const double* d_rays, uint32_t nsens,
     ~Events() { for (hipEvent_t e : ev) (void)hipEventDestroy(e); }
   } evs;
   const bool timing = stats && stats->timing;
-  constexpr int kInFlight = 2;
   for (int k = 0; k < kInFlight; ++k) {
     hipEvent_t e;
     check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event");
@@ -2198,173 +2178,181 @@ void render(const DevScene& S, RunCfg cfg, const double* d_rays, uint32_t nsens,
       }
   }
   const int ev_per = timing ? 4 : 1;
-  static_assert(8 + 4 * kInFlight <= 16, "host counters");
-  uint32_t* h_win = h_cnt + 8;   // per in-flight window: spawn count, work counter, child total (64 bits)
-  // Depth first, one window at a time: after each window its children are
-  // opened and walked before the next window of the same batch, so live
-  // spawn buffers are bounded by the depth of the ray tree, not by the size
-  // of a generation.
-  struct Frame { Batch bt; uint64_t* offs; uint64_t total; uint64_t c0; };
+  // Depth first, one window at a time: after each window what it appended is
+  // walked before the next window of the same frame, so live slots are
+  // bounded by the depth of the ray tree, not by the size of a generation.
+  // A frame is a slot's rays (hemi false: chunks [at, total)) or its
+  // hemispheres' children (hemi true: children [at, total)).  counted: the
+  // host knows how many rays a ray frame holds.
+  struct Frame { int slot; bool hemi, counted; uint32_t nhemi; uint64_t total, at; };
   std::vector<Frame> frames;
-  // compact child counts and their exclusive scan, per slot
-  auto slot_counts = [&](int s, size_t cap) -> uint32_t* {
-    return (uint32_t*)arena.get("counts" + std::to_string(s), sizeof(uint32_t) * (cap + 1), st, false);
+  // children [c0, c0 + nth) of a slot's nh hemispheres, appended to sk
+  auto hemi_rays = [&](const Slot& in, uint32_t nh, uint64_t c0, uint32_t nth, const Sink& sk) {
+    const uint32_t grid = (nth + BLOCK - 1) / BLOCK;
+    if (adj)
+      hipLaunchKernelGGL(k_hemi_rays<true>, dim3(grid), dim3(BLOCK), 0, st, cfg, in.hemi, in.hpath, in.hoffs, nh, c0,
+                         nth, sk);
+    else
+      hipLaunchKernelGGL(k_hemi_rays<false>, dim3(grid), dim3(BLOCK), 0, st, cfg, in.hemi, in.hpath, in.hoffs, nh, c0,
+                         nth, sk);
   };
-  auto slot_offs = [&](int s, size_t cap) -> uint64_t* {
-    return (uint64_t*)arena.get("offs" + std::to_string(s), sizeof(uint64_t) * (cap + 1), st, false);
-  };
-  // A batch whose size the host knows: scan its child counts (recounted
-  // from the records after a scene regroup), read the total.
-  auto open_frame = [&](const Batch& b, bool recount) {
-    if (b.n == 0) { free_slots.push_back(b.slot); return; }
+  // the frames of a slot whose launch has reported `h` (k_window_done)
+  auto open_slot = [&](int s, const uint32_t* h) {
+    Slot& o = slots[s];
+    const uint32_t nh = std::min(h[2], o.hcap);
+    if (!h[0] && !nh) { free_slots.push_back(s); return; }
     if (++gens > max_batches) throw std::runtime_error("ray tree did not terminate");
-    uint32_t* counts = slot_counts(b.slot, b.n);
-    uint64_t* offs = slot_offs(b.slot, b.n);
-    if (recount) hipLaunchKernelGGL(k_counts, dim3((b.n + BLOCK - 1) / BLOCK), dim3(BLOCK), 0, st, b.buf, b.n, counts);
-    exclusive_scan64<uint32_t>(counts, offs, b.n, arena, st, 0);
-    check(hipMemcpyAsync(h_cnt, offs + b.n, sizeof(uint64_t), hipMemcpyDeviceToHost, st), "total");
-    check(hipStreamSynchronize(st), "scan");
-    const uint64_t total = (uint64_t)h_cnt[0] | ((uint64_t)h_cnt[1] << 32);   // little-endian 64-bit total
-    frames.push_back({b, offs, total, 0});
+    const uint64_t kids = (uint64_t)h[4] | ((uint64_t)h[5] << 32);
+    if (nh) scan_children(o.hcount, o.hoffs, nh, ncu, arena, st);
+    // Hemispheres beside rays: where their children fit behind the rays and
+    // all of them make one window, they join the rays, which saves the walk
+    // of a second, smaller window (a window's last wavefronts take 50-100 us).
+    const uint32_t nseg = 1u << o.seg_log;
+    if (h[0] && nh && kids <= win) {
+      const uint32_t grid = (uint32_t)((kids + BLOCK - 1) / BLOCK);
+      const uint64_t most = (uint64_t)h[1] + (uint64_t)(grid + nseg - 1) / nseg * BLOCK;
+      const uint64_t chunks = (most + kChunk - 1) / kChunk << o.seg_log;
+      if (most <= o.segcap && chunks <= std::max<uint32_t>(win / kChunk, 1u)) {
+        Sink sk = sink_of(s, d_ctr);
+        sk.have = o.cnt;
+        hemi_rays(o, nh, 0, (uint32_t)kids, sk);
+        hipLaunchKernelGGL(k_hemi_done, dim3(1), dim3(kRaySegs), 0, st, d_ctr, o.segcap, o.cnt, true);
+        check(hipGetLastError(), "k_hemi_rays launch");
+        frames.push_back({s, false, false, 0, chunks, 0});
+        ++o.frames;
+        return;
+      }
+    }
+    if (nh) {
+      frames.push_back({s, true, false, nh, kids, 0});
+      ++o.frames;
+    }
+    if (h[0]) {
+      const uint64_t tiles = (h[1] + kChunk - 1) / kChunk;
+      frames.push_back({s, false, true, 0, tiles << o.seg_log, 0});
+      ++o.frames;
+      traced += h[0];
+    }
   };
-  const uint32_t scan_grid = 2u * (uint32_t)std::max(1, ncu);
   // Generation 0 per chunk of sensors (buffers are sized to the work at hand
   // and kept by the arena for later calls, so a context that only ever
   // traces a few sensors stays small); each chunk's tree is walked to the
   // end before the next chunk is seeded.
-  const uint32_t chunk = std::max<uint32_t>(1u, std::min<uint32_t>(nsens, slot_children));
+  const uint32_t chunk = std::max<uint32_t>(1u, std::min<uint32_t>(nsens, slot_rays));
   for (uint32_t s0 = 0; s0 < nsens; s0 += chunk) {
     const uint32_t ns = std::min(chunk, nsens - s0);
-    const size_t batch_cap = (size_t)ns * per_child;
     const double* rays0 = d_rays + 6 * (size_t)s0;
     {
-      int s = new_slot();
-      Spawn* b = slot_buf(s, batch_cap);
-      PathRec* pb = slot_path(s, batch_cap);
-      uint32_t* bc = slot_counts(s, batch_cap);
-      check(hipMemsetAsync(d_cnt, 0, sizeof(uint32_t), st), "memset");
-      uint32_t grid = (ns + BLOCK - 1) / BLOCK;
-      if (imm_irrad) {
-        Sink sk{b, d_cnt, (uint32_t)batch_cap, cfg.err, pb, bc};
-        if (adj) hipLaunchKernelGGL(k_irrad_seed<true>, dim3(grid), dim3(BLOCK), 0, st, S, cfg, rays0, ns, s0, sk);
-        else hipLaunchKernelGGL(k_irrad_seed<false>, dim3(grid), dim3(BLOCK), 0, st, S, cfg, rays0, ns, s0, sk);
-        if (cfg.nscenes <= 1) {
-          // child counts scanned on the device: one read-back of the spawn
-          // count and the child total
-          uint64_t* offs = slot_offs(s, batch_cap);
-          uint64_t* sums =
-              (uint64_t*)arena.get("scan_dev_sums", sizeof(uint64_t) * (batch_cap / SCAN_TILE + 2), st, false);
-          hipLaunchKernelGGL(k_scan_tiles_dev, dim3(scan_grid), dim3(SCAN_BLOCK), 0, st, bc, offs, d_cnt,
-                             (uint32_t)batch_cap, sums);
-          hipLaunchKernelGGL(k_scan_sums_dev, dim3(1), dim3(SUMS_BLOCK), 0, st, d_cnt, (uint32_t)batch_cap, sums, offs,
-                             (uint64_t*)(d_cnt + 2));
-          hipLaunchKernelGGL(k_scan_add_dev, dim3(scan_grid), dim3(SCAN_BLOCK), 0, st, offs, d_cnt,
-                             (uint32_t)batch_cap, sums);
-          check(hipGetLastError(), "scan launch");
-          check(hipMemcpyAsync(h_cnt, d_cnt, 4 * sizeof(uint32_t), hipMemcpyDeviceToHost, st), "count");
-          check(hipStreamSynchronize(st), "seed");
-          const uint32_t nseed = std::min<uint32_t>(h_cnt[0], (uint32_t)batch_cap);
-          if (nseed) {
-            if (++gens > max_batches) throw std::runtime_error("ray tree did not terminate");
-            const uint64_t total = (uint64_t)h_cnt[2] | ((uint64_t)h_cnt[3] << 32);
-            frames.push_back({Batch{b, pb, nseed, s}, offs, total, 0});
-          } else {
-            free_slots.push_back(s);
-          }
-        } else {
-          check(hipMemcpyAsync(h_cnt, d_cnt, sizeof(uint32_t), hipMemcpyDeviceToHost, st), "count");
-          check(hipStreamSynchronize(st), "seed");
-          open_frame({b, pb, std::min<uint32_t>(h_cnt[0], (uint32_t)batch_cap), s}, false);
-        }
-      } else {
-        hipLaunchKernelGGL(k_primary_seed, dim3(grid), dim3(BLOCK), 0, st, cfg, rays0, ns, s0, b, bc);
-        if (pb) check(hipMemsetAsync(pb, 0, sizeof(PathRec) * ns, st), "memset");   // empty paths
-        open_frame({b, pb, ns, s}, false);
-      }
+      const uint32_t grid = (ns + BLOCK - 1) / BLOCK;
+      const int s = new_slot(grid, imm_irrad ? per_ray : 1u, imm_irrad ? seg_log_for(grid) : 0u);
+      const Sink sk = sink_of(s, d_ctr);
+      if (imm_irrad && adj)
+        hipLaunchKernelGGL(k_irrad_seed<true>, dim3(grid), dim3(BLOCK), 0, st, S, cfg, rays0, ns, s0, sk);
+      else if (imm_irrad)
+        hipLaunchKernelGGL(k_irrad_seed<false>, dim3(grid), dim3(BLOCK), 0, st, S, cfg, rays0, ns, s0, sk);
+      else if (adj)
+        hipLaunchKernelGGL(k_primary_seed<true>, dim3(grid), dim3(BLOCK), 0, st, cfg, rays0, ns, s0, sk);
+      else
+        hipLaunchKernelGGL(k_primary_seed<false>, dim3(grid), dim3(BLOCK), 0, st, cfg, rays0, ns, s0, sk);
+      hipLaunchKernelGGL(k_window_done, dim3(1), dim3(kRaySegs), 0, st, d_ctr, sk.segcap, slots[s].cnt,
+                         (uint32_t*)nullptr, h_win);
+      check(hipGetLastError(), "seed launch");
+      check(hipStreamSynchronize(st), "seed");
+      open_slot(s, h_win);
     }
     // With tn.inflight = 2 windows are pipelined: while the GPU runs one, the
-    // host waits for the counts of the one before and pushes its children's
-    // frame.  All work is on one stream, so windows run in the order they
-    // were queued and a slot freed on the host is only overwritten after the
-    // kernels reading it.  Batched launches regroup each window's spawns by
-    // scene before their frame opens, and run one window at a time.
-    struct Pending { Batch out; size_t cap; uint32_t nth; int pair; };
+    // host waits for the counts of the one before and opens its frames.  All
+    // work is on one stream, so windows run in the order they were queued and
+    // a slot freed on the host is only overwritten after the kernels reading
+    // it.
+    struct Pending { int slot; uint32_t nth; int pair; };
     std::vector<Pending> inflight;
     int next_pair = 0;
-    const size_t depth = cfg.nscenes <= 1 ? (size_t)std::max(1, std::min(tn.inflight, kInFlight)) : 1;
+    const size_t depth = (size_t)std::max(1, std::min(tn.inflight, kInFlight));
     auto launch_window = [&]() {
-      const Batch bt = frames.back().bt;
-      const uint64_t* offs = frames.back().offs;
-      const uint64_t c0 = frames.back().c0;
-      const uint64_t total = frames.back().total;
-      uint32_t nth = (uint32_t)std::min<uint64_t>(win, total - c0);
-      frames.back().c0 += nth;
-      size_t cap = (size_t)nth * per_child;
-      int s = new_slot();
-      Spawn* ob = slot_buf(s, cap);
-      PathRec* opb = slot_path(s, cap);
-      uint32_t* ocnt = slot_counts(s, cap);
-      uint64_t* ooffs = slot_offs(s, cap);
-      TraceOut* tout = (TraceOut*)arena.get("trace_out", sizeof(TraceOut) * nth, st, false);
+      Frame& f = frames.back();
       const int pair = next_pair;
       next_pair = (next_pair + 1) % kInFlight;
+      uint32_t* ctr = d_ctr + (size_t)pair * kCtrWords;
       hipEvent_t* e = &evs.ev[pair * ev_per];
-      check(hipMemsetAsync(d_cnt, 0, 2 * sizeof(uint32_t), st), "memset");   // spawn count, work counter
-      Sink sk{ob, d_cnt, (uint32_t)cap, cfg.err, opb, ocnt};
       if (timing) check(hipEventRecord(e[1], st), "event");
-      const uint32_t tblocks = (nth + TBLOCK - 1) / TBLOCK;
-      if (tn.trace_kernel == 1) {
-        const uint32_t nch = (nth + (1u << CHUNK_LOG) - 1) >> CHUNK_LOG;
-        uint32_t* first = (uint32_t*)arena.get("chunk_spawn", sizeof(uint32_t) * (nch + 1), st, false);
-        hipLaunchKernelGGL(k_chunk_spawn, dim3((nch + BLOCK) / BLOCK), dim3(BLOCK), 0, st, offs, bt.n, c0, nth, first);
-        const uint32_t nb = std::min(tblocks, pf_blocks);
-        if (cfg.nscenes && tn.wide)
-          hipLaunchKernelGGL((k_trace_pf<TBLOCK, true, true>), dim3(nb), dim3(TBLOCK), 0, st, S, cfg, bt.buf, offs,
-                             first, c0, nth, tout, d_cnt + 1, tn.refill);
-        else if (cfg.nscenes)
-          hipLaunchKernelGGL((k_trace_pf<TBLOCK, true, false>), dim3(nb), dim3(TBLOCK), 0, st, S, cfg, bt.buf, offs,
-                             first, c0, nth, tout, d_cnt + 1, tn.refill);
-        else if (tn.wide)
-          hipLaunchKernelGGL((k_trace_pf<TBLOCK, false, true>), dim3(nb), dim3(TBLOCK), 0, st, S, cfg, bt.buf, offs,
-                             first, c0, nth, tout, d_cnt + 1, tn.refill);
-        else
-          hipLaunchKernelGGL((k_trace_pf<TBLOCK, false, false>), dim3(nb), dim3(TBLOCK), 0, st, S, cfg, bt.buf, offs,
-                             first, c0, nth, tout, d_cnt + 1, tn.refill);
+      RayMap map;
+      const RayGeo* geo;
+      const RaySt* rst;
+      const PathRec* path;
+      uint32_t* in_cnt = nullptr;     // ray counts only the device knows
+      if (f.hemi) {
+        // build the rays of the next children into a buffer of their own
+        const Slot in = slots[f.slot];
+        const uint32_t nth = (uint32_t)std::min<uint64_t>(win, f.total - f.at);
+        const uint32_t grid = (nth + BLOCK - 1) / BLOCK, sl = seg_log_for(grid), nseg = 1u << sl;
+        const uint32_t segcap = (grid + nseg - 1) / nseg * BLOCK;
+        const size_t cap = (size_t)segcap * nseg;
+        Sink sk{};
+        sk.geo = (RayGeo*)arena.get("hemi_geo", sizeof(RayGeo) * cap, st, false);
+        sk.st = (RaySt*)arena.get("hemi_rst", sizeof(RaySt) * cap, st, false);
+        sk.pbuf = adj ? (PathRec*)arena.get("hemi_path", sizeof(PathRec) * cap, st, false) : nullptr;
+        sk.seg_log = sl;
+        sk.segcap = segcap;
+        sk.ctr = ctr;
+        sk.err = cfg.err;
+        in_cnt = (uint32_t*)arena.get("hemi_cnt", sizeof(uint32_t) * kRaySegs, st, false);
+        hemi_rays(in, f.nhemi, f.at, nth, sk);
+        hipLaunchKernelGGL(k_hemi_done, dim3(1), dim3(kRaySegs), 0, st, ctr, segcap, in_cnt, false);
+        check(hipGetLastError(), "k_hemi_rays launch");
+        f.at += nth;
+        geo = sk.geo;
+        rst = sk.st;
+        path = sk.pbuf;
+        map = RayMap{in_cnt, sl, segcap, 0u, ((segcap + kChunk - 1) / kChunk) << sl};
       } else {
-        hipLaunchKernelGGL(k_trace, dim3(tblocks), dim3(TBLOCK), 0, st, S, cfg, bt.buf, offs, bt.n, c0, nth, tout);
+        const Slot& in = slots[f.slot];
+        const uint32_t nck = (uint32_t)std::min<uint64_t>(std::max<uint32_t>(win / kChunk, 1u), f.total - f.at);
+        map = RayMap{in.cnt, in.seg_log, in.segcap, (uint32_t)f.at, nck};
+        f.at += nck;
+        if (!f.counted) in_cnt = in.cnt;
+        geo = in.geo;
+        rst = in.rst;
+        path = in.path;
+      }
+      const uint32_t sblocks = map.nchunk * (kChunk / BLOCK);
+      const int s = new_slot(sblocks, per_ray, seg_log_for(sblocks));   // may move `slots`
+      const Sink sk = sink_of(s, ctr);
+      TraceOut* tout = (TraceOut*)arena.get("trace_out", sizeof(TraceOut) * kChunk * (size_t)map.nchunk, st, false);
+      if (tn.trace_kernel == 1) {
+        const uint32_t nunit = map.nchunk * (kChunk / 64u);
+        const uint32_t nb = std::min((nunit + TBLOCK / 64 - 1) / (TBLOCK / 64), pf_blocks);
+        const uint32_t grab = std::min(std::max(nunit / (8u * nb * (TBLOCK / 64)), 1u), 16u);
+        uint32_t* work = ctr + CTR_WORK * kCtrStride;
+        auto go = [&](auto kern) {
+          hipLaunchKernelGGL(kern, dim3(nb), dim3(TBLOCK), 0, st, S, cfg, geo, rst, map, tout, work, tn.refill, grab);
+        };
+        if (cfg.nscenes && tn.wide) go(k_trace_pf<TBLOCK, true, true>);
+        else if (cfg.nscenes) go(k_trace_pf<TBLOCK, true, false>);
+        else if (tn.wide) go(k_trace_pf<TBLOCK, false, true>);
+        else go(k_trace_pf<TBLOCK, false, false>);
+      } else {
+        hipLaunchKernelGGL(k_trace, dim3(map.nchunk), dim3(TBLOCK), 0, st, S, cfg, geo, rst, map, tout);
       }
       check(hipGetLastError(), "k_trace launch");
       if (timing) check(hipEventRecord(e[2], st), "event");
       if (adj)
-        hipLaunchKernelGGL(k_shade<true>, dim3((nth + BLOCK - 1) / BLOCK), dim3(BLOCK), 0, st, S, cfg, bt.buf,
-                           bt.pbuf, offs, c0, nth, tout, sk);
+        hipLaunchKernelGGL(k_shade<true>, dim3(sblocks), dim3(BLOCK), 0, st, S, cfg, geo, rst, path, map, tout, sk);
       else
-        hipLaunchKernelGGL(k_shade<false>, dim3((nth + BLOCK - 1) / BLOCK), dim3(BLOCK), 0, st, S, cfg, bt.buf,
-                           bt.pbuf, offs, c0, nth, tout, sk);
+        hipLaunchKernelGGL(k_shade<false>, dim3(sblocks), dim3(BLOCK), 0, st, S, cfg, geo, rst, path, map, tout, sk);
       check(hipGetLastError(), "k_shade launch");
       if (timing) check(hipEventRecord(e[3], st), "event");
-      if (cfg.nscenes <= 1) {
-        // the new batch's child counts scanned on the device right after
-        // shading: one read-back (spawn count and child total) per window
-        uint64_t* sums = (uint64_t*)arena.get("scan_dev_sums", sizeof(uint64_t) * (cap / SCAN_TILE + 2), st, false);
-        hipLaunchKernelGGL(k_scan_tiles_dev, dim3(scan_grid), dim3(SCAN_BLOCK), 0, st, ocnt, ooffs, d_cnt,
-                           (uint32_t)cap, sums);
-        hipLaunchKernelGGL(k_scan_sums_dev, dim3(1), dim3(SUMS_BLOCK), 0, st, d_cnt, (uint32_t)cap, sums, ooffs,
-                           (uint64_t*)(d_cnt + 2));
-        hipLaunchKernelGGL(k_scan_add_dev, dim3(scan_grid), dim3(SCAN_BLOCK), 0, st, ooffs, d_cnt, (uint32_t)cap,
-                           sums);
-        check(hipGetLastError(), "scan launch");
-      }
-      check(hipMemcpyAsync(h_win + 4 * pair, d_cnt, 4 * sizeof(uint32_t), hipMemcpyDeviceToHost, st), "count");
+      hipLaunchKernelGGL(k_window_done, dim3(1), dim3(kRaySegs), 0, st, ctr, sk.segcap, slots[s].cnt, in_cnt,
+                         h_win + kHostWords * pair);
+      check(hipGetLastError(), "k_window_done launch");
       check(hipEventRecord(e[0], st), "event");
-      inflight.push_back({Batch{ob, opb, 0, s}, cap, nth, pair});
+      inflight.push_back({s, map.nchunk * kChunk, pair});
     };
     auto finish_window = [&]() {
       const Pending pw = inflight.front();
       inflight.erase(inflight.begin());
       hipEvent_t* e = &evs.ev[pw.pair * ev_per];
       check(hipEventSynchronize(e[0]), "bounce");
-      const uint32_t* h = h_win + 4 * pw.pair;
       if (timing) {
         float ms = 0, ms2 = 0;
         check(hipEventElapsedTime(&ms, e[1], e[2]), "event time");
@@ -2373,35 +2361,14 @@ void render(const DevScene& S, RunCfg cfg, const double* d_rays, uint32_t nsens,
         stats->shade_ms += ms2;
       }
       if (stats) { stats->launches++; stats->threads += pw.nth; }
-      const int s = pw.out.slot;
-      const uint32_t nout = std::min<uint32_t>(h[0], (uint32_t)pw.cap);
-      if (!nout) {
-        free_slots.push_back(s);
-        return;
-      }
-      if (cfg.nscenes <= 1) {
-        if (++gens > max_batches) throw std::runtime_error("ray tree did not terminate");
-        const uint64_t total = (uint64_t)h[2] | ((uint64_t)h[3] << 32);
-        frames.push_back({Batch{pw.out.buf, pw.out.pbuf, nout, s}, slot_offs(s, pw.cap), total, 0});
-        return;
-      }
-      // regroup by scene into the slot's second buffer, which the batch then uses
-      const size_t cap = pw.cap;
-      Spawn* sb = (Spawn*)arena.get("spawn_sorted" + std::to_string(s), sizeof(Spawn) * cap, st, false);
-      PathRec* spb = adj ? (PathRec*)arena.get("path_sorted" + std::to_string(s), sizeof(PathRec) * cap, st, false)
-                         : nullptr;
-      uint32_t* hist = (uint32_t*)arena.get("scene_hist", sizeof(uint32_t) * 3 * NSC, st, true);
-      const uint32_t nb = (nout + SORT_BLOCK * SORT_ITEMS - 1) / (SORT_BLOCK * SORT_ITEMS);
-      hipLaunchKernelGGL(k_scene_hist, dim3(nb), dim3(SORT_BLOCK), 0, st, pw.out.buf, nout, hist);
-      hipLaunchKernelGGL(k_scene_start, dim3(1), dim3(1024), 0, st, hist, hist + NSC);
-      hipLaunchKernelGGL(k_scene_scatter, dim3(nb), dim3(SORT_BLOCK), 0, st, pw.out.buf, pw.out.pbuf, nout,
-                         hist + NSC, hist + 2 * NSC, sb, spb);
-      check(hipGetLastError(), "scene sort launch");
-      open_frame(Batch{sb, spb, nout, s}, true);
+      const uint32_t* h = h_win + kHostWords * pw.pair;
+      traced += h[3];
+      open_slot(pw.slot, h);
     };
     while (!frames.empty() || !inflight.empty()) {
-      while (!frames.empty() && frames.back().c0 >= frames.back().total) {
-        free_slots.push_back(frames.back().bt.slot);
+      while (!frames.empty() && frames.back().at >= frames.back().total) {
+        Slot& o = slots[frames.back().slot];
+        if (--o.frames == 0) free_slots.push_back(frames.back().slot);
         frames.pop_back();
       }
       if (!frames.empty() && inflight.size() < depth) {
@@ -2413,6 +2380,7 @@ void render(const DevScene& S, RunCfg cfg, const double* d_rays, uint32_t nsens,
   }
   if (stats) {
     stats->generations = gens;
+    stats->rays = traced;
     stats->node_bytes = (tn.trace_kernel == 1 && tn.wide) ? (int)sizeof(BVH4Node) : (int)sizeof(BVHNode);
   }
 }

@@ -68,6 +68,7 @@ struct RenderStats {
   long generations = 0;
   long launches = 0;
   unsigned long long threads = 0;
+  unsigned long long rays = 0;   // rays traced (admitted children)
   bool timing = false;       // time every generation's kernels with HIP events
   double bounce_ms = 0;      // summed traversal-kernel (k_trace) durations
   double shade_ms = 0;       // summed shading-kernel (k_shade) durations

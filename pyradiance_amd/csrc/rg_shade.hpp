@@ -10,7 +10,29 @@
 
 namespace rg {
 
-// A spawn record: one parent event that produces `count` child rays.
+// A ray ready to be traced, in two parallel arrays: what the walk reads (origin
+// and unit direction), and what shading needs beside them.  Rays are built
+// and admitted (rayorigin(), rt/raytrace.c:40-135) where they are spawned.
+struct alignas(16) RayGeo {
+  double o[3], d[3];
+};
+struct alignas(16) RaySt {
+  uint64_t key;
+  float coef[3];     // cumulative coefficient
+  float w;           // weight
+  float crc;         // largest channel of the ray's own rcoef
+  uint32_t sensor;
+  uint16_t crtype;   // cumulative ray type
+  int16_t rsrc;      // aimed source
+  uint8_t rlvl;      // reflection level
+  uint8_t adepth;    // ambient recursion depth
+  uint16_t scene;    // scene of a batched launch
+  uint32_t pad[2];
+};
+static_assert(sizeof(RayGeo) == 48 && sizeof(RaySt) == 48, "ray layout");
+
+// A spawn record: one hemisphere of `count` stratified child rays (or, while
+// it is being built, one explicit ray).
 struct alignas(16) Spawn {
   double org[3];     // child origin (parent hit point)
   float d0[3];       // explicit direction, or hemisphere normal
@@ -141,7 +163,6 @@ struct RunCfg {
   double* out;         // [nsensor][ncols]
   double fix;          // > 0: deposits add up as int64 multiples of 1 / fix in `out` (order-independent,
                        // so results repeat bit for bit); 0: FP64 atomics
-  unsigned long long* nrays;
   unsigned long long* visits;  // optional: [0] BVH nodes visited, [1] primitives tested
   uint32_t* err;       // error flags
   // adjoint replay (adj != 0): instead of writing `out`, each binned

@@ -537,3 +537,76 @@ def test_child_order_changes_only_the_order(L):
     c.close()
     assert res[0][1] == res[1][1]
     assert np.allclose(res[0][0], res[1][0], rtol=1e-9, atol=1e-15)
+
+
+@pytest.fixture(scope="module")
+def mirror_room(L):
+    """A room whose trees hold every kind of child at once: hemispheres,
+    single rays, mirror and pane continuations and shadow rays of a sun."""
+    room = scenes.Room()
+    rad = (scenes.room_rad(room) + "void metal mirror_mat\n0\n0\n5 .8 .8 .8 .9 0\n"
+           + scenes.box_quads_rad("mirror_mat", "mbox", (2.0, 1.5, 0.01), (3.1, 2.4, 1.7), 2, 2)
+           + scenes.furniture_rad(np.random.default_rng(3), 6, room)
+           + scenes.sun_rad(scenes.sun_direction(35.0, 170.0)) + scenes.sky_rad((1, 1, 1), ground=(1, 1, 1)))
+    sens = np.zeros((600, 6))
+    rng = np.random.default_rng(9)
+    sens[:, 0], sens[:, 1], sens[:, 2] = rng.uniform(0.1, 5.9, 600), rng.uniform(0.1, 3.9, 600), 0.8
+    sens[:, 5] = 1.0
+    c = _ctx(L, rad)
+    c.set_params(_rc_params(L, ambounce=3, ambdiv=96, minweight=1e-3, seed=4))
+    mods = _sky_mods(L)
+    full = c.contrib(sens, mods, 1, L.RT_IMM_IRRAD)
+    yield c, mods, sens, full, c.last_nrays()
+    c.close()
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 127, 129, 255, 256, 257, 600])
+@pytest.mark.parametrize("window", [1 << 10, 1 << 15, 1 << 24])
+def test_records_do_not_depend_on_the_batch_around_them(L, mirror_room, n, window):
+    """A sensor's samples follow from its index alone, so its record is the
+    same bit for bit however many sensors share the call and however the
+    rays fall into segments, chunks and windows (window 1024 splits every
+    generation, 2^15 some of them, 2^24 none)."""
+    _say(f"records of {n} sensors, window {window}")
+    c, mods, sens, full, _ = mirror_room
+    c.set_tuning(window=window)
+    got = c.contrib(sens[:n], mods, 1, L.RT_IMM_IRRAD)
+    c.set_tuning(window=1 << 24)
+    assert np.array_equal(got, full[:n])
+
+
+@pytest.mark.parametrize("shape", [dict(window=1 << 10), dict(window=1 << 12, inflight=2), dict(trace_kernel=0),
+                                   dict(refill=1), dict(refill=64, blocks_per_cu=1)])
+def test_ray_count_does_not_depend_on_the_launch_shape(L, mirror_room, shape):
+    """Every admitted ray is traced and counted once, whichever windows,
+    wavefronts and units of work it falls into."""
+    _say(f"ray count at {shape}")
+    c, mods, sens, full, nrays = mirror_room
+    c.set_tuning(**shape)
+    got = c.contrib(sens, mods, 1, L.RT_IMM_IRRAD)
+    count = c.last_nrays()
+    c.set_tuning(window=1 << 24, inflight=1, trace_kernel=1, refill=16, blocks_per_cu=4)
+    again = c.contrib(sens, mods, 1, L.RT_IMM_IRRAD)
+    assert np.array_equal(got, full) and np.array_equal(again, full)
+    assert count == c.last_nrays()
+
+
+def test_path_records_follow_their_rays_through_every_window(L):
+    """The adjoint's gradient with every generation split into windows of
+    1,024 children equals the one of whole generations (FP64 atomics: to
+    summation order)."""
+    from pyradiance_amd.adjoint import DiffScene
+    _say("adjoint over split windows")
+    rad, sens, groups = scenes.config4(nsensors=40)
+    sc = DiffScene(rad, sens, groups, _sky_mods(L), _rc_params(L, ambounce=2, ambdiv=128, minweight=1e-3, seed=2))
+    rng = np.random.default_rng(1)
+    dlde, sky = rng.normal(size=(40, 3)), rng.uniform(0.5, 2.0, (146, 3))
+    res = []
+    for shape in (dict(window=1 << 24), dict(window=1 << 10), dict(window=1 << 11, inflight=2)):
+        sc.ctx.set_tuning(**shape)
+        res.append(sc.adjoint(dlde, sky))
+    sc.close()
+    scale = np.abs(res[0]).max()
+    assert scale > 0
+    for g in res[1:]:
+        assert np.abs(g - res[0]).max() <= 1e-11 * scale
