@@ -45,10 +45,10 @@ HBM_PEAK_GBS = 8000.0          # MI355X HBM3E
 BF16_PEAK_TFLOPS = 2500.0      # MI355X dense BF16 MFMA
 
 # Algorithmic bytes per ray segment: ray record in + hit out (48 B), one node
-# per BVH node visited (64 B binary, 128 B four-wide, as the renderer
-# reports), one 48-byte primitive record per primitive tested, one 32-byte
-# path-state read-modify-write.
-B_RAY, B_NODE, B_PRIM, B_STATE = 48.0, 64.0, 48.0, 32.0
+# per BVH node visited (64 B, as the renderer reports), one 128-byte
+# primitive record per primitive tested, one 32-byte path-state
+# read-modify-write.
+B_RAY, B_NODE, B_PRIM, B_STATE = 48.0, 64.0, 128.0, 32.0
 
 
 def log(*a):
@@ -636,7 +636,7 @@ def config5_bench(seed: int = 0):
                         "10-storey office, then DC x sky 20000x2306x8760",
             "primitives": int(info["primitives"]), "sensors": int(len(sens)), "scene_generate_s": t_gen,
             "scene_commit_s": t_commit, "rays": int(rays), "trace_s": t_trace, "Mrays_per_s": rays / t_trace / 1e6,
-            "rays_per_sensor": rays / len(sens), "walk": "wide" if st.get("node_bytes") == 128 else "binary",
+            "rays_per_sensor": rays / len(sens), "walk": "wide" if info["primitives"] <= (4 << 20) else "binary",
             "dcsky_s": t_dc, "dcsky_output_finite": finite,
             "dc_nonzero_fraction": float((A > 0).mean())}
 
@@ -953,7 +953,7 @@ def main():
     st_c = ctx.last_stats()
     ctx.set_profiling(0)
     nr = st_c["rays"]
-    b_node = st_c.get("node_bytes") or B_NODE   # 64 B binary node, 128 B four-wide node
+    b_node = st_c.get("node_bytes") or B_NODE
     per_ray = B_RAY + b_node * st_c["nodes"] / nr + B_PRIM * st_c["prims"] / nr + B_STATE
     avg_launch_ms = st_t["trace_ms"] / max(st_t["launches"], 1)
     bytes_per_launch = per_ray * st_t["rays"] / max(st_t["launches"], 1)
@@ -1019,7 +1019,7 @@ def main():
     bvh_name = args.bvh if args.bvh != "auto" else ("sah" if info["primitives"] <= (4 << 20) else "lbvh")
     if scene_tuned:
         bvh_name = "sah" if scene_tuned["best"]["builder"] == _lib.BVH_SAH else "lbvh"
-    walk = "wide" if st_c.get("node_bytes") == 128 else "binary"
+    walk = "wide" if bvh_name == "sah" else "binary"
     traffic_ray = committed_traffic(bvh_name, walk)
     # HBM bytes per launch = measured bytes per ray x rays per launch of this run
     traffic = traffic_ray * st_t["rays"] / max(st_t["launches"], 1) if traffic_ray else None

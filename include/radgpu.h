@@ -202,8 +202,8 @@ int rg_set_tuning(rg_ctx *ctx, const char *key, long long value);
 int rg_set_bvh_builder(rg_ctx *ctx, int kind);
 /* out[0..8] = rays, generation launches, threads launched, summed traversal-
  * kernel milliseconds, nodes visited, primitives tested, batches, summed
- * shading-kernel milliseconds, bytes per node visited (64 binary, 128
- * four-wide) */
+ * shading-kernel milliseconds, bytes per node visited (64 in
+ * either tree) */
 int rg_last_stats(rg_ctx *ctx, double *out, int n);
 
 /* DC x sky product, replaces cm_multiply() (util/cmatrix.c:421-474):

@@ -289,12 +289,18 @@ int rg_scene_commit(rg_ctx* c) {
     // three per four-wide node) fit the traversal stack
     std::vector<BVHNode> hn;
     std::vector<BVH4Node> h4;
+    std::vector<BVH4Q> h4q;
+    std::vector<int32_t> lpos;
     int root = -1;
     bool wide = false;
     if (sah) {
       root = build_sah_bvh(slo_v.data(), shi_v.data(), small_ids.data(), n, hn, kMaxTreeDepth);
       const int d4 = collapse_bvh4(hn, root, h4);
       wide = root == 0 && !h4.empty() && 3 * d4 <= kTraceStackEntries;   // both walks start at node 0
+      if (wide) {
+        quantize_bvh4(h4, h4q);
+        lpos = leaf_positions(hn, root, cs.prims.size());
+      }
     }
     // every table in one device block, sent in one copy
     Pack pk;
@@ -306,7 +312,7 @@ int rg_scene_commit(rg_ctx* c) {
                  o_nodes = pk.add(hn.data(), sizeof(BVHNode) * hn.size(), sizeof(BVHNode) * std::max<uint32_t>(n, 1)),
                  o_leaf = pk.add(sah ? small_ids.data() : nullptr, sah ? sizeof(int32_t) * n : 0,
                                  sizeof(int32_t) * std::max<uint32_t>(n, 1)),
-                 o_nodes4 = wide ? pk.add(h4) : 0, o_blo = sah ? 0 : pk.add(slo_v), o_bhi = sah ? 0 : pk.add(shi_v),
+                 o_nodes4 = wide ? pk.add(h4q) : 0, o_lpos = wide ? pk.add(lpos) : 0, o_blo = sah ? 0 : pk.add(slo_v), o_bhi = sah ? 0 : pk.add(shi_v),
                  o_bids = sah ? 0 : pk.add(small_ids);
     char* blob = (char*)c->scene_mem.get("blob", pk.total, c->st, false);
     pk.send(c, blob);
@@ -323,7 +329,7 @@ int rg_scene_commit(rg_ctx* c) {
     S.bigpl = to_global((const BigPlane*)(blob + o_bigpl));
     S.nbig = (int)big.size();
     S.nbvh = (int)n;
-    S.nodes4 = wide ? to_global((const BVH4Node*)(blob + o_nodes4)) : nullptr;
+    S.nodes4 = wide ? to_global((const BVH4Q*)(blob + o_nodes4)) : nullptr;
     BVHNode* nodes = (BVHNode*)(blob + o_nodes);
     int32_t* leaf = (int32_t*)(blob + o_leaf);
     if (n == 0) S.root = -1;
@@ -332,6 +338,12 @@ int rg_scene_commit(rg_ctx* c) {
                              nodes, leaf, c->arena, c->st);
     S.nodes = to_global(nodes);
     S.leaf_prim = to_global(leaf);
+    S.leafs = nullptr;
+    if (wide) {
+      LeafRec* recs = (LeafRec*)c->scene_mem.get("leafs", sizeof(LeafRec) * cs.prims.size(), c->st, false);
+      leaf_records(S, (const int32_t*)(blob + o_lpos), recs, c->st);
+      S.leafs = to_global((const LeafRec*)recs);
+    }
     hipck(hipStreamSynchronize(c->st), "scene commit");
     c->committed = true;
   });

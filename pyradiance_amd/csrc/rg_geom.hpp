@@ -31,6 +31,29 @@ struct alignas(16) BVH4Node {
   int32_t pad[4];
 };
 
+// The same four boxes in 64 bytes, the form the walk fetches: planes in steps
+// of scale[a] from org[a], rounded outward (one byte each, four children per
+// word), so every box holds the one it stands for.
+struct alignas(16) BVH4Q {
+  float org[3], scale[3];
+  uint32_t lox, hix, loy, hiy, loz, hiz;
+  int32_t child[4];
+};
+static_assert(sizeof(BVH4Q) == 64, "one node, half a cache line");
+
+// A primitive as the walk tests it, in one cache line.  Polygons of three or
+// four vertices: plane, then the vertices in the two coordinates of the
+// inside test (a triangle's last one twice); other shapes hold only their
+// index and are tested from the primitive tables.
+struct alignas(16) LeafRec {
+  double n[3], off;
+  double v[4][2];
+  int32_t ax;        // coordinate the inside test leaves out, -1: not such a polygon
+  int32_t pos;       // place among the tree's leaves, left to right (-1: kept out of the tree)
+  int32_t pad[6];
+};
+static_assert(sizeof(LeafRec) == 128, "one primitive, one cache line");
+
 // Planes of the first kBigPlanes room-sized primitives, in one contiguous
 // table: the walk estimates their hit distances from these before any
 // primitive test, with one load per entry instead of the chain big index ->
@@ -54,7 +77,8 @@ struct DevScene {
   const RG_GLOBAL Material* mats;
   const RG_GLOBAL Source* srcs;
   const RG_GLOBAL BVHNode* nodes;
-  const RG_GLOBAL BVH4Node* nodes4;    // four-wide form of `nodes` (root 0); null: none
+  const RG_GLOBAL BVH4Q* nodes4;       // four-wide form of `nodes` (root 0); null: none
+  const RG_GLOBAL LeafRec* leafs;      // per primitive, with nodes4
   const RG_GLOBAL int32_t* leaf_prim;   // sorted leaf position -> primitive index
   const RG_GLOBAL int32_t* big;         // primitives kept out of the BVH, tested first
   const RG_GLOBAL BigPlane* bigpl;      // kBigPlanes entries, see BigPlane
@@ -76,9 +100,10 @@ struct HitRec {
   double t;                     // rot
   double rod;
   int32_t prim;                 // -1: none
+  int32_t tie;                  // set when only the order decided between two primitives (within FTINY of each other)
 };
 
-RG_HD bool ray_reject(const DevScene& S, int prim, double t, double rod, const HitRec& h) {
+RG_HD bool ray_reject(const DevScene& S, int prim, double t, double rod, HitRec& h) {
   if ((t <= FTINY) | (t > h.t + FTINY)) return true;
   if (t < h.t - FTINY) return false;
   if (h.prim == prim) return true;
@@ -98,7 +123,9 @@ RG_HD bool ray_reject(const DevScene& S, int prim, double t, double rod, const H
   } else if (h.rod <= 0) {
     return false;
   }
-  return S.prims[h.prim].omod >= S.prims[prim].omod;
+  const int oh = S.prims[h.prim].omod, on = S.prims[prim].omod;
+  if (oh == on) h.tie = 1;
+  return oh >= on;
 }
 
 // polygon geometry block: n[3], offset, ax, then nv vertices
@@ -205,6 +232,130 @@ RG_HD void hit_polygon(const DevScene& S, int pi, V3 n, double off, const double
   V3 p = o + d * t;
   if (!in_face(p, g, nv)) return;
   h.t = t; h.rod = rdot; h.prim = pi;
+}
+
+// in_face() for the two coordinates of a leaf record: the same comparisons of
+// the same numbers, without early exits (each only returns true, and the
+// crossing count does not matter then).
+RG_HD bool in_leaf(const LeafRec& L, V3 p) {
+  const double x = L.ax == 0 ? p.y : (L.ax == 1 ? p.z : p.x);
+  const double y = L.ax == 0 ? p.z : (L.ax == 1 ? p.x : p.y);
+  bool on = false, odd = false;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const double* a = L.v[(k + 3) & 3];
+    const double* b = L.v[k];
+    const bool ax = a[0] > x, bx = b[0] > x;
+    on |= (fabs(a[1] - y) <= FTINY) & (fabs(b[1] - y) <= FTINY) & (ax != bx);
+    const bool cross = (a[1] > y) != (b[1] > y);
+    const double pa = (a[1] - y) * (b[0] - x), pb = (a[0] - x) * (b[1] - y);
+    const bool mixed = cross & (ax != bx);
+    on |= mixed & (fabs(pa - pb) <= FTINY);
+    on |= cross & !(ax | bx) & (fabs(a[0] - x) <= FTINY) & (fabs(b[0] - x) <= FTINY);
+    odd ^= (cross & ax & bx) | (mixed & ((b[1] > a[1]) != (pa > pb)));
+  }
+  return on | odd;
+}
+
+// hit_prim() from a leaf record.
+RG_HD void hit_prim(const DevScene& S, int pi, V3 o, V3 d, HitRec& h);
+RG_HD void hit_leaf(const DevScene& S, const LeafRec& L, int pi, V3 o, V3 d, HitRec& h) {
+  if (L.ax < 0) { hit_prim(S, pi, o, d, h); return; }
+  const V3 n = load3(L.n);
+  const double rdot = -dot(d, n);
+  if ((rdot <= FTINY) & (rdot >= -FTINY)) return;
+  const double t = (dot(o, n) - L.off) / rdot;
+  if (ray_reject(S, pi, t, rdot, h)) return;
+  if (!in_leaf(L, o + d * t)) return;
+  h.t = t; h.rod = rdot; h.prim = pi;
+}
+
+// Whether a four-wide walk of the unrounded boxes meets the leaf at position
+// pa before the one at pb: in the node where their paths part (a binary node
+// and its grandchildren, or a child that is a leaf), the child entered nearer
+// comes first, equal entries in slot order.  o: origin times inverse
+// direction, iv: inverse direction.  Nodes are numbered depth first, left
+// subtree first, so a subtree of m leaves takes the m - 1 numbers from its
+// root on, and a node's leaf range follows from its children's numbers.
+RG_HD bool met_before(const DevScene& S, int pa, int pb, const float o[3], const float iv[3]) {
+  int idx = S.root, b = 0, e = S.nbvh;
+  for (;;) {
+    const BVHNode N = S.nodes[idx];
+    const int m = N.left < 0 ? 1 : (N.right >= 0 ? N.right - idx : e - b - 1);
+    float tn[2] = {0.f, 0.f};
+    int slot[2], kid[2] = {0, 0}, kb[2] = {0, 0}, ke[2] = {0, 0};
+    for (int w = 0; w < 2; ++w) {
+      const int p = w ? pb : pa;
+      const bool rt = p >= b + m;
+      const int c = rt ? N.right : N.left;
+      const float *lo = rt ? N.rmin : N.lmin, *hi = rt ? N.rmax : N.lmax;
+      BVHNode G;
+      slot[w] = rt && N.left >= 0 ? 2 : (rt ? 1 : 0);
+      kid[w] = c;
+      kb[w] = rt ? b + m : b;
+      ke[w] = rt ? e : b + m;
+      if (c >= 0) {
+        G = S.nodes[c];
+        const int g = G.left < 0 ? 1 : (G.right >= 0 ? G.right - c : ke[w] - kb[w] - 1);
+        const bool gr = p >= kb[w] + g;
+        slot[w] += gr;
+        kid[w] = gr ? G.right : G.left;
+        lo = gr ? G.rmin : G.lmin;
+        hi = gr ? G.rmax : G.lmax;
+        if (gr) kb[w] += g; else ke[w] = kb[w] + g;
+      }
+      for (int a = 0; a < 3; ++a) {
+        const float t0 = fmaf(lo[a], iv[a], -o[a]), t1 = fmaf(hi[a], iv[a], -o[a]);
+        const float t = fminf(t0, t1);
+        tn[w] = a == 0 ? t : fmaxf(tn[w], t);
+      }
+    }
+    if (slot[0] != slot[1]) return tn[0] < tn[1] || (tn[0] == tn[1] && slot[0] < slot[1]);
+    if (kid[0] < 0) return true;          // one leaf: nothing to order
+    idx = kid[0];
+    b = kb[0];
+    e = ke[0];
+  }
+}
+
+// hit_leaf() as a walk in the order of the unrounded boxes decides it: where
+// only the order decides between the hit so far and this primitive
+// (HitRec.tie), the one met_before() the other stays.
+RG_HD void hit_leaf_ordered(const DevScene& S, const LeafRec& L, int pi, V3 o, V3 d, const float ot[3],
+                            const float iv[3], HitRec& h) {
+  h.tie = 0;
+  const HitRec was = h;
+  hit_leaf(S, L, pi, o, d, h);
+  if (!h.tie) return;
+  // this primitive alone, at a distance within FTINY of the other's
+  HitRec q;
+  q.t = FHUGE; q.rod = 1.0; q.prim = -1; q.tie = 0;
+  hit_leaf(S, L, pi, o, d, q);
+  h = was;
+  if (q.prim != pi || q.t > was.t + FTINY || q.t < was.t - FTINY) return;
+  const int pos = S.leafs[was.prim].pos;
+  if (pos < 0 || met_before(S, pos, L.pos, ot, iv)) return;     // kept out of the tree: tested first
+  h = q;
+}
+
+// The leaf record of a primitive at leaf position `pos`.
+RG_HD LeafRec leaf_rec(const DevScene& S, int pi, int pos) {
+  LeafRec L = {};
+  const Prim& P = S.prims[pi];
+  L.ax = -1;
+  L.pos = pos;
+  if (P.kind != PK_POLYGON || P.nv < 3 || P.nv > 4) return L;
+  const double* g = S.geom + P.goff;
+  for (int a = 0; a < 3; ++a) L.n[a] = g[a];
+  L.off = g[3];
+  L.ax = (int)g[4];
+  const int xi = (L.ax + 1) % 3, yi = (xi + 1) % 3;
+  for (int k = 0; k < 4; ++k) {
+    const double* v = g + 5 + 3 * (k < P.nv ? k : P.nv - 1);
+    L.v[k][0] = v[xi];
+    L.v[k][1] = v[yi];
+  }
+  return L;
 }
 
 RG_HD void hit_prim(const DevScene& S, int pi, V3 o, V3 d, HitRec& h) {

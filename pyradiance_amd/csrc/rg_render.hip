@@ -72,7 +72,7 @@ struct RayMap {
 // every output segment, the hemisphere records and their children, and the
 // walk's next unit of work.  k_window_done copies them out and clears them.
 constexpr uint32_t kCtrStride = 32;     // 32-bit words
-enum : uint32_t { CTR_HEMI = kRaySegs, CTR_KIDS = kRaySegs + 1, CTR_WORK = kRaySegs + 2, CTR_COUNT = kRaySegs + 3 };
+enum : uint32_t { CTR_HEMI = kRaySegs, CTR_KIDS, CTR_WORK, CTR_COUNT };
 constexpr uint32_t kCtrWords = CTR_COUNT * kCtrStride;
 
 // Where a launch appends.  pbuf / hpath: path records (adjoint replay, else null).
@@ -1479,7 +1479,7 @@ __global__ void __launch_bounds__(BLOCK) k_hemi_rays(RunCfg c, const Spawn* in, 
 struct alignas(16) TraceOut {
   double t;
   int32_t prim;
-  int32_t pad;
+  int32_t front;     // ahead of the four-wide walk: the hit faces the ray (only its sign decides ties)
 };
 
 // One generation, part 1: the rays of a window -> closest hits, one ray per thread.
@@ -1497,7 +1497,7 @@ k_trace(DevScene Sarg, RunCfg c, const RayGeo* geo, const RaySt* st, RayMap map,
   if (threadIdx.x >= n) return;
   const RayGeo g = geo[at];
   TraceOut o;
-  o.pad = 0;
+  o.front = 0;
   HitRec h;
   closest_hit<TBLOCK>(scene_of(Sarg, c, c.nscenes ? st[at].scene : 0), v3(g.o[0], g.o[1], g.o[2]),
                       v3(g.d[0], g.d[1], g.d[2]), h, stk, stn, tes, c.err, c.visits);
@@ -1518,9 +1518,9 @@ k_trace(DevScene Sarg, RunCfg c, const RayGeo* geo, const RaySt* st, RayMap map,
 // pass waited for 4.2 M of them).  Same closest-hit walk and output record as
 // k_trace.  BATCH: rays of several scenes (each lane keeps its ray's scene
 // tables); otherwise the kernel argument's scene, held in scalar registers.
-// WIDE: the walk fetches the four-wide tree (four child boxes per node; the
-// children hit are taken nearest first, the others pushed farthest first).
-template <int BS, bool BATCH, bool WIDE>
+// Walks the binary tree: the scenes without a four-wide one (device LBVH
+// trees, and trees too deep for its stack).
+template <int BS, bool BATCH>
 __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(RG_TRACE_WAVES)))
 k_trace_pf(DevScene Sarg, RunCfg c, const RayGeo* geo, const RaySt* st, RayMap map, TraceOut* outp, uint32_t* work,
            uint32_t refill, uint32_t grab) {
@@ -1619,69 +1619,8 @@ k_trace_pf(DevScene Sarg, RunCfg c, const RayGeo* geo, const RaySt* st, RayMap m
       }
       return DONE;
     };
-    auto push = [&](int32_t ref, float t) -> bool {
-      if (sp < LSTACK) { stk[sp * BS + lane] = ref; stn[sp * BS + lane] = t; }
-      else if (sp < LSTACK + PSTACK) deep[sp - LSTACK] = pack_entry(ref, t);
-      else return false;
-      ++sp;
-      return true;
-    };
-    if (WIDE) {
-      const BVH4Node* __restrict__ n4 = S.nodes4;
-      while (node >= 0) {
-        if (++iter > S.nbvh + 8) { atomicOr(c.err, ERR_STACK); node = DONE; leaf = -1; break; }
-        const BVH4Node& N = n4[node];
-        ++nvis;
-        const float tmax = (float)(h.t + 2 * FTINY) * 1.000001f;
-        const float kInf = __int_as_float(0x7f800000);
-        float t0, t1, t2, t3;
-        int32_t c0r = N.child[0], c1r = N.child[1], c2r = N.child[2], c3r = N.child[3];
-        {
-          float tk, lo[3], hi[3];
-          lo[0] = N.lox[0]; lo[1] = N.loy[0]; lo[2] = N.loz[0]; hi[0] = N.hix[0]; hi[1] = N.hiy[0]; hi[2] = N.hiz[0];
-          t0 = (slab(lo, hi, ox, oy, oz, ix, iy, iz, tmax, tk) & (c0r != DONE)) ? tk : kInf;
-          lo[0] = N.lox[1]; lo[1] = N.loy[1]; lo[2] = N.loz[1]; hi[0] = N.hix[1]; hi[1] = N.hiy[1]; hi[2] = N.hiz[1];
-          t1 = (slab(lo, hi, ox, oy, oz, ix, iy, iz, tmax, tk) & (c1r != DONE)) ? tk : kInf;
-          lo[0] = N.lox[2]; lo[1] = N.loy[2]; lo[2] = N.loz[2]; hi[0] = N.hix[2]; hi[1] = N.hiy[2]; hi[2] = N.hiz[2];
-          t2 = (slab(lo, hi, ox, oy, oz, ix, iy, iz, tmax, tk) & (c2r != DONE)) ? tk : kInf;
-          lo[0] = N.lox[3]; lo[1] = N.loy[3]; lo[2] = N.loz[3]; hi[0] = N.hix[3]; hi[1] = N.hiy[3]; hi[2] = N.hiz[3];
-          t3 = (slab(lo, hi, ox, oy, oz, ix, iy, iz, tmax, tk) & (c3r != DONE)) ? tk : kInf;
-        }
-        // ascending entry distance, equal distances in slot order: five
-        // compare-exchanges on (distance, slot)
-        int s0 = 0, s1 = 1, s2 = 2, s3 = 3;
-        auto cx = [](float& ta, int32_t& ca, int& sa, float& tb, int32_t& cb, int& sb) {
-          const bool sw = (ta > tb) | ((ta == tb) & (sa > sb));
-          if (sw) {
-            float tt = ta; ta = tb; tb = tt;
-            int32_t cc = ca; ca = cb; cb = cc;
-            int ss = sa; sa = sb; sb = ss;
-          }
-        };
-        cx(t0, c0r, s0, t1, c1r, s1);
-        cx(t2, c2r, s2, t3, c3r, s3);
-        cx(t0, c0r, s0, t2, c2r, s2);
-        cx(t1, c1r, s1, t3, c3r, s3);
-        cx(t1, c1r, s1, t2, c2r, s2);
-        if (t0 == kInf) {
-          node = pop(tmax);
-        } else {
-          bool ok = true;
-          if (t3 != kInf) ok &= push(c3r, t3);
-          if (t2 != kInf) ok &= push(c2r, t2);
-          if (t1 != kInf) ok &= push(c1r, t1);
-          if (!ok) { atomicOr(c.err, ERR_STACK); node = DONE; leaf = -1; break; }
-          node = c0r;
-        }
-        if ((node < 0) & (node != DONE) & (leaf < 0)) {
-          leaf = ~node;
-          node = pop((float)(h.t + 2 * FTINY) * 1.000001f);
-        }
-        if (__ballot(leaf < 0) == 0ull) break;
-      }
-    }
     const BVHNode* __restrict__ nodes = S.nodes;
-    while (!WIDE && node >= 0) {
+    while (node >= 0) {
       if (++iter > S.nbvh + 8) { atomicOr(c.err, ERR_STACK); node = DONE; leaf = -1; break; }
       const BVHNode N = nodes[node];
       ++nvis;
@@ -1725,7 +1664,7 @@ k_trace_pf(DevScene Sarg, RunCfg c, const RayGeo* geo, const RaySt* st, RayMap m
       TraceOut to;
       to.t = h.t;
       to.prim = h.prim;
-      to.pad = 0;
+      to.front = 0;
       outp[tcur] = to;
       tcur = -1;
     }
@@ -1734,6 +1673,271 @@ k_trace_pf(DevScene Sarg, RunCfg c, const RayGeo* geo, const RaySt* st, RayMap m
     atomicAdd(c.visits, (unsigned long long)nvis);
     atomicAdd(c.visits + 1, (unsigned long long)nprim);
   }
+}
+
+// The room-sized primitives of every ray of a window, ahead of the four-wide
+// walk: the nearest of them (or none) bounds it.  In the walk's refill the
+// same tests ran on the few lanes that had just become idle, a quarter of the
+// walk's instructions; here every lane has a ray.
+template <bool BATCH>
+__global__ void __launch_bounds__(TBLOCK) k_big_first(DevScene Sarg, RunCfg c, const RayGeo* geo, const RaySt* st,
+                                                      RayMap map, TraceOut* outp) {
+  __shared__ float tes[NBIG_ORDER * TBLOCK];
+  uint32_t n;
+  const uint32_t at = map.chunk(blockIdx.x, n) + threadIdx.x;
+  if (threadIdx.x >= n) return;
+  const RayGeo g = geo[at];
+  const DevScene S = scene_of(Sarg, c, BATCH ? st[at].scene : 0);
+  HitRec h;
+  h.t = FHUGE; h.rod = 1.0; h.prim = -1;
+  uint32_t nprim = 0;
+  big_hits<TBLOCK>(S, v3(g.o[0], g.o[1], g.o[2]), v3(g.d[0], g.d[1], g.d[2]), h, nprim, tes + threadIdx.x);
+  TraceOut o;
+  o.t = h.t;
+  o.prim = h.prim;
+  o.front = h.rod > 0.0;
+  outp[blockIdx.x * kChunk + threadIdx.x] = o;
+  if (c.visits) atomicAdd(c.visits + 1, (unsigned long long)nprim);
+}
+
+// Persistent four-wide walk (rays handed out as in k_trace_pf; their first
+// hit comes from k_big_first when the scene has room-sized primitives).
+//
+// One step is either a node (four boxes from 64 bytes, the children hit taken
+// nearest first, the others pushed farthest first) or a leaf (one primitive
+// record, one cache line).  A lane that meets a leaf keeps it and walks on
+// until it meets the next; nodes go on while at least kNodeLanes lanes have
+// one to enter, then every lane with a leaf tests it, so neither kind of step
+// runs for a few lanes at a time.
+//
+// Where two primitives meet within FTINY, rayreject() (rt/raytrace.c:536-575)
+// may keep the one met first; the rounded boxes must not change which that
+// is, so such ties (about one ray in 10^4: edges of adjoining polygons) are
+// decided by the order of the unrounded boxes (hit_leaf_ordered).
+//
+// What bounds it: vector-memory addresses and instruction issue, not bytes.
+// A divergent load costs the texture unit a cycle per lane and 16 bytes, and
+// a node in seven 16-byte loads kept it busy for 16 of 27 ms (2,500-sensor
+// pass); the 64-byte node takes four.  Entry distances are sorted as integers
+// with the child's slot in the low two bits (ten min / max; boxes entered at
+// distances equal in the other 30 bits come in slot order).
+#ifndef RG_NODE_LANES
+#define RG_NODE_LANES 32
+#endif
+#ifndef RG_WALK_WAVES
+#define RG_WALK_WAVES 4
+#endif
+constexpr int WSTACK = RG_LSTACK;                     // walk stack entries per lane in LDS
+constexpr int WDEEP = kTraceStackEntries - WSTACK;    // further entries in private memory
+__device__ __forceinline__ HitRec first_hit_of(bool big, const TraceOut* outp, int32_t t) {
+  HitRec h;
+  h.t = FHUGE; h.rod = 1.0; h.prim = -1; h.tie = 0;
+  if (big) {
+    const TraceOut b = outp[t];
+    h.t = b.t; h.prim = b.prim; h.rod = b.front ? 1.0 : -1.0;
+  }
+  return h;
+}
+template <int BS, bool BATCH>
+__global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(RG_WALK_WAVES)))
+k_walk4(DevScene Sarg, RunCfg c, const RayGeo* geo, const RaySt* st, RayMap map, TraceOut* outp, uint32_t* work,
+        uint32_t refill, uint32_t grab) {
+  __shared__ uint64_t stk[WSTACK * BS];         // (entry distance, child)
+  constexpr int32_t DONE = INT32_MIN;
+  constexpr uint32_t kUnits = kChunk / 64;      // units of 64 rays per chunk
+  constexpr uint32_t kNoHit = 0xffffffffu;
+  const int lane = threadIdx.x;
+  const uint32_t nunit = map.nchunk * kUnits;
+  uint64_t deep[WDEEP];
+  int32_t tcur = -1;              // window index of this lane's ray, -1: idle
+  // wave-uniform: units [u0, u1) still to open, rays [rpos, rend) of the open
+  // range, record index minus window index there, no unit left to take
+  uint32_t u0 = 0, u1 = 0, rpos = 0, rend = 0, rdelta = 0;
+  bool exhausted = false;
+  DevScene S = Sarg;
+  V3 o = v3(0, 0, 0), d = v3(0, 0, 1);
+  HitRec h;
+  h.t = FHUGE; h.rod = 1.0; h.prim = -1; h.tie = 0;
+  int32_t node = DONE, leaf = -1;
+  int sp = 0;
+  float ox = 0, oy = 0, oz = 0, ix = 0, iy = 0, iz = 0, tlim = 0;
+  uint32_t nvis = 0, nprim = 0;
+  auto limit = [](double t) { return (float)(t + 2 * FTINY) * 1.000001f; };
+  // next subtree whose box starts within the current closest hit
+  auto pop = [&]() -> int32_t {
+    while (sp > 0) {
+      --sp;
+      const uint64_t e = sp < WSTACK ? stk[sp * BS + lane] : deep[sp - WSTACK];
+      if (__uint_as_float((uint32_t)(e >> 32)) <= tlim) return (int32_t)(uint32_t)e;
+    }
+    return DONE;
+  };
+  for (;;) {
+    // ---- refill idle lanes ----
+    const unsigned long long idle = __ballot(tcur < 0);
+    const uint32_t nidle = (uint32_t)__popcll(idle);
+    if (!exhausted && (nidle >= refill || nidle == 64u)) {
+      while (rpos >= rend) {
+        if (u0 >= u1) {
+          uint32_t b = 0;
+          if (__lane_id() == 0) b = atomicAdd(work, grab);
+          u0 = __builtin_amdgcn_readfirstlane(b);
+          if (u0 >= nunit) { exhausted = true; break; }
+          u1 = min(u0 + grab, nunit);
+        }
+        const uint32_t ck = u0 / kUnits, ue = min(u1, (ck + 1) * kUnits);
+        uint32_t n;
+        const uint32_t base = map.chunk(ck, n);
+        rdelta = base - ck * kChunk;
+        rpos = u0 * 64u;
+        rend = min(ue * 64u, ck * kChunk + n);
+        u0 = ue;
+      }
+      if (rpos < rend) {
+        const uint32_t take = min(nidle, rend - rpos);
+        const uint32_t rank = lane_rank(idle);
+        if (tcur < 0 && rank < take) {
+          tcur = (int32_t)(rpos + rank);
+          const uint32_t at = rpos + rank + rdelta;
+          const RayGeo g = geo[at];
+          if (BATCH) S = scene_of(Sarg, c, st[at].scene);
+          h = first_hit_of(BATCH || S.nbig > 0, outp, tcur);
+          o = v3(g.o[0], g.o[1], g.o[2]);
+          d = v3(g.d[0], g.d[1], g.d[2]);
+          tlim = limit(h.t);
+          node = 0;
+          leaf = -1;
+          sp = 0;
+          auto inv = [](double v) -> float {
+            float f = (float)v;
+            if (fabsf(f) < 1e-20f) f = f < 0 ? -1e-20f : 1e-20f;
+            return 1.0f / f;
+          };
+          ix = inv(d.x); iy = inv(d.y); iz = inv(d.z);
+          ox = (float)o.x * ix; oy = (float)o.y * iy; oz = (float)o.z * iz;   // origin x inverse direction
+        }
+        rpos += take;
+      }
+    }
+    if (__ballot(tcur >= 0) == 0ull) {
+      if (exhausted) break;
+      continue;
+    }
+    // ---- nodes ----
+    // every node is entered at most once (children follow their parent in
+    // the array), so the walk ends
+    for (;;) {
+      const uint32_t nn = (uint32_t)__popcll(__ballot(node >= 0));
+      if (nn == 0u || (nn < RG_NODE_LANES && __ballot(leaf >= 0))) break;
+      if (node >= 0) {
+        const RG_GLOBAL u32x4* np = (const RG_GLOBAL u32x4*)(S.nodes4 + node);
+        const u32x4 w0 = np[0], w1 = np[1], w2 = np[2], w3 = np[3];
+        ++nvis;
+        const float gx = __uint_as_float(w0[0]), gy = __uint_as_float(w0[1]), gz = __uint_as_float(w0[2]);
+        const float sx = __uint_as_float(w0[3]), sy = __uint_as_float(w1[0]), sz = __uint_as_float(w1[1]);
+        const bool mx = ix < 0.f, my = iy < 0.f, mz = iz < 0.f;
+        const uint32_t nx = mx ? w1[3] : w1[2], fx = mx ? w1[2] : w1[3];
+        const uint32_t ny = my ? w2[1] : w2[0], fy = my ? w2[0] : w2[1];
+        const uint32_t nz = mz ? w2[3] : w2[2], fz = mz ? w2[2] : w2[3];
+        const float ax = sx * ix, ay = sy * iy, az = sz * iz;
+        const float bx = fmaf(gx, ix, -ox), by = fmaf(gy, iy, -oy), bz = fmaf(gz, iz, -oz);
+        uint32_t key[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          auto byte = [&](uint32_t v) { return (float)((v >> (8 * k)) & 255u); };
+          const float tn = fmaxf(fmaxf(fmaxf(fmaf(byte(nx), ax, bx), fmaf(byte(ny), ay, by)), fmaf(byte(nz), az, bz)), 0.f);
+          const float tf = fminf(fminf(fminf(fmaf(byte(fx), ax, bx), fmaf(byte(fy), ay, by)), fmaf(byte(fz), az, bz)), tlim);
+          const bool hit = (tn <= tf) & ((int32_t)w3[k] != DONE);
+          key[k] = hit ? ((__float_as_uint(tn) & ~3u) | (uint32_t)k) : kNoHit;
+        }
+        auto cx = [&](int a, int b) {
+          const uint32_t lo = min(key[a], key[b]), hi = max(key[a], key[b]);
+          key[a] = lo;
+          key[b] = hi;
+        };
+        cx(0, 1); cx(2, 3); cx(0, 2); cx(1, 3); cx(1, 2);
+        auto child = [&](uint32_t k) -> uint32_t {
+          const uint32_t a = (k & 1u) ? w3[1] : w3[0], b = (k & 1u) ? w3[3] : w3[2];
+          return (k & 2u) ? b : a;
+        };
+        if (key[0] == kNoHit) {
+          node = pop();
+        } else {
+          node = (int32_t)child(key[0]);
+          if (key[1] != kNoHit) {
+            auto entry = [&](uint32_t k) { return ((uint64_t)(k & ~3u) << 32) | child(k); };
+            const uint64_t e1 = entry(key[1]), e2 = entry(key[2]), e3 = entry(key[3]);
+            const int h2 = key[2] != kNoHit, h3 = key[3] != kNoHit;
+            if (sp <= WSTACK - 3) {
+              // farthest first; a slot that is not used is overwritten
+              stk[sp * BS + lane] = e3;
+              stk[(sp + h3) * BS + lane] = e2;
+              stk[(sp + h3 + h2) * BS + lane] = e1;
+              sp += 1 + h2 + h3;
+            } else {
+              bool ok = true;
+              auto push = [&](uint64_t e) {
+                if (sp < WSTACK) stk[sp * BS + lane] = e;
+                else if (sp < WSTACK + WDEEP) deep[sp - WSTACK] = e;
+                else { ok = false; return; }
+                ++sp;
+              };
+              if (h3) push(e3);
+              if (h2) push(e2);
+              push(e1);
+              if (!ok) { atomicOr(c.err, ERR_STACK); node = DONE; leaf = -1; }
+            }
+          }
+        }
+        if ((node < 0) & (node != DONE) & (leaf < 0)) {
+          leaf = ~node;
+          node = pop();
+        }
+      }
+    }
+    // ---- leaves ----
+    if (leaf >= 0) {
+      const RG_GLOBAL u32x4* lp = (const RG_GLOBAL u32x4*)(S.leafs + leaf);
+      LeafRec L;
+      {
+        const u32x4 l0 = lp[0], l1 = lp[1], l2 = lp[2], l3 = lp[3], l4 = lp[4], l5 = lp[5], l6 = lp[6];
+        const u32x4 lv[7] = {l0, l1, l2, l3, l4, l5, l6};
+        __builtin_memcpy(&L, lv, sizeof lv);
+      }
+      const float ot[3] = {ox, oy, oz}, iv[3] = {ix, iy, iz};
+      hit_leaf_ordered(S, L, leaf, o, d, ot, iv, h);
+      tlim = limit(h.t);
+      ++nprim;
+      leaf = -1;
+      if ((node < 0) & (node != DONE)) {
+        leaf = ~node;
+        node = pop();
+      }
+    }
+    // ---- finished rays: write the record, free the lane ----
+    if ((tcur >= 0) & (node == DONE) & (leaf < 0)) {
+      TraceOut to;
+      to.t = h.t;
+      to.prim = h.prim;
+      to.front = 0;
+      outp[tcur] = to;
+      tcur = -1;
+    }
+  }
+  if (c.visits) {
+    atomicAdd(c.visits, (unsigned long long)nvis);
+    atomicAdd(c.visits + 1, (unsigned long long)nprim);
+  }
+}
+
+__global__ void __launch_bounds__(TBLOCK) k_leaf_recs(DevScene S, const int32_t* pos, LeafRec* out) {
+  const uint32_t i = blockIdx.x * TBLOCK + threadIdx.x;
+  if (i < (uint32_t)S.nprims) out[i] = leaf_rec(S, (int)i, pos[i]);
+}
+
+void leaf_records(const DevScene& S, const int32_t* d_pos, LeafRec* d_out, hipStream_t st) {
+  hipLaunchKernelGGL(k_leaf_recs, dim3((S.nprims + TBLOCK - 1) / TBLOCK), dim3(TBLOCK), 0, st, S, d_pos, d_out);
+  if (hipGetLastError() != hipSuccess) throw std::runtime_error("k_leaf_recs launch");
 }
 
 static void check(hipError_t e, const char* what) {
@@ -2327,10 +2531,18 @@ void render(const DevScene& S, RunCfg cfg, const double* d_rays, uint32_t nsens,
         auto go = [&](auto kern) {
           hipLaunchKernelGGL(kern, dim3(nb), dim3(TBLOCK), 0, st, S, cfg, geo, rst, map, tout, work, tn.refill, grab);
         };
-        if (cfg.nscenes && tn.wide) go(k_trace_pf<TBLOCK, true, true>);
-        else if (cfg.nscenes) go(k_trace_pf<TBLOCK, true, false>);
-        else if (tn.wide) go(k_trace_pf<TBLOCK, false, true>);
-        else go(k_trace_pf<TBLOCK, false, false>);
+        if (tn.wide && cfg.nscenes) {
+          hipLaunchKernelGGL(k_big_first<true>, dim3(map.nchunk), dim3(TBLOCK), 0, st, S, cfg, geo, rst, map, tout);
+          go(k_walk4<TBLOCK, true>);
+        } else if (tn.wide) {
+          if (S.nbig)
+            hipLaunchKernelGGL(k_big_first<false>, dim3(map.nchunk), dim3(TBLOCK), 0, st, S, cfg, geo, rst, map, tout);
+          go(k_walk4<TBLOCK, false>);
+        } else if (cfg.nscenes) {
+          go(k_trace_pf<TBLOCK, true>);
+        } else {
+          go(k_trace_pf<TBLOCK, false>);
+        }
       } else {
         hipLaunchKernelGGL(k_trace, dim3(map.nchunk), dim3(TBLOCK), 0, st, S, cfg, geo, rst, map, tout);
       }
@@ -2381,7 +2593,7 @@ void render(const DevScene& S, RunCfg cfg, const double* d_rays, uint32_t nsens,
   if (stats) {
     stats->generations = gens;
     stats->rays = traced;
-    stats->node_bytes = (tn.trace_kernel == 1 && tn.wide) ? (int)sizeof(BVH4Node) : (int)sizeof(BVHNode);
+    stats->node_bytes = (tn.trace_kernel == 1 && tn.wide) ? (int)sizeof(BVH4Q) : (int)sizeof(BVHNode);
   }
 }
 

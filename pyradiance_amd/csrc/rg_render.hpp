@@ -72,7 +72,7 @@ struct RenderStats {
   bool timing = false;       // time every generation's kernels with HIP events
   double bounce_ms = 0;      // summed traversal-kernel (k_trace) durations
   double shade_ms = 0;       // summed shading-kernel (k_shade) durations
-  int node_bytes = 64;       // bytes of one tree node the traversal fetched (64 binary, 128 four-wide)
+  int node_bytes = 64;       // bytes of one tree node the traversal fetched
 };
 
 // Per-lane traversal stack entries (LDS and private memory together).
@@ -98,6 +98,10 @@ struct Tuning {
 // spawn buffers); S.nsrcs is used when that is larger.
 void render(const DevScene& S, RunCfg cfg, const double* d_rays, uint32_t nsens, bool imm_irrad, int max_srcs,
             const Tuning& tn, DevArena& arena, hipStream_t st, RenderStats* stats);
+
+// Leaf records of all primitives of a scene (LeafRec); d_pos: their places
+// among the tree's leaves.
+void leaf_records(const DevScene& S, const int32_t* d_pos, LeafRec* d_out, hipStream_t st);
 
 // First intersection of n rays (n x 6 doubles): distance (FHUGE on a miss),
 // unflipped normal (n x 3), primitive index (-1 on a miss).
