@@ -12,6 +12,7 @@
 // mode 0: plain FP32 FMA, tiled through LDS (accuracy baseline).
 #include <hip/hip_runtime.h>
 #include <mutex>
+#include <type_traits>
 #include "rg_render.hpp"
 
 namespace rg {
@@ -178,107 +179,208 @@ __global__ void __launch_bounds__(DB) k_dcsky_mfma(const unsigned short* Ah, con
   }
 }
 
-// LDS-staged form.  A block of 16 wavefronts (4 x 4) computes a
-// 128 x 128 tile of all three channels; each wavefront holds a 32 x 32 tile
-// (2 x 2 MFMA tiles x 3 channels of accumulators).  For each K step of 32
-// and channel, the block's A and B hi/lo tiles (128 rows x 32 K each, 32 KB)
-// are loaded once into LDS and read by all 16 wavefronts; the next stage's
-// global loads are issued before the current stage's MFMAs, into the second
-// LDS buffer.  Rows are padded to 40 bf16 so the 16 lanes that read one
-// fragment column hit different banks.
+// Ring form for long K.  A block of four wavefronts (2 x 2) computes a
+// 128 x 128 tile of all three channels, each wavefront 64 x 64 of it (4 x 4
+// MFMA tiles x 3 channels of accumulators: 192 registers).  A stage is one
+// channel of one K step of 32: the A and B hi/lo tiles (128 rows x 32 K, 8 KB
+// each), loaded straight into LDS by global_load_lds (no staging registers)
+// into a ring of four buffers, three stages ahead of their use.  Fragments
+// are read one stage ahead into a second register set, so a stage is 48 MFMAs
+// with the next stage's 16 LDS reads and the fourth's 8 loads between them,
+// and one barrier.
+//
+// The operands are laid out for it by k_split_tiled: a stage's tile of one
+// plane is 8 KB in one piece, so a load instruction fetches eight whole cache
+// lines.  (From row-major planes it fetched sixteen half lines, and the
+// texture unit, 61 cycles per instruction, was busy 80 % of the time.)
+// 20000 x 2306 x 8760: 6.9 ms, 1.05 PFLOP/s issued, where 128 x 128 tiles of
+// 32 x 32 per wavefront staged through registers took 10.5 ms; matrix cores
+// busy 54 % of the cycles, at a clock that falls to 1.9 GHz.  The
+// 16-byte parts of a row sit at part ^ ((row >> 1) & 3): the eight lanes that
+// read LDS together (same part, consecutive rows of 64 bytes) then cover
+// eight different 16-byte columns of the banks.
 constexpr int LBM = 128, LBN = 128;
-#ifndef RG_DCSKY_LKS
-#define RG_DCSKY_LKS 64
-#endif
-constexpr int LKS = RG_DCSKY_LKS;             // K per stage (32 or 64; 64 measured 22-28 % faster at K = 2306)
-constexpr int LROW = LKS + 8;                 // padded row length (bf16)
-constexpr int LTILE = 128 * LROW;             // one 128 x LKS plane tile in LDS (bf16)
-constexpr int LCPR = LKS / 8;                 // 16-byte chunks per tile row
+constexpr int RING = 4;                       // stages in LDS
+constexpr int RPLANE = 128 * 32;              // one plane of a stage (bf16)
 
-// WM x WN wavefronts, each holding TA x TB 16 x 16 MFMA tiles of all three
-// channels (16 * TA * WM = 16 * TB * WN = 128).
-template <int WM, int WN, int TA, int TB>
-__global__ void __launch_bounds__(64 * WM * WN) k_dcsky_lds(const unsigned short* Ah, const unsigned short* Al,
-                                                            const unsigned short* Bh, const unsigned short* Bl,
-                                                            float* C, int M, int N, int Kp, int Mt, int Nt) {
-  static_assert(16 * TA * WM == LBM && 16 * TB * WN == LBN, "block tile");
-  constexpr int NT = 64 * WM * WN;
-  constexpr int NCH = 4 * 128 * LCPR / NT;    // 16-byte chunks each thread stages per stage
-  __shared__ __attribute__((aligned(16))) unsigned short lds[2][4][LTILE];   // [buffer][Ah, Al, Bh, Bl]
+// Operands to tiled hi/lo planes: [channel][tile of 128 rows][K step of 32]
+// [row][part swizzled][8], rows and K zero-padded.  A wavefront takes 16 rows
+// of one K step in all three channels: 1,536 floats, read in runs of 96 (a row
+// of A) or 48 (a K row of B) consecutive ones and turned in LDS, so that each
+// lane then holds eight K of one row; its six stores are 1 KB in one piece
+// over the wavefront.  (Lanes reading their own 24 floats from memory touched
+// 64 lines per load: 568 against 294 us for both operands of the largest
+// product, 20000 x 2306 x 8760.)  Blocks [0, nba) split A[M][K][3], the others B[K][N][3].
+constexpr int TROW = 97;                      // padded row in LDS (floats)
+__global__ void __launch_bounds__(256) k_split_tiled(const float* A, const float* B, int M, int K, int N, int nk,
+                                                     int Mt, int Nt, unsigned nba, unsigned short* Ah,
+                                                     unsigned short* Al, unsigned short* Bh, unsigned short* Bl) {
+  __shared__ float turn[4][16 * TROW];
+  const bool isb = blockIdx.x >= nba;
+  const size_t g = ((size_t)(isb ? blockIdx.x - nba : blockIdx.x) * 256 + threadIdx.x) >> 6;   // wavefront
+  const int lane = threadIdx.x & 63, T = isb ? Nt : Mt, R = isb ? N : M;
+  float* tl = turn[threadIdx.x >> 6];
+  // wavefront -> (K step, group of 16 rows): A walks K first (a row's steps
+  // follow each other in memory), B walks the rows
+  const int groups = T * 8;
+  if (g >= (size_t)groups * nk) return;
+  const int ks = (int)(isb ? g / groups : g % nk), rg = (int)(isb ? g % groups : g / nk);
+  float x[24];
+#pragma unroll
+  for (int j = 0; j < 24; ++j) {
+    const int i = j * 64 + lane;
+    int r, e;                                 // row, 3 x K + channel within the tile
+    size_t at;
+    if (isb) {
+      const int k = i / 48, q = i % 48;
+      r = q / 3;
+      e = 3 * k + q % 3;
+      at = ((size_t)(ks * 32 + k) * N + rg * 16) * 3 + q;
+    } else {
+      r = i / 96;
+      e = i % 96;
+      at = ((size_t)(rg * 16 + r) * K + ks * 32) * 3 + e;
+    }
+    x[j] = (rg * 16 + r < R && ks * 32 + e / 3 < K) ? (isb ? B : A)[at] : 0.0f;
+  }
+#pragma unroll
+  for (int j = 0; j < 24; ++j) {
+    const int i = j * 64 + lane;
+    const int k = i / 48, q = i % 48;
+    tl[isb ? (q / 3) * TROW + 3 * k + q % 3 : (i / 96) * TROW + i % 96] = x[j];
+  }
+  __builtin_amdgcn_wave_barrier();            // one wavefront's own LDS, in order
+  const int row = rg * 16 + (lane >> 2), part = lane & 3;
+  const float* mine = tl + (lane >> 2) * TROW + part * 24;
+  unsigned short* H = isb ? Bh : Ah;
+  unsigned short* L = isb ? Bl : Al;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    u16x8 h, l;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float v = mine[3 * j + c];
+      const unsigned short u = f2bf(v);
+      h[j] = u;
+      l[j] = f2bf(v - bf2f(u));
+    }
+    const size_t o = (((size_t)c * T + (row >> 7)) * nk + ks) * RPLANE + (row & 127) * 32 + (part ^ ((row >> 1) & 3)) * 8;
+    *(u16x8*)(H + o) = h;
+    *(u16x8*)(L + o) = l;
+  }
+}
+
+// Every LDS read of this wavefront done, at most N of its loads under way,
+// then the block's barrier.
+template <int N>
+__device__ __forceinline__ void ring_wait() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory");
+}
+
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+k_dcsky_ring(const unsigned short* Ah, const unsigned short* Al, const unsigned short* Bh, const unsigned short* Bl,
+             float* C, int M, int N, int nkall, int Mt, int Nt) {
+  __shared__ __attribute__((aligned(16))) unsigned short lds[RING][4][RPLANE];   // [buffer][Ah, Al, Bh, Bl]
   int tm, tn;
   if (!tile_of(Mt, Nt, tm, tn)) return;
-  const int t = threadIdx.x;
-  const int lane = t & 63, wave = t >> 6;
-  const int wm = wave / WN, wn = wave % WN;
-  const int r16 = lane & 15, kq = (lane >> 4) * 8;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const int r16 = lane & 15;
   const int mb = tm * LBM, nb = tn * LBN;
-  // staging: chunk q (16 B = 8 bf16) of the stage: plane q / (128 LCPR),
-  // row (q mod 128 LCPR) / LCPR, part q mod LCPR
-  int soff[NCH], splane[NCH];
-  size_t sg[NCH];
-  const size_t csz[4] = {(size_t)M * Kp, (size_t)M * Kp, (size_t)N * Kp, (size_t)N * Kp};
-  for (int j = 0; j < NCH; ++j) {
-    const int q = t + j * NT;
-    const int pl = q / (128 * LCPR), row = (q % (128 * LCPR)) / LCPR, part = q % LCPR;
-    splane[j] = pl;
-    soff[j] = row * LROW + part * 8;
-    sg[j] = (pl < 2 ? (size_t)min(mb + row, M - 1) : (size_t)min(nb + row, N - 1)) * Kp + part * 8;
-  }
-  const unsigned short* planes[4] = {Ah, Al, Bh, Bl};
-  auto gload = [&](int stage, u16x8* reg) {
-    const int k0 = (stage / 3) * LKS, c = stage % 3;
-    for (int j = 0; j < NCH; ++j) reg[j] = *(const u16x8*)(planes[splane[j]] + c * csz[splane[j]] + sg[j] + k0);
+  // this block's share of the K steps and, when K is split, its own partial C
+  const int kb = (int)((long long)nkall * blockIdx.y / gridDim.y);
+  const int nk = (int)((long long)nkall * (blockIdx.y + 1) / gridDim.y) - kb;
+  C += (size_t)blockIdx.y * M * N * 3;
+  // this wavefront stages plane `wave`; stage s is channel s % 3 of K step
+  // s / 3.  Past the end the last stage is loaded again, so that the counts
+  // of loads under way stay the same
+  const int T = wave < 2 ? Mt : Nt, t = wave < 2 ? tm : tn;
+  const unsigned short* src = (wave == 0 ? Ah : (wave == 1 ? Al : (wave == 2 ? Bh : Bl))) +
+                              ((size_t)t * nkall + kb) * RPLANE;
+  const size_t cstep = (size_t)T * nkall * RPLANE;   // next channel
+  const int lo8 = lane * 8;
+  int left = 3 * nk, lc = 0;
+  auto load_part = [&](int buf, int j) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + j * 512 + lo8),
+                                     (__attribute__((address_space(3))) void*)&lds[buf][wave][j * 512], 16, 0, 0);
   };
-  auto lstore = [&](int buf, const u16x8* reg) {
-    for (int j = 0; j < NCH; ++j) *(u16x8*)&lds[buf][splane[j]][soff[j]] = reg[j];
+  auto next_stage = [&]() {
+    if (--left <= 0) return;
+    if (lc == 2) { src += RPLANE; src -= 2 * cstep; lc = 0; }
+    else { src += cstep; ++lc; }
   };
-  f32x4 acc[3][TA][TB];
-  for (int c = 0; c < 3; ++c)
-    for (int a = 0; a < TA; ++a)
-      for (int b = 0; b < TB; ++b) acc[c][a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int nstage = 3 * (Kp / LKS);
-  u16x8 reg[NCH];
-  gload(0, reg);
-  lstore(0, reg);
-  __syncthreads();
-  for (int s = 0; s < nstage; ++s) {
-    const int buf = s & 1;
-    if (s + 1 < nstage) gload(s + 1, reg);
-    const int c = s % 3;
+  f32x4 acc[3][4][4];
 #pragma unroll
-    for (int kk = 0; kk < LKS; kk += 32) {
-      bf16x8 fah[TA], fal[TA], fbh[TB], fbl[TB];
-      for (int a = 0; a < TA; ++a) {
-        const int row = wm * 16 * TA + 16 * a + r16;
-        fah[a] = __builtin_bit_cast(bf16x8, *(const u16x8*)&lds[buf][0][row * LROW + kk + kq]);
-        fal[a] = __builtin_bit_cast(bf16x8, *(const u16x8*)&lds[buf][1][row * LROW + kk + kq]);
-      }
-      for (int b = 0; b < TB; ++b) {
-        const int row = wn * 16 * TB + 16 * b + r16;
-        fbh[b] = __builtin_bit_cast(bf16x8, *(const u16x8*)&lds[buf][2][row * LROW + kk + kq]);
-        fbl[b] = __builtin_bit_cast(bf16x8, *(const u16x8*)&lds[buf][3][row * LROW + kk + kq]);
-      }
-      for (int a = 0; a < TA; ++a)
-        for (int b = 0; b < TB; ++b) {
-          f32x4 v = c == 0 ? acc[0][a][b] : (c == 1 ? acc[1][a][b] : acc[2][a][b]);
-          v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fbh[b], fah[a], v, 0, 0, 0);
-          v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fbl[b], fah[a], v, 0, 0, 0);
-          v = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fbh[b], fal[a], v, 0, 0, 0);
-          if (c == 0) acc[0][a][b] = v;
-          else if (c == 1) acc[1][a][b] = v;
-          else acc[2][a][b] = v;
-        }
-    }
-    if (s + 1 < nstage) lstore(buf ^ 1, reg);
-    __syncthreads();
+  for (int c = 0; c < 3; ++c)
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) acc[c][a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int part = (((lane >> 4) ^ ((r16 >> 1) & 3))) * 8;
+  const int ra = (wm * 64 + r16) * 32 + part, rb = (wn * 64 + r16) * 32 + part;
+  // fragments [set][plane: Ah, Al, Bh, Bl][tile]
+  bf16x8 fr[2][4][4];
+  auto read_frag = [&](int buf, int f, int i) {       // i = 4 x tile + plane
+    const int pl = i & 3, q = i >> 2;
+    fr[f][pl][q] = ld8(&lds[buf][pl][(pl < 2 ? ra : rb) + q * 512]);
+  };
+#pragma unroll
+  for (int s = 0; s < RING; ++s) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) load_part(s, j);
+    next_stage();
   }
+  ring_wait<8 * (RING - 1)>();
+#pragma unroll
+  for (int i = 0; i < 16; ++i) read_frag(0, 0, i);
+  // One K step (three stages).  J: its place among four, which settles each
+  // stage's buffer and register set at compile time (12 stages = 3 channels x
+  // 4 buffers).  The loop runs whole groups of four; leaving it in between
+  // would copy all accumulators at every exit.
+  auto kstep = [&](auto J) {
+#pragma unroll
+    for (int q = 3 * decltype(J)::value; q < 3 * decltype(J)::value + 3; ++q) {
+      const int c = q % 3, buf = q % RING, f = q & 1;
+      // stage s + 1 is in LDS for everyone, and everyone has read stage s
+      ring_wait<8 * (RING - 2)>();
+#pragma unroll
+      for (int g = 0; g < 8; ++g) {
+        load_part(buf, g);
+        if (g < 6)
+#pragma unroll
+          for (int i = 0; i < 3; ++i)
+            if (3 * g + i < 16) read_frag((buf + 1) % RING, f ^ 1, 3 * g + i);
+#pragma unroll
+        for (int i = 6 * g; i < 6 * g + 6; ++i) {
+          const int p = i / 16, a = (i / 4) & 3, b = i & 3;    // hi hi, lo hi, hi lo
+          acc[c][a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fr[f][p == 1 ? 3 : 2][b], fr[f][p == 2 ? 1 : 0][a],
+                                                                 acc[c][a][b], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      next_stage();
+    }
+  };
+  for (int k = 0; k < nk / 4; ++k) {
+    kstep(std::integral_constant<int, 0>());
+    kstep(std::integral_constant<int, 1>());
+    kstep(std::integral_constant<int, 2>());
+    kstep(std::integral_constant<int, 3>());
+  }
+  if ((nk & 3) > 0) kstep(std::integral_constant<int, 0>());
+  if ((nk & 3) > 1) kstep(std::integral_constant<int, 1>());
+  if ((nk & 3) > 2) kstep(std::integral_constant<int, 2>());
+  // the loads still under way write LDS: the block must not end before them
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   // D layout: lane holds D[n = 4 * (lane >> 4) + i][m = lane & 15]
   const bool vec = (N & 3) == 0;
-  for (int a = 0; a < TA; ++a) {
-    const int m = mb + wm * 16 * TA + 16 * a + r16;
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const int m = mb + wm * 64 + 16 * a + r16;
     if (m >= M) continue;
-    for (int b = 0; b < TB; ++b) {
-      const int nq = nb + wn * 16 * TB + 16 * b + (lane >> 4) * 4;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const int nq = nb + wn * 64 + 16 * b + (lane >> 4) * 4;
       if (nq >= N) continue;
       float* dst = C + ((size_t)m * N + nq) * 3;
       const f32x4 r = acc[0][a][b], g = acc[1][a][b], u = acc[2][a][b];
@@ -296,6 +398,26 @@ __global__ void __launch_bounds__(64 * WM * WN) k_dcsky_lds(const unsigned short
       }
     }
   }
+}
+
+// Sum of the partial products of a split K, in order.
+__global__ void __launch_bounds__(256) k_dcsky_sum(const float* part, float* C, size_t n, int parts) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  float v = part[i];
+  for (int p = 1; p < parts; ++p) v += part[(size_t)p * n + i];
+  C[i] = v;
+}
+
+// Parts the K steps of the ring form are split into: with fewer tiles than
+// compute units the others would idle for the whole K (3 tiles of K = 2306:
+// 133 us; in 18 parts 51 us), so K is shared by as many blocks as there
+// are units for, at least four steps each.  From half as many tiles as units
+// on a second round would cost what the split saves.
+static int ring_parts(long long tiles, int nk) {
+  int dev = 0, ncu = 256;
+  if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+  return (int)std::max<long long>(1, std::min<long long>(ncu / tiles, nk / 4));
 }
 
 // Short-K form (K <= 160, e.g. 146 Klems patches): the product is bound by
@@ -546,15 +668,33 @@ void dcsky(const float* A, const float* B, float* C, int M, int K, int N, int mo
   if (mode == 4 && k32 > 32 * SHORT_KS) throw std::runtime_error("dcsky: mode 4 needs K <= 160");
   const bool shortk = mode == 4 || (mode == 1 && k32 <= 32 * SHORT_KS);
   const bool staged = !shortk && (mode == 3 || (mode == 1 && K > 256));
-  const int kstep = staged ? LKS : 32;
-  int Kp = (K + kstep - 1) / kstep * kstep;
-  size_t na = (size_t)3 * M * Kp, nb = (size_t)3 * N * Kp;
+  const int Kp = k32;
+  const int Mt = (M + LBM - 1) / LBM, Nt = (N + LBN - 1) / LBN;      // the ring form's tiles
+  const size_t na = (size_t)3 * (staged ? Mt * LBM : M) * Kp, nb = (size_t)3 * (staged ? Nt * LBN : N) * Kp;
   std::lock_guard<std::mutex> lk(g_dc_mu);
-  // split planes, then (16-byte aligned) the short form's output sink
+  // split planes, then (16-byte aligned) the short form's output sink or a
+  // split K's partial products
   const size_t plane_bytes = (2 * (na + nb) * sizeof(unsigned short) + 255) / 256 * 256;
-  unsigned short* buf = dc_scratch(plane_bytes + SINK_FLOATS * sizeof(float), st);
+  const int parts = staged ? ring_parts((long long)Mt * Nt, Kp / 32) : 1;
+  const size_t tail_bytes = std::max((size_t)SINK_FLOATS, parts > 1 ? (size_t)parts * M * N * 3 : 0) * sizeof(float);
+  unsigned short* buf = dc_scratch(plane_bytes + tail_bytes, st);
   unsigned short *Ah = buf, *Al = buf + na, *Bh = buf + 2 * na, *Bl = buf + 2 * na + nb;
   float* sink = (float*)((char*)buf + plane_bytes);
+  if (staged) {
+    const int nk = Kp / 32;
+    const size_t nba = ((size_t)Mt * 8 * nk + 3) / 4, nbb = ((size_t)Nt * 8 * nk + 3) / 4;
+    const long long tiles = (long long)Mt * Nt;
+    if (nba + nbb > 0x7fffffffu || tiles > 0x7fffffffLL - 8) throw std::runtime_error("dcsky: matrix too large");
+    hipLaunchKernelGGL(k_split_tiled, dim3((unsigned)(nba + nbb)), dim3(256), 0, st, A, B, M, K, N, nk, Mt, Nt,
+                       (unsigned)nba, Ah, Al, Bh, Bl);
+    hipLaunchKernelGGL(k_dcsky_ring, dim3((unsigned)((tiles + 7) / 8 * 8), (unsigned)parts), dim3(256), 0, st, Ah, Al,
+                       Bh, Bl, parts > 1 ? sink : C, M, N, nk, Mt, Nt);
+    if (parts > 1) {
+      const size_t n = (size_t)M * N * 3;
+      hipLaunchKernelGGL(k_dcsky_sum, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, sink, C, n, parts);
+    }
+    return;
+  }
   const size_t nba = (na + 255) / 256, nbb = (size_t)((N + 31) / 32) * (Kp / 32);
   if (nba + nbb > 0x7fffffffu) throw std::runtime_error("dcsky: matrix too large");
   hipLaunchKernelGGL(k_split, dim3((unsigned)(nba + nbb)), dim3(256), 0, st, A, B, M, K, N, Kp, (unsigned)nba, Ah, Al,
@@ -567,19 +707,12 @@ void dcsky(const float* A, const float* B, float* C, int M, int K, int N, int mo
       case 4: launch_short<4>(Ah, Al, Bh, Bl, C, sink, M, N, st); break;
       default: launch_short<5>(Ah, Al, Bh, Bl, C, sink, M, N, st); break;
     }
-  } else if (!staged) {
-    const int Mt = (M + BM - 1) / BM, Nt = (N + BN - 1) / BN;
-    const long long tiles = (long long)Mt * Nt;
-    if (tiles > 0x7fffffffLL - 8) throw std::runtime_error("dcsky: matrix too large");
-    const unsigned nblk = (unsigned)((tiles + 7) / 8 * 8);
-    hipLaunchKernelGGL(k_dcsky_mfma, dim3(nblk), dim3(DB), 0, st, Ah, Al, Bh, Bl, C, M, N, Kp, Mt, Nt);
   } else {
-    const int Mt = (M + LBM - 1) / LBM, Nt = (N + LBN - 1) / LBN;
-    const long long tiles = (long long)Mt * Nt;
+    const int Wt = (M + BM - 1) / BM, Vt = (N + BN - 1) / BN;
+    const long long tiles = (long long)Wt * Vt;
     if (tiles > 0x7fffffffLL - 8) throw std::runtime_error("dcsky: matrix too large");
     const unsigned nblk = (unsigned)((tiles + 7) / 8 * 8);
-    hipLaunchKernelGGL((k_dcsky_lds<4, 4, 2, 2>), dim3(nblk), dim3(1024), 0, st, Ah, Al, Bh, Bl, C, M, N, Kp, Mt,
-                       Nt);
+    hipLaunchKernelGGL(k_dcsky_mfma, dim3(nblk), dim3(DB), 0, st, Ah, Al, Bh, Bl, C, M, N, Kp, Wt, Vt);
   }
 }
 

@@ -610,3 +610,27 @@ def test_path_records_follow_their_rays_through_every_window(L):
     assert scale > 0
     for g in res[1:]:
         assert np.abs(g - res[0]).max() <= 1e-11 * scale
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 257, 1), (127, 288, 129), (128, 289, 128), (129, 320, 127), (300, 2306, 4),
+                                   (33, 384, 1157), (2049, 352, 2051), (1500, 578, 1408)])
+def test_long_k_product_at_tile_and_split_edges(L, m, k, n):
+    """The ring form of the K > 256 product: tile remainders in both
+    directions, K steps that do and do not fill a group of four, K shared by
+    many blocks and by one, sky columns that do and do not allow 16-byte
+    stores.  Operands are positive, so every term's relative error bounds the
+    sum's: the dropped lo x lo part and the rounding of lo are each at most
+    2^-16 of a term (hi and lo hold 8 bits each), twice over both operands,
+    and the FP32 sum adds at most K 2^-24."""
+    import torch
+    _say(f"long-K product {m} x {k} x {n}")
+    g = torch.Generator(device="cuda").manual_seed(m + k + n)
+    a = torch.rand((m, k, 3), generator=g, device="cuda")
+    b = torch.exp(torch.randn((k, n, 3), generator=g, device="cuda"))
+    c = torch.full((m, n, 3), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    L.dcsky_device(a.data_ptr(), b.data_ptr(), c.data_ptr(), m, k, n)
+    for ch in range(3):
+        ref = a[:, :, ch].double().contiguous() @ b[:, :, ch].double().contiguous()
+        rel = ((c[:, :, ch].double() - ref) / ref).abs().max().item()
+        assert rel <= 3 * 2.0 ** -16 + k * 2.0 ** -24, (ch, rel)
