@@ -5,10 +5,9 @@
 // mode 1 (default): BF16 MFMA with split operands.  Each FP32 value x is
 // carried as hi = bf16(x), lo = bf16(x - hi); the product is accumulated in
 // FP32 as hi*hi + hi*lo + lo*hi, which leaves a relative error near 2^-16
-// per term instead of bf16's 2^-8.  v_mfma_f32_16x16x32_bf16 (gfx950) does
-// the products; both operands are first re-laid out K-contiguous per channel
-// so every lane fetches its 8 bf16 values with one 16-byte load, and the next
-// K step is fetched while the current one is on the matrix cores.
+// per term instead of bf16's 2^-8.  gfx950's double-rate bf16 MFMAs do the
+// products; both operands are first re-laid out K-contiguous per channel, in
+// the tiles the product kernels load whole.
 // mode 0: plain FP32 FMA, tiled through LDS (accuracy baseline).
 #include <hip/hip_runtime.h>
 #include <mutex>
@@ -19,6 +18,7 @@ namespace rg {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
 
 __device__ __forceinline__ unsigned short f2bf(float f) {   // round to nearest even
@@ -180,12 +180,14 @@ __global__ void __launch_bounds__(DB) k_dcsky_mfma(const unsigned short* Ah, con
 }
 
 // Ring form for long K.  A block of four wavefronts (2 x 2) computes a
-// 128 x 128 tile of all three channels, each wavefront 64 x 64 of it (4 x 4
-// MFMA tiles x 3 channels of accumulators: 192 registers).  A stage is one
+// 128 x 128 tile of all three channels, each wavefront 64 x 64 of it (2 x 2
+// MFMA tiles x 3 channels of accumulators: 192 registers).  The 32 x 32 x 16
+// MFMA, because there is one wavefront per SIMD: alone it issues 2.2 PFLOP/s
+// of them, but only 1.3 of 16 x 16 x 32 (measured, independent products).  A stage is one
 // channel of one K step of 32: the A and B hi/lo tiles (128 rows x 32 K, 8 KB
 // each), loaded straight into LDS by global_load_lds (no staging registers)
 // into a ring of four buffers, three stages ahead of their use.  Fragments
-// are read one stage ahead into a second register set, so a stage is 48 MFMAs
+// are read one stage ahead into a second register set, so a stage is 24 MFMAs
 // with the next stage's 16 LDS reads and the fourth's 8 loads between them,
 // and one barrier.
 //
@@ -285,7 +287,7 @@ k_dcsky_ring(const unsigned short* Ah, const unsigned short* Al, const unsigned 
   if (!tile_of(Mt, Nt, tm, tn)) return;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave >> 1, wn = wave & 1;
-  const int r16 = lane & 15;
+  const int r32 = lane & 31;
   const int mb = tm * LBM, nb = tn * LBN;
   // this block's share of the K steps and, when K is split, its own partial C
   const int kb = (int)((long long)nkall * blockIdx.y / gridDim.y);
@@ -309,20 +311,18 @@ k_dcsky_ring(const unsigned short* Ah, const unsigned short* Al, const unsigned 
     if (lc == 2) { src += RPLANE; src -= 2 * cstep; lc = 0; }
     else { src += cstep; ++lc; }
   };
-  f32x4 acc[3][4][4];
+  f32x16 acc[3][2][2];
 #pragma unroll
   for (int c = 0; c < 3; ++c)
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) acc[c][a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int part = (((lane >> 4) ^ ((r16 >> 1) & 3))) * 8;
-  const int ra = (wm * 64 + r16) * 32 + part, rb = (wn * 64 + r16) * 32 + part;
-  // fragments [set][plane: Ah, Al, Bh, Bl][tile]
-  bf16x8 fr[2][4][4];
-  auto read_frag = [&](int buf, int f, int i) {       // i = 4 x tile + plane
-    const int pl = i & 3, q = i >> 2;
-    fr[f][pl][q] = ld8(&lds[buf][pl][(pl < 2 ? ra : rb) + q * 512]);
+    for (int i = 0; i < 16; ++i) acc[c][0][0][i] = acc[c][0][1][i] = acc[c][1][0][i] = acc[c][1][1][i] = 0.f;
+  // fragments [set][plane: Ah, Al, Bh, Bl][tile][half of the K step]
+  const int ra = (wm * 64 + r32) * 32, rb = (wn * 64 + r32) * 32;
+  const int part[2] = {((lane >> 5) ^ ((r32 >> 1) & 3)) * 8, ((2 + (lane >> 5)) ^ ((r32 >> 1) & 3)) * 8};
+  bf16x8 fr[2][4][2][2];
+  auto read_frag = [&](int buf, int f, int i) {       // i = 8 x half + 4 x tile + plane
+    const int pl = i & 3, q = (i >> 2) & 1, kk = i >> 3;
+    fr[f][pl][q][kk] = ld8(&lds[buf][pl][(pl < 2 ? ra : rb) + q * 1024 + part[kk]]);
   };
 #pragma unroll
   for (int s = 0; s < RING; ++s) {
@@ -351,9 +351,9 @@ k_dcsky_ring(const unsigned short* Ah, const unsigned short* Al, const unsigned 
           for (int i = 0; i < 3; ++i)
             if (3 * g + i < 16) read_frag((buf + 1) % RING, f ^ 1, 3 * g + i);
 #pragma unroll
-        for (int i = 6 * g; i < 6 * g + 6; ++i) {
-          const int p = i / 16, a = (i / 4) & 3, b = i & 3;    // hi hi, lo hi, hi lo
-          acc[c][a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fr[f][p == 1 ? 3 : 2][b], fr[f][p == 2 ? 1 : 0][a],
+        for (int i = 3 * g; i < 3 * g + 3; ++i) {
+          const int kk = i / 12, p = i / 4 % 3, a = (i >> 1) & 1, b = i & 1;    // products: hi hi, lo hi, hi lo
+          acc[c][a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[f][p == 1 ? 3 : 2][b][kk], fr[f][p == 2 ? 1 : 0][a][kk],
                                                                  acc[c][a][b], 0, 0, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -372,29 +372,32 @@ k_dcsky_ring(const unsigned short* Ah, const unsigned short* Al, const unsigned 
   if ((nk & 3) > 2) kstep(std::integral_constant<int, 2>());
   // the loads still under way write LDS: the block must not end before them
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  // D layout: lane holds D[n = 4 * (lane >> 4) + i][m = lane & 15]
+  // D layout: lane holds D[n = 8 * (i / 4) + 4 * (lane >> 5) + i % 4][m = lane & 31]
   const bool vec = (N & 3) == 0;
 #pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    const int m = mb + wm * 64 + 16 * a + r16;
+  for (int a = 0; a < 2; ++a) {
+    const int m = mb + wm * 64 + 32 * a + r32;
     if (m >= M) continue;
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      const int nq = nb + wn * 64 + 16 * b + (lane >> 4) * 4;
+    for (int bg = 0; bg < 8; ++bg) {
+      const int b = bg >> 2, i0 = (bg & 3) * 4;
+      const int nq = nb + wn * 64 + 32 * b + 2 * i0 + 4 * (lane >> 5);
       if (nq >= N) continue;
       float* dst = C + ((size_t)m * N + nq) * 3;
-      const f32x4 r = acc[0][a][b], g = acc[1][a][b], u = acc[2][a][b];
+      const f32x16 r = acc[0][a][b], g = acc[1][a][b], u = acc[2][a][b];
       if (vec) {
         float4* d4 = (float4*)dst;
-        d4[0] = make_float4(r[0], g[0], u[0], r[1]);
-        d4[1] = make_float4(g[1], u[1], r[2], g[2]);
-        d4[2] = make_float4(u[2], r[3], g[3], u[3]);
+        d4[0] = make_float4(r[i0], g[i0], u[i0], r[i0 + 1]);
+        d4[1] = make_float4(g[i0 + 1], u[i0 + 1], r[i0 + 2], g[i0 + 2]);
+        d4[2] = make_float4(u[i0 + 2], r[i0 + 3], g[i0 + 3], u[i0 + 3]);
       } else {
-        for (int i = 0; i < 4 && nq + i < N; ++i) {
-          dst[3 * i + 0] = r[i];
-          dst[3 * i + 1] = g[i];
-          dst[3 * i + 2] = u[i];
-        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (nq + i < N) {
+            dst[3 * i + 0] = r[i0 + i];
+            dst[3 * i + 1] = g[i0 + i];
+            dst[3 * i + 2] = u[i0 + i];
+          }
       }
     }
   }
@@ -422,13 +425,22 @@ static int ring_parts(long long tiles, int nk) {
 
 // Short-K form (K <= 160, e.g. 146 Klems patches): the product is bound by
 // the output write, and the operands are small enough that a wavefront keeps
-// its 16 rows of A (hi and lo, all K, three channels) in registers for the
-// whole launch.  A block of 8 wavefronts owns a slab of 128 rows of A and
-// walks a range of sky columns in chunks of 32: each chunk's B planes (hi/lo,
-// three channels, all K) are staged into LDS once, double-buffered (the next
-// chunk's global loads are in flight during this chunk's MFMAs), and every
-// wavefront multiplies its rows by them and stores its 16 x 32 x 3 outputs
-// before the next chunk.  No K loop over global memory, one barrier per chunk.
+// 16 rows of A (hi and lo, all K, three channels: 120 registers at K = 160)
+// for the whole launch.  A block of 8 wavefronts owns a slab of 128 rows of A
+// and walks a range of sky columns in chunks of 32: each chunk's B planes
+// (hi/lo, three channels, all K) are loaded straight into LDS, double-
+// buffered (the next chunk's loads are under way during this chunk's MFMAs).  No K loop over global
+// memory, one barrier per chunk.
+//
+// Outputs go through LDS: a lane ends up with 12 consecutive floats of a row,
+// and storing those as they are writes 16 bytes every 48, three times as many
+// partial lines as the rows have.  Turned in LDS, a store instruction covers
+// runs of 192 bytes.  2500 x 146 x 8760: 88 us (104 with 48-byte runs and the
+// chunk staged through registers), 3.0 of the 6.9 TB/s that a plain fill
+// reaches; what is left is the wait for a chunk's loads, which complete in
+// order behind the stores of the chunk before, and LDS reads (61 KB per
+// wavefront and chunk).  Four wavefronts of 32 rows halve those and lose
+// more: one wavefront per SIMD, 106 us.
 // Every lane issues the same loads and stores in every chunk (pieces past
 // the chunk load a valid piece again; outputs outside C go to `sink`), so the
 // wait for the next chunk's loads never waits for this chunk's stores.
@@ -437,120 +449,122 @@ constexpr int SROWS = 16 * SW;         // rows of A per block (a slab)
 constexpr int SCOLS = 32;              // sky columns per staged chunk
 constexpr int SHORT_KS = 5;            // K steps of 32 the short form covers (Kp <= 160)
 constexpr int SINK_FLOATS = 64 * 12;   // one wavefront's worth of redirected outputs
+constexpr int SOUT = 52;               // padded output row in LDS (floats): 16 columns x 3 channels
 
 template <int KS, bool VEC>
-__global__ void __launch_bounds__(64 * SW) k_dcsky_short(const unsigned short* Ah, const unsigned short* Al,
-                                                         const unsigned short* Bh, const unsigned short* Bl, float* C,
-                                                         float* sink, int M, int N, int nslab, int nrange) {
-  constexpr int Kp = 32 * KS;
-  constexpr int ROW = Kp + 8;                  // padded LDS row (bf16)
-  constexpr int PL = SCOLS * ROW;              // one (channel, hi|lo) tile
-  constexpr int NT = 64 * SW;
-  constexpr int CPR = Kp / 8;                  // 16-byte pieces per row
-  constexpr int NPC = 6 * SCOLS * CPR;         // pieces per chunk
-  constexpr int NLD = (NPC + NT - 1) / NT;     // pieces per thread
-  __shared__ __attribute__((aligned(16))) unsigned short lds[2][6][PL];   // [buffer][2 c + lo]
+__global__ void __launch_bounds__(64 * SW)
+k_dcsky_short(const unsigned short* Ah, const unsigned short* Al, const unsigned short* Bh, const unsigned short* Bl,
+              float* C, float* sink, int M, int N, int Mt, int Nt, int nrange) {
+  static_assert(SROWS == LBM, "a slab is a tile of the split planes");
+  constexpr int NPC = 6 * KS * 2;              // 1 KB pieces (16 rows of one K step) per chunk
+  constexpr int NLD = (NPC + SW - 1) / SW;     // pieces per wavefront
+  __shared__ __attribute__((aligned(16))) unsigned short lds[2][6 * KS * SCOLS * 32];   // [buffer][2 c + lo][step][row][32]
+  __shared__ __attribute__((aligned(16))) float turn[SW][16 * SOUT];
   // block -> (slab, column range); blocks run on XCD b % 8, and the blocks
   // of one XCD take consecutive q: all slabs of one column range, which
   // share its B chunks in that XCD's L2
   const int per = (int)((gridDim.x + 7) / 8);
   const int q = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
-  if (q >= nslab * nrange) return;
-  const int slab = q % nslab, range = q / nslab;
+  if (q >= Mt * nrange) return;
+  const int slab = q % Mt, range = q / Mt;
   const int nchunk = (N + SCOLS - 1) / SCOLS;
   const int cb = (int)((long long)range * nchunk / nrange), ce = (int)((long long)(range + 1) * nchunk / nrange);
   if (cb >= ce) return;
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int r16 = lane & 15, kq = (lane >> 4) * 8;
-  const int m = slab * SROWS + wave * 16 + r16;
-  const int mc = min(m, M - 1);                // clamped for loads; rows >= M are not stored
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, part = ((lane >> 4) ^ ((r16 >> 1) & 3)) * 8;
   bf16x8 ah[3][KS], al[3][KS];
 #pragma unroll
   for (int c = 0; c < 3; ++c)
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
-      const size_t o = ((size_t)c * M + mc) * Kp + s * 32 + kq;
+      const size_t o = (((size_t)c * Mt + slab) * KS + s) * RPLANE + (wave * 16 + r16) * 32 + part;
       ah[c][s] = ld8(Ah + o);
       al[c][s] = ld8(Al + o);
     }
-  // staging piece j of this thread: plane pl = 2 c + lo, row, 16-byte part
-  int soff[NLD], spl[NLD], srow[NLD], spart[NLD];
+  // piece p: plane p / (2 KS) (2 c + lo), K step, half of the chunk's rows
+  const unsigned short* psrc[NLD];
 #pragma unroll
   for (int j = 0; j < NLD; ++j) {
-    const int p = min(t + j * NT, NPC - 1);
-    const int rem = p % (SCOLS * CPR);
-    spl[j] = p / (SCOLS * CPR);
-    srow[j] = rem / CPR;
-    spart[j] = rem % CPR;
-    soff[j] = srow[j] * ROW + spart[j] * 8;
+    const int p = min(wave + j * SW, NPC - 1);
+    const int pl = p / (2 * KS), s = (p % (2 * KS)) >> 1, half = p & 1;
+    psrc[j] = ((pl & 1) ? Bl : Bh) + ((size_t)(pl >> 1) * Nt * KS + s) * RPLANE + half * 512;
   }
-  auto gload = [&](int chunk, u16x8* reg) {
+  auto load_chunk = [&](int chunk, int buf) {
     const int n0 = chunk * SCOLS;
+    const size_t at = (size_t)(n0 >> 7) * KS * RPLANE + (n0 & 127) * 32 + lane * 8;
 #pragma unroll
-    for (int j = 0; j < NLD; ++j) {
-      const unsigned short* src = (spl[j] & 1) ? Bl : Bh;
-      reg[j] = *(const u16x8*)(src + ((size_t)(spl[j] >> 1) * N + min(n0 + srow[j], N - 1)) * Kp + spart[j] * 8);
-    }
+    for (int j = 0; j < NLD; ++j)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(psrc[j] + at),
+                                       (__attribute__((address_space(3))) void*)&lds[buf][min(wave + j * SW, NPC - 1) * 512],
+                                       16, 0, 0);
   };
-  auto lstore = [&](int buf, const u16x8* reg) {
-#pragma unroll
-    for (int j = 0; j < NLD; ++j) *(u16x8*)&lds[buf][spl[j]][soff[j]] = reg[j];
-  };
-  u16x8 reg[NLD];
-  gload(cb, reg);
-  lstore(0, reg);
+  load_chunk(cb, 0);
   // every load so far (A and the first chunk) complete here, so that no wait
   // inside the loop, where this chunk's stores are also outstanding, is
   // counted against them
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
+  ring_wait<0>();
   float* const mysink = sink + lane * 12;
+  float* const tw = turn[wave];
+  constexpr int NST = VEC ? 3 : 12;      // stores per 16 columns: 16 bytes each, or 4
   for (int ch = cb; ch < ce; ++ch) {
     const int buf = (ch - cb) & 1;
-    gload(min(ch + 1, ce - 1), reg);
+    load_chunk(min(ch + 1, ce - 1), buf ^ 1);
     __builtin_amdgcn_sched_barrier(0);     // the next chunk's loads go out before the MFMAs
-    f32x4 acc[3][2];
+    f32x4 acc[2][3];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) acc[c][0] = acc[c][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < 2; ++b)
 #pragma unroll
-    for (int s = 0; s < KS; ++s)
+      for (int c = 0; c < 3; ++c) acc[b][c] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        const int row = 16 * b + r16;
+    for (int s = 0; s < KS; ++s) {
+      // the six accumulators take turns, so that no MFMA waits for the one before it
+      bf16x8 fb[2][3][2];
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-          const bf16x8 bh = __builtin_bit_cast(bf16x8, *(const u16x8*)&lds[buf][2 * c][row * ROW + s * 32 + kq]);
-          const bf16x8 bl = __builtin_bit_cast(bf16x8, *(const u16x8*)&lds[buf][2 * c + 1][row * ROW + s * 32 + kq]);
-          acc[c][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh, ah[c][s], acc[c][b], 0, 0, 0);
-          acc[c][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bl, ah[c][s], acc[c][b], 0, 0, 0);
-          acc[c][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh, al[c][s], acc[c][b], 0, 0, 0);
-        }
-      }
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            fb[b][c][h] = ld8(&lds[buf][((2 * c + h) * KS + s) * (SCOLS * 32) + (16 * b + r16) * 32 + part]);
+#pragma unroll
+      for (int p = 0; p < 3; ++p)            // hi hi, lo hi, hi lo
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int c = 0; c < 3; ++c)
+            acc[b][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[b][c][p == 1], p == 2 ? al[c][s] : ah[c][s],
+                                                                acc[b][c], 0, 0, 0);
+    }
     // D layout: lane holds D[n = 4 * (lane >> 4) + i][m = lane & 15], 12
-    // consecutive floats of row m
+    // consecutive floats of row m; turned through this wavefront's own LDS
+    const int m0 = slab * SROWS + wave * 16;
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
-      const int nq = ch * SCOLS + 16 * b + (lane >> 4) * 4;
-      const f32x4 r = acc[0][b], g = acc[1][b], u = acc[2][b];
-      if (VEC) {   // N a multiple of 4: nq < N implies nq + 3 < N, 16-byte aligned
-        float* dst = (m < M && nq < N) ? C + ((size_t)m * N + nq) * 3 : mysink;
-        float4* d4 = (float4*)dst;
-        d4[0] = make_float4(r[0], g[0], u[0], r[1]);
-        d4[1] = make_float4(g[1], u[1], r[2], g[2]);
-        d4[2] = make_float4(u[2], r[3], g[3], u[3]);
-      } else {
+      const f32x4 r = acc[b][0], g = acc[b][1], u = acc[b][2];
+      float4* t4 = (float4*)(tw + r16 * SOUT + (lane >> 4) * 12);
+      t4[0] = make_float4(r[0], g[0], u[0], r[1]);
+      t4[1] = make_float4(g[1], u[1], r[2], g[2]);
+      t4[2] = make_float4(u[2], r[3], g[3], u[3]);
+      __builtin_amdgcn_wave_barrier();
+      const int f0 = (ch * SCOLS + 16 * b) * 3;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float* dst = (m < M && nq + i < N) ? C + ((size_t)m * N + nq + i) * 3 : mysink + 3 * i;
-          dst[0] = r[i];
-          dst[1] = g[i];
-          dst[2] = u[i];
-        }
+      for (int i = 0; i < NST; ++i) {
+        const int l = i * 64 + lane;
+        constexpr int W = VEC ? 4 : 1;         // floats per store
+        const int row = l / (48 / W), f = l % (48 / W) * W;
+        // N a multiple of 4 (VEC): 16-byte aligned, and a piece is inside C or outside as a whole
+        const bool in = m0 + row < M && f0 + f < 3 * N;
+        float* dst = in ? C + (size_t)(m0 + row) * N * 3 + f0 + f : mysink;
+        if (VEC) *(float4*)dst = *(const float4*)(tw + row * SOUT + f);
+        else *dst = tw[row * SOUT + f];
       }
+      __builtin_amdgcn_wave_barrier();
     }
-    lstore(buf ^ 1, reg);    // the last chunk stages a copy of itself into the idle buffer
-    __syncthreads();
+    // the next chunk's loads (issued before these stores) done, every LDS
+    // read of this one too
+    ring_wait<2 * NST>();
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
 // FP32 reference path: 16x16 threads, 64x64 tile, LDS staged.
@@ -641,18 +655,18 @@ static int short_ranges(int nslab, int nchunk) {
 
 template <int KS>
 static void launch_short(const unsigned short* Ah, const unsigned short* Al, const unsigned short* Bh,
-                         const unsigned short* Bl, float* C, float* sink, int M, int N, hipStream_t st) {
-  const int nslab = (M + SROWS - 1) / SROWS, nchunk = (N + SCOLS - 1) / SCOLS;
-  const int nrange = short_ranges(nslab, nchunk);
-  const long long G = (long long)nslab * nrange;
+                         const unsigned short* Bl, float* C, float* sink, int M, int N, int Mt, int Nt,
+                         hipStream_t st) {
+  const int nrange = short_ranges(Mt, (N + SCOLS - 1) / SCOLS);
+  const long long G = (long long)Mt * nrange;
   if (G > 0x7fffffffLL - 8) throw std::runtime_error("dcsky: matrix too large");
   const unsigned nblk = (unsigned)((G + 7) / 8 * 8);
   if (N % 4 == 0)
     hipLaunchKernelGGL((k_dcsky_short<KS, true>), dim3(nblk), dim3(64 * SW), 0, st, Ah, Al, Bh, Bl, C, sink, M, N,
-                       nslab, nrange);
+                       Mt, Nt, nrange);
   else
     hipLaunchKernelGGL((k_dcsky_short<KS, false>), dim3(nblk), dim3(64 * SW), 0, st, Ah, Al, Bh, Bl, C, sink, M, N,
-                       nslab, nrange);
+                       Mt, Nt, nrange);
 }
 
 void dcsky(const float* A, const float* B, float* C, int M, int K, int N, int mode, hipStream_t st) {
@@ -660,33 +674,44 @@ void dcsky(const float* A, const float* B, float* C, int M, int K, int N, int mo
     hipLaunchKernelGGL(k_dcsky_f32, dim3((N + 63) / 64, (M + 63) / 64), dim3(256), 0, st, A, B, C, M, K, N);
     return;
   }
-  // Short K (a few K steps) is bound by the output write: K <= 160 keeps A in
-  // registers (mode 4 forces that form), up to 256 the per-wavefront kernel;
-  // long K is MFMA work and needs the LDS-staged tiles.  mode 2 forces the
-  // per-wavefront kernel, mode 3 the staged one.
+  // K <= 160 is bound by the output write and keeps A in registers (mode 4
+  // forces that form); longer K is MFMA work and takes the ring of LDS
+  // buffers (mode 3; 2500 x 146 x 8760: 155 us there).  mode 2 forces
+  // per-wavefront loads, slower everywhere (2500 x 200 x 8760: 299 us where
+  // the ring takes 179).
   const int k32 = (K + 31) / 32 * 32;
   if (mode == 4 && k32 > 32 * SHORT_KS) throw std::runtime_error("dcsky: mode 4 needs K <= 160");
   const bool shortk = mode == 4 || (mode == 1 && k32 <= 32 * SHORT_KS);
-  const bool staged = !shortk && (mode == 3 || (mode == 1 && K > 256));
-  const int Kp = k32;
-  const int Mt = (M + LBM - 1) / LBM, Nt = (N + LBN - 1) / LBN;      // the ring form's tiles
-  const size_t na = (size_t)3 * (staged ? Mt * LBM : M) * Kp, nb = (size_t)3 * (staged ? Nt * LBN : N) * Kp;
+  const bool staged = !shortk && mode != 2;
+  const bool tiled = shortk || staged;
+  const int Kp = k32, nk = Kp / 32;
+  const int Mt = (M + LBM - 1) / LBM, Nt = (N + LBN - 1) / LBN;      // tiles of the tiled planes
+  const size_t na = (size_t)3 * (tiled ? Mt * LBM : M) * Kp, nb = (size_t)3 * (tiled ? Nt * LBN : N) * Kp;
   std::lock_guard<std::mutex> lk(g_dc_mu);
   // split planes, then (16-byte aligned) the short form's output sink or a
   // split K's partial products
   const size_t plane_bytes = (2 * (na + nb) * sizeof(unsigned short) + 255) / 256 * 256;
-  const int parts = staged ? ring_parts((long long)Mt * Nt, Kp / 32) : 1;
+  const int parts = staged ? ring_parts((long long)Mt * Nt, nk) : 1;
   const size_t tail_bytes = std::max((size_t)SINK_FLOATS, parts > 1 ? (size_t)parts * M * N * 3 : 0) * sizeof(float);
   unsigned short* buf = dc_scratch(plane_bytes + tail_bytes, st);
   unsigned short *Ah = buf, *Al = buf + na, *Bh = buf + 2 * na, *Bl = buf + 2 * na + nb;
   float* sink = (float*)((char*)buf + plane_bytes);
-  if (staged) {
-    const int nk = Kp / 32;
+  if (tiled) {
     const size_t nba = ((size_t)Mt * 8 * nk + 3) / 4, nbb = ((size_t)Nt * 8 * nk + 3) / 4;
     const long long tiles = (long long)Mt * Nt;
     if (nba + nbb > 0x7fffffffu || tiles > 0x7fffffffLL - 8) throw std::runtime_error("dcsky: matrix too large");
     hipLaunchKernelGGL(k_split_tiled, dim3((unsigned)(nba + nbb)), dim3(256), 0, st, A, B, M, K, N, nk, Mt, Nt,
                        (unsigned)nba, Ah, Al, Bh, Bl);
+    if (shortk) {
+      switch (nk) {
+        case 1: launch_short<1>(Ah, Al, Bh, Bl, C, sink, M, N, Mt, Nt, st); break;
+        case 2: launch_short<2>(Ah, Al, Bh, Bl, C, sink, M, N, Mt, Nt, st); break;
+        case 3: launch_short<3>(Ah, Al, Bh, Bl, C, sink, M, N, Mt, Nt, st); break;
+        case 4: launch_short<4>(Ah, Al, Bh, Bl, C, sink, M, N, Mt, Nt, st); break;
+        default: launch_short<5>(Ah, Al, Bh, Bl, C, sink, M, N, Mt, Nt, st); break;
+      }
+      return;
+    }
     hipLaunchKernelGGL(k_dcsky_ring, dim3((unsigned)((tiles + 7) / 8 * 8), (unsigned)parts), dim3(256), 0, st, Ah, Al,
                        Bh, Bl, parts > 1 ? sink : C, M, N, nk, Mt, Nt);
     if (parts > 1) {
@@ -699,21 +724,11 @@ void dcsky(const float* A, const float* B, float* C, int M, int K, int N, int mo
   if (nba + nbb > 0x7fffffffu) throw std::runtime_error("dcsky: matrix too large");
   hipLaunchKernelGGL(k_split, dim3((unsigned)(nba + nbb)), dim3(256), 0, st, A, B, M, K, N, Kp, (unsigned)nba, Ah, Al,
                      Bh, Bl);
-  if (shortk) {
-    switch (Kp / 32) {
-      case 1: launch_short<1>(Ah, Al, Bh, Bl, C, sink, M, N, st); break;
-      case 2: launch_short<2>(Ah, Al, Bh, Bl, C, sink, M, N, st); break;
-      case 3: launch_short<3>(Ah, Al, Bh, Bl, C, sink, M, N, st); break;
-      case 4: launch_short<4>(Ah, Al, Bh, Bl, C, sink, M, N, st); break;
-      default: launch_short<5>(Ah, Al, Bh, Bl, C, sink, M, N, st); break;
-    }
-  } else {
-    const int Wt = (M + BM - 1) / BM, Vt = (N + BN - 1) / BN;
-    const long long tiles = (long long)Wt * Vt;
-    if (tiles > 0x7fffffffLL - 8) throw std::runtime_error("dcsky: matrix too large");
-    const unsigned nblk = (unsigned)((tiles + 7) / 8 * 8);
-    hipLaunchKernelGGL(k_dcsky_mfma, dim3(nblk), dim3(DB), 0, st, Ah, Al, Bh, Bl, C, M, N, Kp, Wt, Vt);
-  }
+  const int Wt = (M + BM - 1) / BM, Vt = (N + BN - 1) / BN;
+  const long long tiles = (long long)Wt * Vt;
+  if (tiles > 0x7fffffffLL - 8) throw std::runtime_error("dcsky: matrix too large");
+  hipLaunchKernelGGL(k_dcsky_mfma, dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(DB), 0, st, Ah, Al, Bh, Bl, C, M, N, Kp,
+                     Wt, Vt);
 }
 
 }  // namespace rg

@@ -634,3 +634,25 @@ def test_long_k_product_at_tile_and_split_edges(L, m, k, n):
         ref = a[:, :, ch].double().contiguous() @ b[:, :, ch].double().contiguous()
         rel = ((c[:, :, ch].double() - ref) / ref).abs().max().item()
         assert rel <= 3 * 2.0 ** -16 + k * 2.0 ** -24, (ch, rel)
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 1, 1), (15, 32, 33), (16, 33, 31), (127, 64, 2048), (129, 65, 130), (128, 146, 128),
+                                   (257, 160, 1001), (2500, 146, 97), (40, 161, 36)])
+def test_short_k_product_at_chunk_and_slab_edges(L, m, k, n):
+    """The short-K form: rows that do and do not fill a wavefront's 16 or a
+    slab's 128, sky columns around the 32-column chunks and not a multiple of
+    four, every number of K steps, and the first K that leaves the form.  The
+    bound is the long-K test's."""
+    import torch
+    _say(f"short-K product {m} x {k} x {n}")
+    g = torch.Generator(device="cuda").manual_seed(m + k + n)
+    a = torch.rand((m, k, 3), generator=g, device="cuda")
+    b = torch.exp(torch.randn((k, n, 3), generator=g, device="cuda"))
+    c = torch.full((m + 1, n, 3), -1.0, device="cuda")
+    torch.cuda.synchronize()
+    L.dcsky_device(a.data_ptr(), b.data_ptr(), c.data_ptr(), m, k, n)
+    assert (c[m] == -1.0).all()                    # nothing past the last row
+    for ch in range(3):
+        ref = a[:, :, ch].double().contiguous() @ b[:, :, ch].double().contiguous()
+        rel = ((c[:m, :, ch].double() - ref) / ref).abs().max().item()
+        assert rel <= 3 * 2.0 ** -16 + k * 2.0 ** -24, (ch, rel)
