@@ -567,6 +567,62 @@ k_dcsky_short(const unsigned short* Ah, const unsigned short* Al, const unsigned
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
+// Small products in one launch, FP32 throughout: a block of 16 wavefronts
+// takes 64 columns of RM rows (all three channels), each wavefront a
+// sixteenth of K, and adds the parts in LDS in order.  Splitting the operands
+// first takes a launch of its own, 7 us of latency whatever the size: 67 x 41
+// x 5 takes 14 us here and 25 there, 100 x 578 x 100 22 and 36.  From 2^22
+// multiply-adds on four rows share a column's loads (11 x 146 x 8760: 26 us,
+// 44 split), which needs columns enough that a wavefront's lie in one group
+// of rows (14000 x 578 x 1: 174 us with four rows, 50 with one).  The lines
+// to the split forms lie where they catch up; past K = 1024 the parts' chains
+// of loads are longer than the ring's split K (2000 x 2306 x 1: 125 against
+// 53 us).
+constexpr int TW = 16;
+constexpr long long SMALL_MACS = 1ll << 23, SMALL_ROW_MACS = 1ll << 22, SMALL_WIDE_MACS = 1ll << 24;
+constexpr int SMALL_K = 1024, SMALL_WIDE_N = 256;
+template <int RM>
+__global__ void __launch_bounds__(64 * TW) k_dcsky_small(const float* A, const float* B, float* C, int M, int K, int N) {
+  __shared__ float part[TW][RM][64 * 3 + 1];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  // column `col` of the row groups laid end to end
+  const size_t all = (size_t)((M + RM - 1) / RM) * N, col0 = (size_t)blockIdx.x * 64;
+  const size_t col = min(col0 + lane, all - 1);
+  const int m = (int)(col / N) * RM;
+  const float* b = B + (col % N) * 3;
+  const float* a[RM];
+#pragma unroll
+  for (int i = 0; i < RM; ++i) a[i] = A + (size_t)min(m + i, M - 1) * K * 3;
+  const int k0 = (int)((long long)K * w / TW), k1 = (int)((long long)K * (w + 1) / TW);
+  float acc[RM][3] = {};
+#pragma unroll 8
+  for (int k = k0; k < k1; ++k) {
+    const float* bk = b + (size_t)k * N * 3;
+    const float b0 = bk[0], b1 = bk[1], b2 = bk[2];
+#pragma unroll
+    for (int i = 0; i < RM; ++i) {
+      acc[i][0] = fmaf(a[i][3 * k], b0, acc[i][0]);
+      acc[i][1] = fmaf(a[i][3 * k + 1], b1, acc[i][1]);
+      acc[i][2] = fmaf(a[i][3 * k + 2], b2, acc[i][2]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < RM; ++i)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) part[w][i][3 * lane + c] = acc[i][c];
+  __syncthreads();
+  for (int t = threadIdx.x; t < RM * 192; t += 64 * TW) {
+    const int i = t / 192, f = t % 192;
+    const size_t oc = col0 + f / 3;
+    const int om = (int)(oc / N) * RM + i;
+    if (oc >= all || om >= M) continue;
+    float v = part[0][i][f];
+#pragma unroll
+    for (int k = 1; k < TW; ++k) v += part[k][i][f];
+    C[((size_t)om * N + oc % N) * 3 + f % 3] = v;
+  }
+}
+
 // FP32 reference path: 16x16 threads, 64x64 tile, LDS staged.
 __global__ void __launch_bounds__(256) k_dcsky_f32(const float* A, const float* B, float* C, int M, int K, int N) {
   __shared__ float As[3][64][17];
@@ -672,6 +728,15 @@ static void launch_short(const unsigned short* Ah, const unsigned short* Al, con
 void dcsky(const float* A, const float* B, float* C, int M, int K, int N, int mode, hipStream_t st) {
   if (mode == 0) {
     hipLaunchKernelGGL(k_dcsky_f32, dim3((N + 63) / 64, (M + 63) / 64), dim3(256), 0, st, A, B, C, M, K, N);
+    return;
+  }
+  const bool wide = N >= SMALL_WIDE_N && M >= 4;
+  const double macs = (double)M * N * K;
+  if (mode == 1 && K <= SMALL_K && macs <= (double)(wide ? SMALL_WIDE_MACS : SMALL_MACS)) {
+    const bool rows = wide && macs > (double)SMALL_ROW_MACS;
+    const size_t cols = (size_t)(rows ? (M + 3) / 4 : M) * N;
+    hipLaunchKernelGGL(rows ? k_dcsky_small<4> : k_dcsky_small<1>, dim3((unsigned)((cols + 63) / 64)), dim3(64 * TW), 0,
+                       st, A, B, C, M, K, N);
     return;
   }
   // K <= 160 is bound by the output write and keeps A in registers (mode 4

@@ -656,3 +656,27 @@ def test_short_k_product_at_chunk_and_slab_edges(L, m, k, n):
         ref = a[:, :, ch].double().contiguous() @ b[:, :, ch].double().contiguous()
         rel = ((c[:m, :, ch].double() - ref) / ref).abs().max().item()
         assert rel <= 3 * 2.0 ** -16 + k * 2.0 ** -24, (ch, rel)
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 1, 1), (67, 41, 5), (3, 15, 300), (4, 16, 255), (4, 1024, 1024), (5, 1025, 30),
+                                   (9, 146, 8760), (101, 289, 257), (14000, 578, 1), (63, 513, 256)])
+def test_small_product_against_fp64(L, m, k, n):
+    """The one-launch form: fewer K than wavefronts, row groups cut short,
+    columns that end inside a block, either side of its lines (K 1024, 256
+    columns, 2^22 and 2^24 multiply-adds).  FP32 sums of positive terms:
+    K 2^-24 relative; the split forms past the line add the long-K test's
+    bound."""
+    import torch
+    _say(f"small product {m} x {k} x {n}")
+    g = torch.Generator(device="cuda").manual_seed(m + k + n)
+    a = torch.rand((m, k, 3), generator=g, device="cuda")
+    b = torch.exp(torch.randn((k, n, 3), generator=g, device="cuda"))
+    c = torch.full((m + 1, n, 3), -1.0, device="cuda")
+    torch.cuda.synchronize()
+    L.dcsky_device(a.data_ptr(), b.data_ptr(), c.data_ptr(), m, k, n)
+    assert (c[m] == -1.0).all()
+    split = k > 1024
+    for ch in range(3):
+        ref = a[:, :, ch].double().contiguous() @ b[:, :, ch].double().contiguous()
+        rel = ((c[:m, :, ch].double() - ref) / ref).abs().max().item()
+        assert rel <= (3 * 2.0 ** -16 if split else 0) + (k + 1) * 2.0 ** -24, (ch, rel)
