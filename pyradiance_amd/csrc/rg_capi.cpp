@@ -1060,6 +1060,7 @@ int rg_sky_create(rg_sky** out, const char* weather, const rg_skyopts* o) {
       delete s;
       throw;
     }
+    rg::sky_plan_opened();
     *out = s;
     return 0;
   } catch (const std::exception& e) {
@@ -1068,7 +1069,11 @@ int rg_sky_create(rg_sky** out, const char* weather, const rg_skyopts* o) {
   }
 }
 
-void rg_sky_destroy(rg_sky* s) { delete s; }
+void rg_sky_destroy(rg_sky* s) {
+  if (!s) return;
+  delete s;
+  rg::sky_plan_closed();
+}
 
 const char* rg_sky_error(const rg_sky* s) { return s ? s->err.c_str() : g_create_err.c_str(); }
 

@@ -7,6 +7,7 @@
 // (AddDirect :828-872) and the averaged sky (-A).
 #include "rg_sky.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -443,21 +444,29 @@ struct SkyStepOut {
 // Per-patch terms of the sun-sky angle and of the horizontal-illuminance
 // weight, from the patch's (float) altitude and azimuth as rh_init() stores
 // them (gen/gendaymtx.c:1221-1264).
-struct SkyPatchTab {
-  double czp, szp;     // cos, sin of the patch zenith angle
-  double sinp, domp;   // sin(altitude), solid angle
-  double azi;
-  double dir[3];       // rh_vector() direction
-};
+//
+// One array per term, `n` patches long, so that a wavefront's loads are whole
+// runs (as 80-byte records they touched a line per lane).
+enum : int { TAB_CZP, TAB_SZP,      // cos, sin of the patch zenith angle
+             TAB_SIN, TAB_DOM,      // sin(altitude), solid angle
+             TAB_CA, TAB_SA,        // cos, sin of the azimuth
+             TAB_X, TAB_Y, TAB_Z,   // rh_vector() direction
+             TAB_ROW,               // altitude row, 0 at the horizon (patches of a row share czp)
+             TAB_TERMS };
 
 // CalcRelLuminance() with the sun-sky angle of CalcSkyPatchLumin()
-// (gen/gendaymtx.c:1292-1322, :1172-1191); czs, szs: cos and sin of the sun
-// zenith angle.  The arithmetic is the reference's, term for term, in double.
-__device__ __forceinline__ float patch_lum(const SkyStep& k, double czs, double szs, const SkyPatchTab& t) {
-  const double aas = fabs(t.azi - k.azimuth);
-  const double sspa = acos(czs * t.czp + szs * t.szp * cos(aas));
+// (gen/gendaymtx.c:1292-1322, :1172-1191), in double: grad the row's
+// gradation term 1 + a exp(b / cos zenith), czs, szs cos and sin of the sun
+// zenith angle, cas, sas of its azimuth.  Two transcendental functions per
+// patch: the cosine of the azimuth difference comes from the tables, the
+// cosine of the sun-sky angle is what its arc cosine was taken of, and the
+// gradation is the row's (with all six per patch the kernel took 286 us at
+// MF 4 over a year, all of it FP64 arithmetic; 191 us so).
+__device__ __forceinline__ float patch_lum(const SkyStep& k, double grad, double czs, double szs, double cas, double sas,
+                                           const double* t) {
+  const double cg = fmin(fmax(czs * t[TAB_CZP] + szs * t[TAB_SZP] * (cas * t[TAB_CA] + sas * t[TAB_SA]), -1.0), 1.0);
   const double* pp = k.perez;
-  double l = (1.0 + pp[0] * exp(pp[1] / t.czp)) * (1.0 + pp[2] * exp(pp[3] * sspa) + pp[4] * cos(sspa) * cos(sspa));
+  double l = grad * (1.0 + pp[2] * exp(pp[3] * acos(cg)) + pp[4] * cg * cg);
   float f = (float)l;
   return f < 0 ? 0.f : f;
 }
@@ -493,18 +502,46 @@ __device__ __forceinline__ bool sun_before(double xd, int xp, double yd, int yp)
 }
 
 __global__ void k_sky_patch(const float* __restrict__ palt, const float* __restrict__ pazi,
-                            const float* __restrict__ dom, int np, SkyPatchTab* __restrict__ tab) {
+                            const float* __restrict__ dom, int np, int mf, double* __restrict__ tab) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= np) return;
   const double zsa = kPI * 0.5 - (double)palt[p];
-  SkyPatchTab t;
-  t.czp = cos(zsa);
-  t.szp = sin(zsa);
-  t.sinp = sin((double)palt[p]);
-  t.domp = (double)dom[p];
-  t.azi = (double)pazi[p];
-  patch_dir(t.dir, palt[p], pazi[p]);
-  tab[p] = t;
+  tab[TAB_CZP * np + p] = cos(zsa);
+  tab[TAB_SZP * np + p] = sin(zsa);
+  tab[TAB_SIN * np + p] = sin((double)palt[p]);
+  tab[TAB_DOM * np + p] = (double)dom[p];
+  tab[TAB_CA * np + p] = cos((double)pazi[p]);
+  tab[TAB_SA * np + p] = sin((double)pazi[p]);
+  // rows of the Reinhart division: mf rows of tnaz[k] mf patches for k = 0..6
+  // from patch 1 on, then the zenith
+  {
+    const int tnaz[7] = {30, 30, 24, 24, 18, 12, 6};
+    int q = p > 0 ? p - 1 : 0, r = 0;
+    for (int k = 0; k < 7; ++k) {
+      const int per = tnaz[k] * mf, in = q / per < mf ? q / per : mf;
+      r += in;
+      q -= in * per;
+      if (in < mf) break;
+    }
+    tab[TAB_ROW * np + p] = (double)r;
+  }
+  double dir[3];
+  patch_dir(dir, palt[p], pazi[p]);
+  for (int a = 0; a < 3; ++a) tab[(TAB_X + a) * np + p] = dir[a];
+}
+
+// First patch of altitude row r (the zenith for r = 7 mf).
+__device__ __forceinline__ int rowp(int r, int mf, int np) {
+  const int tnaz[7] = {30, 30, 24, 24, 18, 12, 6};
+  if (r >= 7 * mf) return np - 1;
+  int p = 1;
+  for (int k = 0; k < 7; ++k) {
+    const int in = r < mf ? r : mf;
+    p += in * tnaz[k] * mf;
+    r -= in;
+    if (r <= 0 && in < mf) break;
+  }
+  return p;
 }
 
 // One block per stored step: every patch's relative luminance (written
@@ -515,13 +552,14 @@ __global__ void k_sky_patch(const float* __restrict__ palt, const float* __restr
 // reference's one sequential pass (largest dot products, ties to the lower
 // patch).
 __global__ void __launch_bounds__(SKY_BLOCK) k_sky_step(const SkyStep* __restrict__ steps, int nsteps,
-                                                        const SkyPatchTab* __restrict__ tab, int np, int nsuns,
+                                                        const double* __restrict__ tab, int np, int mf, int nsuns,
                                                         double fixed_sa, float* __restrict__ lum,
                                                         SkyStepOut* __restrict__ out) {
   const int s = blockIdx.x;
   if (s >= nsteps) return;
   const SkyStep k = steps[s];
   const int tid = threadIdx.x;
+  const int nrow = 7 * mf + 1;
   __shared__ double red[SKY_BLOCK];
   __shared__ double cd[SKY_BLOCK * MAXSUN];
   __shared__ int cp[SKY_BLOCK * MAXSUN];
@@ -529,21 +567,44 @@ __global__ void __launch_bounds__(SKY_BLOCK) k_sky_step(const SkyStep* __restric
   double nd[MAXSUN];
   int npch[MAXSUN];
   for (int i = 0; i < MAXSUN; ++i) { nd[i] = -1.0; npch[i] = -1; }
-  const double czs = cos(k.sun_zenith), szs = sin(k.sun_zenith);
+  // the sun's sines and cosines, one lane each
+  __shared__ double trig[6];
+  if (tid < 6) {
+    const double a = tid < 2 ? k.sun_zenith : (tid < 4 ? k.azimuth : k.altitude);
+    trig[tid] = (tid & 1) ? sin(a) : cos(a);
+  }
+  __syncthreads();
+  const double czs = trig[0], szs = trig[1], cas = trig[2], sas = trig[3];
+  extern __shared__ double grad[];            // gradation term of every row
+  if (k.kind == 2) {
+    for (int r = tid; r < nrow; r += SKY_BLOCK) grad[r] = 1.0 + k.perez[0] * exp(k.perez[1] / tab[TAB_CZP * np + rowp(r, mf, np)]);
+    __syncthreads();
+  }
   double sv[3];
-  sv[1] = cos(k.altitude);
-  sv[0] = sv[1] * sin(k.azimuth);
-  sv[1] *= cos(k.azimuth);
-  sv[2] = sin(k.altitude);
+  sv[1] = trig[4];
+  sv[0] = sv[1] * sas;
+  sv[1] *= cas;
+  sv[2] = trig[5];
   float* lrow = lum + (size_t)s * np;
-  for (int p = 1 + tid; p < np; p += SKY_BLOCK) {
-    const SkyPatchTab& t = tab[p];
-    if (k.kind == 2) {
-      const float f = patch_lum(k, czs, szs, t);
-      lrow[p] = f;
-      acc += (double)f * t.sinp * t.domp;
+  if (k.kind == 2 || k.add_sun) {
+    // a patch's table entries are requested while the one before is evaluated
+    double t[TAB_TERMS], nx[TAB_TERMS];
+    auto fetch = [&](int p) {
+#pragma unroll
+      for (int q = 0; q < TAB_TERMS; ++q) nx[q] = tab[q * np + min(p, np - 1)];
+    };
+    fetch(1 + tid);
+    for (int p = 1 + tid; p < np; p += SKY_BLOCK) {
+#pragma unroll
+      for (int q = 0; q < TAB_TERMS; ++q) t[q] = nx[q];
+      fetch(p + SKY_BLOCK);
+      if (k.kind == 2) {
+        const float f = patch_lum(k, grad[(int)t[TAB_ROW]], czs, szs, cas, sas, t);
+        lrow[p] = f;
+        acc += (double)f * t[TAB_SIN] * t[TAB_DOM];
+      }
+      if (k.add_sun) top_insert(nd, npch, nsuns, t[TAB_X] * sv[0] + t[TAB_Y] * sv[1] + t[TAB_Z] * sv[2], p);
     }
-    if (k.add_sun) top_insert(nd, npch, nsuns, t.dir[0] * sv[0] + t.dir[1] * sv[1] + t.dir[2] * sv[2], p);
   }
   red[tid] = acc;
   for (int i = 0; i < MAXSUN; ++i) { cd[tid * MAXSUN + i] = nd[i]; cp[tid * MAXSUN + i] = npch[i]; }
@@ -602,7 +663,7 @@ __global__ void __launch_bounds__(SKY_BLOCK) k_sky_step(const SkyStep* __restric
       for (int i = 0; i < MAXSUN; ++i) {
         if (i >= nsuns || cp[i] < 0) continue;
         float va = (float)(wta[i] * k.dir_illum / (WHTEFFICACY * wtot));
-        va = (float)((double)va / (fixed_sa > 0 ? fixed_sa : (double)tab[cp[i]].domp));
+        va = (float)((double)va / (fixed_sa > 0 ? fixed_sa : tab[TAB_DOM * np + cp[i]]));
         o.sunp[i] = cp[i];
         o.sunv[i] = va;
         o.nsun = i + 1;
@@ -612,9 +673,36 @@ __global__ void __launch_bounds__(SKY_BLOCK) k_sky_step(const SkyStep* __restric
   }
 }
 
+// One entry of the matrix: sky, then the sun's share.
+struct SkyPix { float r, g, b; };
+// `kind`: the step's, already loaded; the rest of it is read for the ground only.
+__device__ __forceinline__ SkyPix sky_value(const SkyStep& st, int kind, const SkyStepOut& o, int p, float l, float3 skyc,
+                                            float3 sunc) {
+  SkyPix v = {0.f, 0.f, 0.f};
+  if (p == 0) return SkyPix{st.ground[0], st.ground[1], st.ground[2]};
+  if (kind == 2) {
+    const float sc = (float)((double)(o.uniform ? 1.f : l) * o.scale);
+    v.r = sc * skyc.x;
+    v.g = sc * skyc.y;
+    v.b = sc * skyc.z;
+  }
+  if (kind > 0)
+    for (int i = 0; i < o.nsun; ++i)
+      if (o.sunp[i] == p) {
+        v.r += o.sunv[i] * sunc.x;
+        v.g += o.sunv[i] * sunc.y;
+        v.b += o.sunv[i] * sunc.z;
+      }
+  return v;
+}
+
 // The matrix, [patch][step][rgb], from the step-major luminances: a tile of
 // FILL_TS steps x FILL_TP patches is read along patches into LDS and written
-// along steps, so both sides move whole contiguous runs.
+// along steps, so both sides move whole contiguous runs.  Bound by the
+// scattered rows of its stores: 78 to 96 us for the 242 MB of MF 4 over a year,
+// where a fill of that size takes 35; tiles of 64 or 128 or 256 steps by 4 to
+// 32 patches, rows turned in LDS for 16-byte stores and tiles kept to one
+// XCD's L2 took 102 to 173 us.
 constexpr int FILL_TS = 64, FILL_TP = 16;
 
 __global__ void __launch_bounds__(SKY_BLOCK) k_sky_fill(const SkyStep* __restrict__ steps, const SkyStepOut* __restrict__ so,
@@ -639,39 +727,51 @@ __global__ void __launch_bounds__(SKY_BLOCK) k_sky_fill(const SkyStep* __restric
   for (int pl = tid / FILL_TS; pl < FILL_TP; pl += SKY_BLOCK / FILL_TS) {
     const int p = p0 + pl;
     if (p >= np) break;
-    float v[3] = {0.f, 0.f, 0.f};
-    if (p == 0) {
-      for (int c = 0; c < 3; ++c) v[c] = steps[s].ground[c];
-    } else if (kind == 2) {
-      const float l = o.uniform ? 1.f : lt[pl][sl];
-      const float sc = (float)((double)l * o.scale);
-      v[0] = sc * skyc.x;
-      v[1] = sc * skyc.y;
-      v[2] = sc * skyc.z;
-    }
-    if (p > 0 && kind > 0)
-      for (int i = 0; i < o.nsun; ++i)
-        if (o.sunp[i] == p) {
-          v[0] += o.sunv[i] * sunc.x;
-          v[1] += o.sunv[i] * sunc.y;
-          v[2] += o.sunv[i] * sunc.z;
-        }
+    const SkyPix v = sky_value(steps[s], kind, o, p, lt[pl][sl], skyc, sunc);
     float* d = out + ((size_t)p * nsteps + s) * 3;
-    d[0] = v[0];
-    d[1] = v[1];
-    d[2] = v[2];
+    d[0] = v.r;
+    d[1] = v.g;
+    d[2] = v.b;
   }
 }
 
-// -A: the rows summed in step order in FP32, then scaled by 1/ntsteps.
-__global__ void k_sky_average(const float* __restrict__ full, int np, int nsteps, double inv, int scale,
-                              float* __restrict__ out) {
+// -A: partial sums of every patch over MEAN_TS steps, in double (the matrix
+// itself is not formed; with one thread per row adding up its steps in order
+// the sums took 263 us of a 421 us call at MF 1 over 91 days).
+constexpr int MEAN_TS = 64;
+__global__ void __launch_bounds__(SKY_BLOCK) k_sky_partial(const SkyStep* __restrict__ steps, const SkyStepOut* __restrict__ so,
+                                                           const float* __restrict__ lum, int nsteps, int np, float3 skyc,
+                                                           float3 sunc, double* __restrict__ part) {
+  __shared__ double red[SKY_BLOCK / 64][64][3];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int p = blockIdx.x * 64 + lane, s0 = blockIdx.y * MEAN_TS;
+  double a[3] = {0.0, 0.0, 0.0};
+  if (p < np)
+    for (int s = s0 + w; s < min(s0 + MEAN_TS, nsteps); s += SKY_BLOCK / 64) {
+      const float l = lum[(size_t)s * np + p];      // no sky there: not used
+      const SkyPix v = sky_value(steps[s], steps[s].kind, so[s], p, l, skyc, sunc);
+      a[0] += v.r;
+      a[1] += v.g;
+      a[2] += v.b;
+    }
+  for (int c = 0; c < 3; ++c) red[w][lane][c] = a[c];
+  __syncthreads();
+  if (w == 0 && p < np)
+    for (int c = 0; c < 3; ++c) {
+      double v = red[0][lane][c];
+      for (int k = 1; k < SKY_BLOCK / 64; ++k) v += red[k][lane][c];
+      part[((size_t)blockIdx.y * np + p) * 3 + c] = v;
+    }
+}
+
+// The partial sums added up in order and scaled by 1/ntsteps.
+__global__ void k_sky_mean(const double* __restrict__ part, int nval, int nparts, double inv, int scale,
+                           float* __restrict__ out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= np * 3) return;
-  const int p = i / 3, c = i % 3;
-  float acc = full[(size_t)p * nsteps * 3 + c];
-  for (int s = 1; s < nsteps; ++s) acc += full[((size_t)p * nsteps + s) * 3 + c];
-  out[i] = scale ? (float)(acc * inv) : acc;
+  if (i >= nval) return;
+  double acc = 0.0;
+  for (int k = 0; k < nparts; ++k) acc += part[(size_t)k * nval + i];
+  out[i] = (float)(scale ? acc * inv : acc);
 }
 
 void ck(hipError_t e, const char* what) {
@@ -681,12 +781,15 @@ void ck(hipError_t e, const char* what) {
 }  // namespace
 
 // Device buffers of one sky_matrix() call, laid out in one block (256-byte
-// aligned parts): step records, step outputs, patch tables, patch altitude /
-// azimuth / solid angle, the luminance plane, and with -A the full matrix
-// before averaging.
+// aligned parts): the uploaded step records and patch altitude / azimuth /
+// solid angle, then step outputs, patch tables, the luminance plane, and with
+// -A the partial sums.
 struct SkyScratch {
-  size_t steps, so, tab, alt, azi, dom, lum, full, bytes;
+  size_t steps, so, tab, alt, azi, dom, lum, part, bytes;
+  size_t noalloc;      // what the allocation-free form counts: with -A a whole matrix as well
 };
+
+static int sky_parts(const SkyPlan& P) { return (P.nsteps + MEAN_TS - 1) / MEAN_TS; }
 
 static SkyScratch sky_scratch_layout(const SkyPlan& P) {
   const size_t np = (size_t)P.npatch, ns = (size_t)P.nsteps;
@@ -694,23 +797,24 @@ static SkyScratch sky_scratch_layout(const SkyPlan& P) {
   SkyScratch L;
   size_t o = 0;
   L.steps = o; o = up(o + sizeof(SkyStep) * ns);
-  L.so = o;    o = up(o + sizeof(SkyStepOut) * ns);
-  L.tab = o;   o = up(o + sizeof(SkyPatchTab) * np);
   L.alt = o;   o = up(o + sizeof(float) * np);
   L.azi = o;   o = up(o + sizeof(float) * np);
   L.dom = o;   o = up(o + sizeof(float) * np);
+  L.so = o;    o = up(o + sizeof(SkyStepOut) * ns);
+  L.tab = o;   o = up(o + sizeof(double) * TAB_TERMS * np);
   L.lum = o;   o = up(o + sizeof(float) * np * ns);
-  L.full = o;  if (P.opts.average) o = up(o + sizeof(float) * 3 * np * ns);
+  L.part = o;  if (P.opts.average) o = up(o + sizeof(double) * 3 * np * sky_parts(P));
   L.bytes = o;
+  L.noalloc = L.part + (P.opts.average ? sizeof(float) * 3 * np * ns : 0);
   return L;
 }
 
 // The kernels of one call, with their buffers at `base` (layout above).
 static void sky_matrix_run(const SkyPlan& P, float* out, hipStream_t st, char* base, const SkyScratch& L) {
-  const int np = P.npatch, ns = P.nsteps;
+  const int np = P.npatch, ns = P.nsteps, mf = P.opts.mfactor;
   SkyStep* dsteps = (SkyStep*)(base + L.steps);
   SkyStepOut* dso = (SkyStepOut*)(base + L.so);
-  SkyPatchTab* dtab = (SkyPatchTab*)(base + L.tab);
+  double* dtab = (double*)(base + L.tab);
   float* dalt = (float*)(base + L.alt);
   float* dazi = (float*)(base + L.azi);
   float* ddom = (float*)(base + L.dom);
@@ -719,38 +823,28 @@ static void sky_matrix_run(const SkyPlan& P, float* out, hipStream_t st, char* b
   ck(hipMemcpyAsync(dalt, P.palt.data(), sizeof(float) * np, hipMemcpyHostToDevice, st), "upload");
   ck(hipMemcpyAsync(dazi, P.pazi.data(), sizeof(float) * np, hipMemcpyHostToDevice, st), "upload");
   ck(hipMemcpyAsync(ddom, P.dom.data(), sizeof(float) * np, hipMemcpyHostToDevice, st), "upload");
-  k_sky_patch<<<(np + 255) / 256, 256, 0, st>>>(dalt, dazi, ddom, np, dtab);
+  k_sky_patch<<<(np + 255) / 256, 256, 0, st>>>(dalt, dazi, ddom, np, mf, dtab);
   ck(hipGetLastError(), "k_sky_patch");
   int nsuns = P.opts.nsuns < 1 ? 1 : (P.opts.nsuns > MAXSUN ? MAXSUN : P.opts.nsuns);
-  k_sky_step<<<ns, SKY_BLOCK, 0, st>>>(dsteps, ns, dtab, np, nsuns, P.opts.fixed_sun_sa, dlum, dso);
+  k_sky_step<<<ns, SKY_BLOCK, sizeof(double) * (7 * mf + 1), st>>>(dsteps, ns, dtab, np, mf, nsuns, P.opts.fixed_sun_sa,
+                                                                   dlum, dso);
   ck(hipGetLastError(), "k_sky_step");
-  float* full = P.opts.average ? (float*)(base + L.full) : out;
   const SkyOpts& o = P.opts;
   float3 skyc = make_float3((float)o.sky_color[0], (float)o.sky_color[1], (float)o.sky_color[2]);
   float3 sunc = make_float3((float)o.sun_color[0], (float)o.sun_color[1], (float)o.sun_color[2]);
-  dim3 grid((ns + FILL_TS - 1) / FILL_TS, (np + FILL_TP - 1) / FILL_TP);
-  k_sky_fill<<<grid, SKY_BLOCK, 0, st>>>(dsteps, dso, dlum, ns, np, skyc, sunc, full);
-  ck(hipGetLastError(), "k_sky_fill");
-  if (P.opts.average) {
-    k_sky_average<<<(np * 3 + 255) / 256, 256, 0, st>>>(full, np, ns, 1. / (double)P.ntsteps, P.ntsteps > 1, out);
-    ck(hipGetLastError(), "k_sky_average");
+  if (o.average) {
+    double* part = (double*)(base + L.part);
+    const int nparts = sky_parts(P);
+    k_sky_partial<<<dim3((np + 63) / 64, nparts), SKY_BLOCK, 0, st>>>(dsteps, dso, dlum, ns, np, skyc, sunc, part);
+    ck(hipGetLastError(), "k_sky_partial");
+    k_sky_mean<<<(np * 3 + 255) / 256, 256, 0, st>>>(part, np * 3, nparts, 1. / (double)P.ntsteps, P.ntsteps > 1, out);
+    ck(hipGetLastError(), "k_sky_mean");
+  } else {
+    dim3 grid((ns + FILL_TS - 1) / FILL_TS, (np + FILL_TP - 1) / FILL_TP);
+    k_sky_fill<<<grid, SKY_BLOCK, 0, st>>>(dsteps, dso, dlum, ns, np, skyc, sunc, out);
+    ck(hipGetLastError(), "k_sky_fill");
   }
   ck(hipStreamSynchronize(st), "gendaymtx");
-}
-
-void sky_matrix(const SkyPlan& P, float* out, hipStream_t st) {
-  if (P.nsteps <= 0) return;
-  const SkyScratch L = sky_scratch_layout(P);
-  char* base = nullptr;
-  ck(hipMalloc((void**)&base, L.bytes), "hipMalloc");
-  try {
-    sky_matrix_run(P, out, st, base, L);
-  } catch (...) {
-    (void)hipStreamSynchronize(st);
-    (void)hipFree(base);
-    throw;
-  }
-  (void)hipFree(base);
 }
 
 // ---- the allocation-free form --------------------------------------------------
@@ -764,14 +858,8 @@ static __device__ __align__(256) unsigned char scratch[kSkyScratchBytes];
 static std::mutex g_scratch_mu;                       // calls share one array per device
 static std::unordered_map<int, char*> g_scratch_ptr;   // device -> address of `scratch`
 
-void sky_matrix_noalloc(const SkyPlan& P, float* out, hipStream_t st) {
-  if (P.nsteps <= 0) return;
-  const SkyScratch L = sky_scratch_layout(P);
-  if (L.bytes > kSkyScratchBytes)
-    throw std::runtime_error("gendaymtx needs " + std::to_string(L.bytes) +
-                             " bytes of device scratch; the allocation-free entry point has " +
-                             std::to_string(kSkyScratchBytes) + " (Reinhart MF:4 over 8760 steps fits, without -A)");
-  std::lock_guard<std::mutex> lock(g_scratch_mu);
+// The array's address on the current device; the lock is held.
+static char* scratch_base() {
   int dev = 0;
   ck(hipGetDevice(&dev), "hipGetDevice");
   auto it = g_scratch_ptr.find(dev);
@@ -780,7 +868,79 @@ void sky_matrix_noalloc(const SkyPlan& P, float* out, hipStream_t st) {
     ck(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)), "hipGetSymbolAddress(scratch)");
     it = g_scratch_ptr.emplace(dev, (char*)p).first;
   }
-  sky_matrix_run(P, out, st, it->second, L);
+  return it->second;
+}
+
+void sky_matrix_noalloc(const SkyPlan& P, float* out, hipStream_t st) {
+  if (P.nsteps <= 0) return;
+  const SkyScratch L = sky_scratch_layout(P);
+  if (std::max(L.bytes, L.noalloc) > kSkyScratchBytes)
+    throw std::runtime_error("gendaymtx needs " + std::to_string(std::max(L.bytes, L.noalloc)) +
+                             " bytes of device scratch; the allocation-free entry point has " +
+                             std::to_string(kSkyScratchBytes) + " (Reinhart MF:4 over 8760 steps fits, without -A)");
+  std::lock_guard<std::mutex> lock(g_scratch_mu);
+  sky_matrix_run(P, out, st, scratch_base(), L);
+}
+
+// The allocating form's buffer: one per device, kept while any plan is open
+// (allocating and freeing 84 MB took 200 us of a 720 us call) and given back
+// with the last; a call that finds it in use by another thread, or that needs
+// more than the fixed array above holds, allocates its own.
+struct SkyPool {
+  void* p = nullptr;
+  size_t bytes = 0;
+};
+static std::mutex g_pool_mu;                           // guards the three below; held by the call that uses a buffer
+static std::unordered_map<int, SkyPool> g_pool;
+static std::mutex g_open_mu;
+static int g_open = 0;                                 // plans open
+
+void sky_plan_opened() {
+  std::lock_guard<std::mutex> lock(g_open_mu);
+  ++g_open;
+}
+void sky_plan_closed() {
+  std::lock_guard<std::mutex> open(g_open_mu);
+  if (--g_open > 0) return;
+  std::lock_guard<std::mutex> lock(g_pool_mu);
+  for (auto& kv : g_pool) (void)hipFree(kv.second.p);
+  g_pool.clear();
+}
+
+void sky_matrix(const SkyPlan& P, float* out, hipStream_t st) {
+  if (P.nsteps <= 0) return;
+  const SkyScratch L = sky_scratch_layout(P);
+  if (L.bytes <= kSkyScratchBytes) {
+    std::unique_lock<std::mutex> lock(g_pool_mu, std::try_to_lock);
+    if (lock.owns_lock()) {
+      int dev = 0;
+      ck(hipGetDevice(&dev), "hipGetDevice");
+      SkyPool& b = g_pool[dev];
+      if (b.bytes < L.bytes) {
+        if (b.p) (void)hipFree(b.p);     // every call ends with its stream synchronised
+        b = SkyPool();
+        ck(hipMalloc(&b.p, L.bytes), "hipMalloc");
+        b.bytes = L.bytes;
+      }
+      try {
+        sky_matrix_run(P, out, st, (char*)b.p, L);
+      } catch (...) {
+        (void)hipStreamSynchronize(st);
+        throw;
+      }
+      return;
+    }
+  }
+  char* base = nullptr;
+  ck(hipMalloc((void**)&base, L.bytes), "hipMalloc");
+  try {
+    sky_matrix_run(P, out, st, base, L);
+  } catch (...) {
+    (void)hipStreamSynchronize(st);
+    (void)hipFree(base);
+    throw;
+  }
+  (void)hipFree(base);
 }
 
 }  // namespace rg

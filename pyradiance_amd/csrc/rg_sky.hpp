@@ -66,6 +66,11 @@ SkyPlan sky_plan(const std::string& weather, const SkyOpts& o);
 // Writes the npatch x ncols x 3 matrix to device memory `out`.
 void sky_matrix(const SkyPlan& plan, float* out, hipStream_t st);
 
+// A plan's life: device buffers that calls share are kept while any plan is
+// open and freed with the last.
+void sky_plan_opened();
+void sky_plan_closed();
+
 // Size of the fixed device array the allocation-free form uses (per GPU).
 constexpr size_t kSkyScratchBytes = size_t(96) << 20;
 

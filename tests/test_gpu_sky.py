@@ -74,3 +74,42 @@ def test_sky_matrix_device_feeds_dcsky(L):
     want = np.einsum("mkc,knc->mnc", A.cpu().numpy().astype(np.float64), mtx.astype(np.float64))
     assert np.allclose(Cm.cpu().numpy(), want, rtol=1e-4, atol=1e-3)
     sky.close()
+
+
+def _season(n):
+    """A weather tape of n hours, one sky each, through day and night."""
+    rng = np.random.default_rng(n)
+    rows = []
+    for i in range(n):
+        day, hour = 1 + i // 24 % 28, i % 24
+        up = 5 < hour < 19
+        rows.append(f"{1 + i // 672} {day} {hour + .5} {int(up * rng.integers(0, 800))} {int(up * rng.integers(10, 300))}")
+    return ("place X\nlatitude 37.0\nlongitude 122.0\ntime_zone 120\nsite_elevation 10\n"
+            "weather_data_file_units 1\n" + "\n".join(rows) + "\n")
+
+
+@pytest.mark.parametrize("mf, n", [(1, 1), (1, 63), (1, 64), (1, 65), (3, 150), (4, 129)])
+def test_mean_sky_is_the_mean_of_the_matrix(L, mf, n):
+    """-A against the matrix' own columns, at the edges of the chunks of steps
+    whose sums are taken apart.  Both hold the same float entries; the mean is
+    summed in double and rounded to float once, so it is off by at most half a
+    unit in the last place and the sum's own rounding, which is far below."""
+    from pyradiance_amd import gen
+    _say(f"-A, MF {mf}, {n} steps")
+    full = gen.sky_matrix(_season(n), ["-m", str(mf)])[0]
+    mean = gen.sky_matrix(_season(n), ["-m", str(mf), "-A"])[0]
+    assert full.shape == (144 * mf * mf + 2, n, 3) and mean.shape == (144 * mf * mf + 2, 1, 3)
+    want = full.astype(np.float64).mean(axis=1)
+    assert np.all(np.abs(mean[:, 0] - want) <= 2.0 ** -23 * np.abs(want))
+
+
+def test_skies_from_threads_are_those_of_one(L):
+    """Calls share a device buffer; one that finds it in use takes its own."""
+    from concurrent.futures import ThreadPoolExecutor
+    from pyradiance_amd import gen
+    _say("two threads")
+    jobs = [(_season(n), ["-m", str(mf)]) for mf, n in [(1, 70), (2, 200), (1, 300), (4, 20)]] * 3
+    one = [gen.sky_matrix(*j)[0] for j in jobs]
+    with ThreadPoolExecutor(2) as ex:
+        many = list(ex.map(lambda j: gen.sky_matrix(*j)[0], jobs))
+    assert all(np.array_equal(a, b) for a, b in zip(one, many))
