@@ -231,6 +231,7 @@ int rg_scene_commit(rg_ctx* c) {
     S.lamb = cs.lamb;
     S.cusize = cs.cusize;
     S.shadow_on = 0;
+    S.slots = nullptr;
     c->shadow_filled = false;
     c->cast_count.assign(cs.srcs.size(), 0);
     c->cast_counted.assign(cs.srcs.size(), 0);
@@ -430,8 +431,9 @@ static unsigned long long shadow_count(rg_ctx* c, const uint32_t* tested) {
 
 // device_io: `rays` and `out` are device memory of the context's device
 // batch_ctx: the contexts of the batch's scenes (their shadow caches).
+// slots: per scene, the tracked-modifier slots of its modifier names (mode 1).
 static void run(rg_ctx* c, const double* rays, long long nrays, int accum, int flags, int mode,
-                const std::vector<BinSpec>& bins, int ncols, double* out,
+                const std::vector<BinSpec>& bins, int ncols, const std::vector<std::vector<int32_t>>* slots, double* out,
                 std::vector<DevScene>* batch = nullptr, const std::vector<uint32_t>* batch_start = nullptr,
                 const AdjSpec* adj = nullptr, bool device_io = false,
                 const std::vector<rg_ctx*>* batch_ctx = nullptr) {
@@ -457,7 +459,7 @@ static void run(rg_ctx* c, const double* rays, long long nrays, int accum, int f
     sc_ctx.push_back(c);
     sc_dev.push_back(&Sd);
   }
-  // The call block, cleared once and read back once: error flags (u32, at
+  // The call block, sent cleared and read back once: error flags (u32, at
   // byte 8), then per scene with a shadow cache the closest-hit
   // queries of its cast rays per source (u64, when this call fills the
   // cache: the first call after a commit, as the reference fills a source's
@@ -480,11 +482,13 @@ static void run(rg_ctx* c, const double* rays, long long nrays, int accum, int f
     tested_at[i] = blk;
     blk += (4 * ns + 7) & ~(size_t)7;
   }
-  char* d_blk = (char*)c->arena.get("call", blk, c->st, true);
-  for (size_t i = 0; i < nsc; ++i)
-    if (sc_dev[i]->shadow_on) sc_dev[i]->src_tested = (RG_GLOBAL uint32_t*)(d_blk + tested_at[i]);
-  // inputs in one copy: bin specs, a batch's scene tables, the rays
+  // inputs in one copy: the cleared call block, modifier slots, bin specs, a
+  // batch's scene tables, the rays
   Pack in;
+  const size_t o_blk = in.zero(blk);
+  std::vector<size_t> o_slots;
+  if (slots)
+    for (const auto& v : *slots) o_slots.push_back(in.add(v));
   const size_t o_bins = bins.empty() ? 0 : in.add(bins);
   const size_t o_sc = batch ? in.add(*batch) : 0, o_ss = batch ? in.add(*batch_start) : 0;
   const bool host_rays = nrays && rays && !device_io;
@@ -494,11 +498,12 @@ static void run(rg_ctx* c, const double* rays, long long nrays, int accum, int f
   const bool stage_out = outn && out && !device_io && outn * sizeof(double) <= ((size_t)64 << 20);
   const size_t o_hout = (blk + 255) & ~(size_t)255;
   stage_buf(c, std::max(in.total, o_hout + (stage_out ? sizeof(double) * outn : 0)));
-  char* d_in = nullptr;
-  if (in.total) {
-    d_in = (char*)c->arena.get("call_in", in.total, c->st, false);
-    in.send(c, d_in);
-  }
+  char* d_in = (char*)c->arena.get("call_in", in.total, c->st, false);
+  char* d_blk = d_in + o_blk;
+  for (size_t i = 0; i < nsc; ++i)
+    if (sc_dev[i]->shadow_on) sc_dev[i]->src_tested = (RG_GLOBAL uint32_t*)(d_blk + tested_at[i]);
+  for (size_t i = 0; i < o_slots.size(); ++i) sc_dev[i]->slots = to_global((const int32_t*)(d_in + o_slots[i]));
+  in.send(c, d_in);
   double* d_rays = host_rays ? (double*)(d_in + o_rays)
                              : (double*)c->arena.get("rays", sizeof(double) * 6 * std::max<long long>(nrays, 1), c->st,
                                                       false);
@@ -624,7 +629,7 @@ static void run(rg_ctx* c, const double* rays, long long nrays, int accum, int f
 int rg_trace(rg_ctx* c, const double* rays, long long n, int flags, double* out) {
   RG_TRY(c, {
     std::vector<BinSpec> none;
-    run(c, rays, n, 1, flags, 0, none, 3, out);
+    run(c, rays, n, 1, flags, 0, none, 3, nullptr, out);
   });
 }
 
@@ -649,7 +654,7 @@ int rg_trace_view(rg_ctx* c, const rg_view* v, int xres, int yres, double pj, in
     view_rays(vs, xres, yres, pj, c->params.seed, d_rays, d_valid, c->st);
     hipck(hipGetLastError(), "view rays");
     std::vector<BinSpec> none;
-    run(c, nullptr, n, 1, flags, 0, none, 3, out);
+    run(c, nullptr, n, 1, flags, 0, none, 3, nullptr, out);
     std::vector<uint8_t> valid((size_t)n);
     hipck(hipMemcpy(valid.data(), d_valid, (size_t)n, hipMemcpyDeviceToHost), "view mask");
     for (long long i = 0; i < n; ++i)
@@ -687,33 +692,23 @@ static std::vector<BinSpec> bin_specs(const rg_modifier* mods, int nmods, std::u
   return bins;
 }
 
-// The context's scene with tracked-modifier slots assigned by modifier name
-// (rt/rcontrib.c:289) and every source followed (rt/rcontrib.c:235-237).
-static DevScene contrib_scene(rg_ctx* c, const std::unordered_map<std::string, int>& slot, hipStream_t st) {
+// Tracked-modifier slots of the scene's modifier names (rt/rcontrib.c:289).
+static std::vector<int32_t> contrib_slots(rg_ctx* c, const std::unordered_map<std::string, int>& slot) {
   if (!c->committed) throw std::runtime_error("scene not committed");
-  CompiledScene& cs = c->cs;
-  std::vector<Prim> prims = cs.prims;
-  for (size_t k = 0; k < prims.size(); ++k) {
-    auto it = slot.find(cs.prim_modname[k]);
-    prims[k].modslot = it == slot.end() ? -1 : it->second;
-  }
-  std::vector<Source> srcs = cs.srcs;
-  for (size_t k = 0; k < srcs.size(); ++k) {
-    auto it = slot.find(cs.src_modname[k]);
-    srcs[k].modslot = it == slot.end() ? -1 : it->second;
-    srcs[k].flags |= SFOLLOW;
+  const CompiledScene& cs = c->cs;
+  std::vector<int32_t> slots(cs.mod_names.size(), -1);
+  for (const auto& m : slot) {
+    auto it = cs.mod_index.find(m.first);
+    if (it != cs.mod_index.end()) slots[it->second] = m.second;
   }
   if (c->params.contrib) {
-    for (size_t k = 0; k < prims.size(); ++k) {
-      int mk = prims[k].mat >= 0 ? cs.mats[prims[k].mat].kind : -1;
-      if (prims[k].modslot >= 0 && mk != MK_LIGHT && mk != MK_GLOW && mk != MK_ILLUM)
+    for (const Prim& P : cs.prims) {
+      int mk = P.mat >= 0 ? cs.mats[P.mat].kind : -1;
+      if (slots[P.mod] >= 0 && mk != MK_LIGHT && mk != MK_GLOW && mk != MK_ILLUM)
         throw std::runtime_error("-V+ is supported for light-source modifiers only on the GPU path");
     }
   }
-  DevScene S = c->dscene;
-  S.prims = to_global(upload(c->arena, "prims_c", prims, st));
-  S.srcs = to_global(upload(c->arena, "srcs_c", srcs, st));
-  return S;
+  return slots;
 }
 
 int rg_contrib(rg_ctx* c, const double* rays, long long nrec, int accum, int flags, const rg_modifier* mods,
@@ -722,16 +717,8 @@ int rg_contrib(rg_ctx* c, const double* rays, long long nrec, int accum, int fla
     std::unordered_map<std::string, int> slot;
     int ncols = 0;
     std::vector<BinSpec> bins = bin_specs(mods, nmods, slot, ncols);
-    DevScene S = contrib_scene(c, slot, c->st);
-    DevScene saved = c->dscene;
-    c->dscene = S;
-    try {
-      run(c, rays, nrec * (long long)accum, accum, flags, 1, bins, ncols, out);
-    } catch (...) {
-      c->dscene = saved;
-      throw;
-    }
-    c->dscene = saved;
+    std::vector<std::vector<int32_t>> slots(1, contrib_slots(c, slot));
+    run(c, rays, nrec * (long long)accum, accum, flags, 1, bins, ncols, &slots, out);
   });
 }
 
@@ -756,16 +743,8 @@ int rg_contrib_device(rg_ctx* c, const double* d_rays, long long nrec, int accum
     std::unordered_map<std::string, int> slot;
     int ncols = 0;
     std::vector<BinSpec> bins = bin_specs(mods, nmods, slot, ncols);
-    DevScene S = contrib_scene(c, slot, c->st);
-    DevScene saved = c->dscene;
-    c->dscene = S;
-    try {
-      run(c, d_rays, nrec * (long long)accum, accum, flags, 1, bins, ncols, d_out, nullptr, nullptr, nullptr, true);
-    } catch (...) {
-      c->dscene = saved;
-      throw;
-    }
-    c->dscene = saved;
+    std::vector<std::vector<int32_t>> slots(1, contrib_slots(c, slot));
+    run(c, d_rays, nrec * (long long)accum, accum, flags, 1, bins, ncols, &slots, d_out, nullptr, nullptr, nullptr, true);
   });
 }
 
@@ -797,16 +776,8 @@ int rg_contrib_adjoint(rg_ctx* c, const double* rays, long long nrec, int accum,
       if (adj.row[mi] >= 0) throw std::runtime_error("duplicate material in the gradient list");
       adj.row[mi] = i;
     }
-    DevScene S = contrib_scene(c, slot, c->st);
-    DevScene saved = c->dscene;
-    c->dscene = S;
-    try {
-      run(c, rays, nrec * (long long)accum, accum, flags, 1, bins, ncols, nullptr, nullptr, nullptr, &adj);
-    } catch (...) {
-      c->dscene = saved;
-      throw;
-    }
-    c->dscene = saved;
+    std::vector<std::vector<int32_t>> slots(1, contrib_slots(c, slot));
+    run(c, rays, nrec * (long long)accum, accum, flags, 1, bins, ncols, &slots, nullptr, nullptr, nullptr, &adj);
   });
 }
 
@@ -860,19 +831,20 @@ int rg_contrib_batch(rg_ctx* const* ctxs, int nctx, const double* rays, const lo
     int ncols = 0;
     std::vector<BinSpec> bins = bin_specs(mods, nmods, slot, ncols);
     std::vector<DevScene> scenes;
+    std::vector<std::vector<int32_t>> slots;
     std::vector<uint32_t> start(1, 0);
     long long total = 0;
     for (int i = 0; i < nctx; ++i) {
       if (!ctxs[i] || ctxs[i]->device != c0->device) throw std::runtime_error("batch contexts must share a device");
       if (nrec[i] < 0) throw std::runtime_error("bad record count");
-      scenes.push_back(contrib_scene(ctxs[i], slot, ctxs[i]->st));
-      hipck(hipStreamSynchronize(ctxs[i]->st), "batch upload");
+      slots.push_back(contrib_slots(ctxs[i], slot));
+      scenes.push_back(ctxs[i]->dscene);
       total += nrec[i] * (long long)accum;
       if (total > 0x7fffffffLL) throw std::runtime_error("bad ray count");
       start.push_back((uint32_t)total);
     }
     std::vector<rg_ctx*> cl(ctxs, ctxs + nctx);
-    run(c0, rays, total, accum, flags, 1, bins, ncols, out, &scenes, &start, nullptr, false, &cl);
+    run(c0, rays, total, accum, flags, 1, bins, ncols, &slots, out, &scenes, &start, nullptr, false, &cl);
   });
 }
 
@@ -899,7 +871,7 @@ int rg_trace_batch(rg_ctx* const* ctxs, int nctx, const double* rays, const long
     }
     std::vector<BinSpec> none;
     std::vector<rg_ctx*> cl(ctxs, ctxs + nctx);
-    run(c0, rays, total, 1, flags, 0, none, 3, out, &scenes, &start, nullptr, false, &cl);
+    run(c0, rays, total, 1, flags, 0, none, 3, nullptr, out, &scenes, &start, nullptr, false, &cl);
   });
 }
 

@@ -94,6 +94,11 @@ struct DevScene {
   const RG_GLOBAL SrcCache* scache;             // per source
   const RG_GLOBAL unsigned long long* shadow_obs;  // blocker cells: (sequence+1) << 32 | primitive; 0 empty
   RG_GLOBAL uint32_t* src_tested;               // per source: shadow-tested during the current call
+  // per modifier name, set for each rcontrib call: tracked-modifier slot, -1
+  // untracked.  (Slots in the primitive records meant hashing every
+  // primitive's name and sending all records again on each call: 5 of 100 ms for
+  // a three-storey office, 18 of 288 us for one desk.)
+  const RG_GLOBAL int32_t* slots;
 };
 
 struct HitRec {

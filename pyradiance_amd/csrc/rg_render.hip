@@ -622,9 +622,11 @@ __device__ __forceinline__ void adjoint_deposit(const DevScene& S, const RunCfg&
 }
 
 // rcontrib's trace callback (rt/rcontrib.c:272-316) in coefficient mode.
-__device__ __forceinline__ void trace_contrib(const DevScene& S, const RunCfg& c, const RayS& r, int modslot, int hitobj,
+__device__ __forceinline__ void trace_contrib(const DevScene& S, const RunCfg& c, const RayS& r, int mod, int hitobj,
                               bool zeroed, C3 rcol) {
-  if (c.mode != 1 || modslot < 0 || zeroed) return;
+  if (c.mode != 1 || zeroed) return;
+  const int modslot = S.slots[mod];
+  if (modslot < 0) return;
   if (r.rsrc >= 0 && src_obj(S.srcs[r.rsrc], r.rsrc) != hitobj) return;
   C3 contr = r.coef;
   if (c.p.contrib) {
@@ -1257,7 +1259,7 @@ __device__ __forceinline__ void shade_hit(const DevScene& S, const RunCfg& c, co
       if (c.mode == 0) deposit(c, r.sensor, 0, r.coef * em);
     }
   }
-  trace_contrib(S, c, r, P.modslot, h.prim, zeroed, rcol);
+  trace_contrib(S, c, r, P.mod, h.prim, zeroed, rcol);
   if (act == NORMAL) {
     shade_normal(S, c, r, hs, S.mats[mi], dmi, sk);
   } else if (act == GLASS) {
@@ -1279,11 +1281,11 @@ __device__ __forceinline__ void shade_miss(const DevScene& S, const RunCfg& c, c
   bool pass;
   bool ok = light_rules(S, c, r, m, -(2 + si), FHUGE, 1.0, &em, &pass);
   if (!ok || pass) {
-    trace_contrib(S, c, r, src.modslot, -(2 + si), true, em);
+    trace_contrib(S, c, r, src.mod, -(2 + si), true, em);
     return;
   }
   if (c.mode == 0) deposit(c, r.sensor, 0, r.coef * em);
-  trace_contrib(S, c, r, src.modslot, -(2 + si), false, em);
+  trace_contrib(S, c, r, src.mod, -(2 + si), false, em);
 }
 
 // ---- kernels -----------------------------------------------------------------

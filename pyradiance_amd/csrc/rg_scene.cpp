@@ -453,6 +453,11 @@ CompiledScene compile_scene(const SceneDB& db) {
   }
   std::vector<int> obj_prim(nobj, -1);
   std::vector<std::array<double, 6>> dbounds;
+  auto mod_id = [&](const std::string& name) {
+    auto it = cs.mod_index.emplace(name, (int32_t)cs.mod_names.size());
+    if (it.second) cs.mod_names.push_back(name);
+    return it.first->second;
+  };
   // One surface object -> one primitive (-1 if degenerate).  mo: material
   // object, omod: modifier that ranks coincident hits and names the
   // primitive for rcontrib; flat: isflat() of the object reported as hit.
@@ -461,7 +466,7 @@ CompiledScene compile_scene(const SceneDB& db) {
     memset(&P, 0, sizeof P);
     P.mat = material_index(mo);
     P.omod = omod;
-    P.modslot = -1;
+    P.mod = mod_id(objs[omod].name);
     P.srcidx = -1;
     P.goff = (int)cs.geom.size();
     P.nv = 0;
@@ -594,7 +599,6 @@ CompiledScene compile_scene(const SceneDB& db) {
     if (!flat) P.flat = 0;
     int idx = (int)cs.prims.size();
     cs.prims.push_back(P);
-    cs.prim_modname.push_back(objs[omod].name);
     dbounds.push_back({lo[0], lo[1], lo[2], hi[0], hi[1], hi[2]});
     grow(lo, hi);
     return idx;
@@ -643,7 +647,7 @@ CompiledScene compile_scene(const SceneDB& db) {
       P.kind = PK_TRIANGLE;
       P.mat = material_index(mo);
       P.omod = mod;
-      P.modslot = -1;
+      P.mod = mod_id(objs[mod].name);
       P.srcidx = -1;
       P.goff = (int)cs.geom.size();
       P.nv = 3;
@@ -668,7 +672,6 @@ CompiledScene compile_scene(const SceneDB& db) {
       cube_point(b);
       cube_point(c);
       cs.prims.push_back(P);
-      cs.prim_modname.push_back(objs[mod].name);
       dbounds.push_back({lo[0], lo[1], lo[2], hi[0], hi[1], hi[2]});
       grow(lo, hi);
     }
@@ -786,7 +789,7 @@ CompiledScene compile_scene(const SceneDB& db) {
     S.prim = -1;
     S.mat = material_index(mo);
     S.objmod = o.omod;
-    S.modslot = -1;
+    S.mod = mod_id(objs[o.omod].name);
     const auto& f = o.fargs;
     auto setflatss = [&]() {
       double u[3];
@@ -893,7 +896,6 @@ CompiledScene compile_scene(const SceneDB& db) {
       if (S.flags & SDISTANT) S.flags |= SSKIP;
     }
     cs.srcs.push_back(S);
-    cs.src_modname.push_back(objs[o.omod].name);
   }
   if (cs.srcs.size() > 32000) throw RadError("too many light sources for the GPU path");
   shadow_cache_setup(cs);

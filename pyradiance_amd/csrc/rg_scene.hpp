@@ -1,6 +1,7 @@
 // Scene compilation: Radiance objects -> flat device tables.
 #pragma once
 #include <string>
+#include <unordered_map>
 #include <vector>
 #include "rg_types.hpp"
 #include "scene_io.hpp"
@@ -14,8 +15,8 @@ struct CompiledScene {
   std::vector<std::string> mat_names;        // name of each material object
   std::vector<Source> srcs;
   std::vector<float> lo, hi;                 // widened FP32 bounds per primitive
-  std::vector<std::string> prim_modname;     // name of each primitive's modifier
-  std::vector<std::string> src_modname;      // name of each source object's modifier
+  std::vector<std::string> mod_names;        // distinct modifier names of primitives and sources (Prim.mod)
+  std::unordered_map<std::string, int32_t> mod_index;   // their indices
   std::vector<std::string> warnings;
   double bmin[3], bmax[3];
   double cusize = 0;

@@ -79,7 +79,7 @@ struct Material {
 // Source flags (rt/source.h)
 enum : int32_t {
   SDISTANT = 01, SSKIP = 02, SPROX = 04, SSPOT = 010, SVIRTUAL = 020,
-  SFLAT = 040, SCYL = 0100, SFOLLOW = 0200, SCIR = 01000,
+  SFLAT = 040, SCYL = 0100, SCIR = 01000,
 };
 
 struct Source {
@@ -92,7 +92,7 @@ struct Source {
   int32_t flags;
   int32_t prim;      // primitive index for local sources, -1 for distant
   int32_t mat;       // material index of the emitter
-  int32_t modslot;   // tracked-modifier slot of the source object (-1 none)
+  int32_t mod;       // name of the source object's modifier, as Prim.mod
   int32_t objmod;    // modifier object number (tie rule / identity)
   int32_t pad;
 };
@@ -125,7 +125,7 @@ struct Prim {
   int32_t kind;      // PrimKind
   int32_t mat;       // resolved material index (-1: none)
   int32_t omod;      // modifier object number, the "later modifier wins" key
-  int32_t modslot;   // tracked-modifier slot (rcontrib), -1 if untracked
+  int32_t mod;       // name of its modifier: index into the scene's distinct names
   int32_t goff;      // offset into geometry pool (doubles)
   int32_t nv;        // polygon vertex count
   int32_t flat;      // PF_FLAT | PF_COMPLEX bits

@@ -680,3 +680,44 @@ def test_small_product_against_fp64(L, m, k, n):
         ref = a[:, :, ch].double().contiguous() @ b[:, :, ch].double().contiguous()
         rel = ((c[:m, :, ch].double() - ref) / ref).abs().max().item()
         assert rel <= (3 * 2.0 ** -16 if split else 0) + (k + 1) * 2.0 ** -24, (ch, rel)
+
+
+def test_tracked_modifiers_belong_to_the_call_and_the_scene(L):
+    """Which modifiers are tracked changes from call to call on one context,
+    and a batch's scenes number the same names differently: every column is
+    that of its modifier, bit for bit, and an unknown name's stays zero."""
+    _say("tracked modifiers per call and per scene")
+    sky = ("void glow sky 0 0 4 1 1 1 0\nsky source up 0 0 4 0 0 1 180\n",
+           "void glow ground 0 0 4 1 1 1 0\nground source down 0 0 4 0 0 -1 180\n",
+           "void plastic wall 0 0 5 .5 .5 .5 0 0\nwall polygon w 0 0 12 1 -1 -1 1 1 -1 1 1 1 1 -1 1\n"
+           "wall polygon v 0 0 12 -2 -1 1 -2 1 1 -2 1 -1 -2 -1 -1\n",
+           "void plastic roof 0 0 5 .3 .3 .3 0 0\nroof polygon r 0 0 12 -1 -1 2 -1 1 2 0 1 2 0 -1 2\n")
+    texts = ["".join(sky), "".join(reversed(sky)), sky[0] + sky[2]]
+    rng = np.random.default_rng(3)
+    sens = [np.hstack([rng.uniform(-.5, .5, (n, 3)), np.tile([0., 0., 1.], (n, 1))]) for n in (7, 65, 1)]
+    p = _rc_params(L, ambounce=2, ambdiv=128, minweight=1e-3, seed=4)
+    names = ["roof", "sky", "nobody", "wall", "ground"]
+
+    def mods(ns):
+        out = [L.RgModifier() for _ in ns]
+        for m, n in zip(out, ns):
+            m.name, m.bin_kind, m.nbins, m.cbin = n.encode(), 0, 1, 0
+        return out
+
+    single = []
+    for k, (t, s) in enumerate(zip(texts, sens)):
+        c = _ctx(L, t)
+        p.seed = 4 + k
+        c.set_params(p)
+        full = c.contrib(s, mods(names), 1, L.RT_IMM_IRRAD).reshape(len(s), -1, 3)
+        assert not full[:, 2].any() and full[:, 1].any() and full[:, 3].any()
+        for ns in (["wall"], ["ground", "sky"], names[::-1]):
+            got = c.contrib(s, mods(ns), 1, L.RT_IMM_IRRAD).reshape(len(s), -1, 3)
+            assert np.array_equal(got, full[:, [names.index(n) for n in ns]]), (k, ns)
+        single.append(full)
+    assert single[0][:, 0].any() and not single[2][:, 0].any()
+    ctxs = [_ctx(L, t) for t in texts]
+    p.seed = 4
+    ctxs[0].set_params(p)
+    for got, want in zip(L.contrib_batch(ctxs, sens, mods(names), 1, L.RT_IMM_IRRAD), single):
+        assert np.array_equal(got.reshape(want.shape), want)
