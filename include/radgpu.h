@@ -187,9 +187,7 @@ int rg_set_profiling(rg_ctx *ctx, int level);
  * every shadow ray is traced; "child_order" 1 (default) hands hemisphere
  * children to wavefronts in 8 x 8 blocks of strata, 0 by stratum row (same
  * samples); "inflight" 1 (default) runs one window at a time, 2 queues the
- * next window before reading back the counts of the one before (the GPU
- * then waits less for the host, but the traversal slows by more on config 2:
- * 53.2 against 52.7 ms per step).
+ * next window before reading back the counts of the one before.
  * Results do not depend on these; only the time does (the walks visit
  * primitives in different orders, which only matters for two surfaces
  * within FTINY of each other along a ray, where the reference's own choice
@@ -208,11 +206,12 @@ int rg_last_stats(rg_ctx *ctx, double *out, int n);
 
 /* DC x sky product, replaces cm_multiply() (util/cmatrix.c:421-474):
  * C[M][N][3] = A[M][K][3] . B[K][N][3], each channel independently.
- * Host pointers.  mode 0 = FP32 accumulate, 1 = BF16 hi/lo split MFMA
- * (K <= 160: rows of A held in registers, sky columns streamed through LDS;
- * K > 256: 128 x 128 tiles over a ring of LDS buffers, K shared by several
- * blocks when there are few tiles; otherwise per-wavefront operand loads),
- * 2 / 3 / 4 = the split product forced to per-wavefront loads / the ring of
+ * Host pointers.  mode 0 = FP32 accumulate, 1 = products of at most 2^23
+ * multiply-adds per channel (2^24 for N >= 256 and M >= 4) and K <= 1024 in
+ * one FP32 launch, larger ones BF16 hi/lo split MFMA (K <= 160: rows of A
+ * held in registers, sky columns streamed through LDS; longer K: 128 x 128
+ * tiles over a ring of LDS buffers, K shared by several blocks when there are
+ * few tiles), 2 / 3 / 4 = the split product forced to per-wavefront loads / the ring of
  * LDS buffers / the short-K form (K <= 160).  The split planes (and a shared
  * K's partial products) live in a buffer kept per device and stream, grown
  * as needed and held until the process ends (2 * 3 * (M + N) * K * 2 bytes,
