@@ -7,7 +7,6 @@
 // (AddDirect :828-872) and the averaged sky (-A).
 #include "rg_sky.hpp"
 
-#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -446,11 +445,12 @@ struct SkyStepOut {
 // them (gen/gendaymtx.c:1221-1264).
 //
 // One array per term, `n` patches long, so that a wavefront's loads are whole
-// runs (as 80-byte records they touched a line per lane).
+// runs (as 64-byte records they touched a line per lane).  The solid angle is
+// read from the uploaded floats: with it the terms would take more than the 64
+// bytes per patch that the fixed array of the allocation-free form is sized for.
 enum : int { TAB_CZP, TAB_SZP,      // cos, sin of the patch zenith angle
-             TAB_SIN, TAB_DOM,      // sin(altitude), solid angle
              TAB_CA, TAB_SA,        // cos, sin of the azimuth
-             TAB_X, TAB_Y, TAB_Z,   // rh_vector() direction
+             TAB_X, TAB_Y, TAB_Z,   // rh_vector() direction; z is sin(altitude)
              TAB_ROW,               // altitude row, 0 at the horizon (patches of a row share czp)
              TAB_TERMS };
 
@@ -501,15 +501,13 @@ __device__ __forceinline__ bool sun_before(double xd, int xp, double yd, int yp)
   return xp >= 0 && (yp < 0 || xd > yd || (xd == yd && xp < yp));
 }
 
-__global__ void k_sky_patch(const float* __restrict__ palt, const float* __restrict__ pazi,
-                            const float* __restrict__ dom, int np, int mf, double* __restrict__ tab) {
+__global__ void k_sky_patch(const float* __restrict__ palt, const float* __restrict__ pazi, int np, int mf,
+                            double* __restrict__ tab) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= np) return;
   const double zsa = kPI * 0.5 - (double)palt[p];
   tab[TAB_CZP * np + p] = cos(zsa);
   tab[TAB_SZP * np + p] = sin(zsa);
-  tab[TAB_SIN * np + p] = sin((double)palt[p]);
-  tab[TAB_DOM * np + p] = (double)dom[p];
   tab[TAB_CA * np + p] = cos((double)pazi[p]);
   tab[TAB_SA * np + p] = sin((double)pazi[p]);
   // rows of the Reinhart division: mf rows of tnaz[k] mf patches for k = 0..6
@@ -552,9 +550,9 @@ __device__ __forceinline__ int rowp(int r, int mf, int np) {
 // reference's one sequential pass (largest dot products, ties to the lower
 // patch).
 __global__ void __launch_bounds__(SKY_BLOCK) k_sky_step(const SkyStep* __restrict__ steps, int nsteps,
-                                                        const double* __restrict__ tab, int np, int mf, int nsuns,
-                                                        double fixed_sa, float* __restrict__ lum,
-                                                        SkyStepOut* __restrict__ out) {
+                                                        const double* __restrict__ tab, const float* __restrict__ dom,
+                                                        int np, int mf, int nsuns, double fixed_sa,
+                                                        float* __restrict__ lum, SkyStepOut* __restrict__ out) {
   const int s = blockIdx.x;
   if (s >= nsteps) return;
   const SkyStep k = steps[s];
@@ -589,19 +587,22 @@ __global__ void __launch_bounds__(SKY_BLOCK) k_sky_step(const SkyStep* __restric
   if (k.kind == 2 || k.add_sun) {
     // a patch's table entries are requested while the one before is evaluated
     double t[TAB_TERMS], nx[TAB_TERMS];
+    float td, nxd;                            // solid angle
     auto fetch = [&](int p) {
 #pragma unroll
       for (int q = 0; q < TAB_TERMS; ++q) nx[q] = tab[q * np + min(p, np - 1)];
+      nxd = dom[min(p, np - 1)];
     };
     fetch(1 + tid);
     for (int p = 1 + tid; p < np; p += SKY_BLOCK) {
 #pragma unroll
       for (int q = 0; q < TAB_TERMS; ++q) t[q] = nx[q];
+      td = nxd;
       fetch(p + SKY_BLOCK);
       if (k.kind == 2) {
         const float f = patch_lum(k, grad[(int)t[TAB_ROW]], czs, szs, cas, sas, t);
         lrow[p] = f;
-        acc += (double)f * t[TAB_SIN] * t[TAB_DOM];
+        acc += (double)f * t[TAB_Z] * (double)td;
       }
       if (k.add_sun) top_insert(nd, npch, nsuns, t[TAB_X] * sv[0] + t[TAB_Y] * sv[1] + t[TAB_Z] * sv[2], p);
     }
@@ -663,7 +664,7 @@ __global__ void __launch_bounds__(SKY_BLOCK) k_sky_step(const SkyStep* __restric
       for (int i = 0; i < MAXSUN; ++i) {
         if (i >= nsuns || cp[i] < 0) continue;
         float va = (float)(wta[i] * k.dir_illum / (WHTEFFICACY * wtot));
-        va = (float)((double)va / (fixed_sa > 0 ? fixed_sa : tab[TAB_DOM * np + cp[i]]));
+        va = (float)((double)va / (fixed_sa > 0 ? fixed_sa : (double)dom[cp[i]]));
         o.sunp[i] = cp[i];
         o.sunv[i] = va;
         o.nsun = i + 1;
@@ -783,10 +784,13 @@ void ck(hipError_t e, const char* what) {
 // Device buffers of one sky_matrix() call, laid out in one block (256-byte
 // aligned parts): the uploaded step records and patch altitude / azimuth /
 // solid angle, then step outputs, patch tables, the luminance plane, and with
-// -A the partial sums.
+// -A the partial sums (over the patch tables, which are not read any more by
+// then, where they fit: one step's sums are more than its share of a matrix).
 struct SkyScratch {
   size_t steps, so, tab, alt, azi, dom, lum, part, bytes;
-  size_t noalloc;      // what the allocation-free form counts: with -A a whole matrix as well
+  // what the allocation-free form accepts a plan by: with -A a whole matrix
+  // in place of the partial sums, never less than `bytes`
+  size_t noalloc;
 };
 
 static int sky_parts(const SkyPlan& P) { return (P.nsteps + MEAN_TS - 1) / MEAN_TS; }
@@ -803,9 +807,12 @@ static SkyScratch sky_scratch_layout(const SkyPlan& P) {
   L.so = o;    o = up(o + sizeof(SkyStepOut) * ns);
   L.tab = o;   o = up(o + sizeof(double) * TAB_TERMS * np);
   L.lum = o;   o = up(o + sizeof(float) * np * ns);
-  L.part = o;  if (P.opts.average) o = up(o + sizeof(double) * 3 * np * sky_parts(P));
+  L.noalloc = o + (P.opts.average ? sizeof(float) * 3 * np * ns : 0);
+  const size_t part = P.opts.average ? sizeof(double) * 3 * np * sky_parts(P) : 0;
+  const bool over = part <= sizeof(double) * TAB_TERMS * np;
+  L.part = over ? L.tab : o;
+  if (!over) o = up(o + part);
   L.bytes = o;
-  L.noalloc = L.part + (P.opts.average ? sizeof(float) * 3 * np * ns : 0);
   return L;
 }
 
@@ -823,11 +830,11 @@ static void sky_matrix_run(const SkyPlan& P, float* out, hipStream_t st, char* b
   ck(hipMemcpyAsync(dalt, P.palt.data(), sizeof(float) * np, hipMemcpyHostToDevice, st), "upload");
   ck(hipMemcpyAsync(dazi, P.pazi.data(), sizeof(float) * np, hipMemcpyHostToDevice, st), "upload");
   ck(hipMemcpyAsync(ddom, P.dom.data(), sizeof(float) * np, hipMemcpyHostToDevice, st), "upload");
-  k_sky_patch<<<(np + 255) / 256, 256, 0, st>>>(dalt, dazi, ddom, np, mf, dtab);
+  k_sky_patch<<<(np + 255) / 256, 256, 0, st>>>(dalt, dazi, np, mf, dtab);
   ck(hipGetLastError(), "k_sky_patch");
   int nsuns = P.opts.nsuns < 1 ? 1 : (P.opts.nsuns > MAXSUN ? MAXSUN : P.opts.nsuns);
-  k_sky_step<<<ns, SKY_BLOCK, sizeof(double) * (7 * mf + 1), st>>>(dsteps, ns, dtab, np, mf, nsuns, P.opts.fixed_sun_sa,
-                                                                   dlum, dso);
+  k_sky_step<<<ns, SKY_BLOCK, sizeof(double) * (7 * mf + 1), st>>>(dsteps, ns, dtab, ddom, np, mf, nsuns,
+                                                                   P.opts.fixed_sun_sa, dlum, dso);
   ck(hipGetLastError(), "k_sky_step");
   const SkyOpts& o = P.opts;
   float3 skyc = make_float3((float)o.sky_color[0], (float)o.sky_color[1], (float)o.sky_color[2]);
@@ -874,10 +881,11 @@ static char* scratch_base() {
 void sky_matrix_noalloc(const SkyPlan& P, float* out, hipStream_t st) {
   if (P.nsteps <= 0) return;
   const SkyScratch L = sky_scratch_layout(P);
-  if (std::max(L.bytes, L.noalloc) > kSkyScratchBytes)
-    throw std::runtime_error("gendaymtx needs " + std::to_string(std::max(L.bytes, L.noalloc)) +
-                             " bytes of device scratch; the allocation-free entry point has " +
-                             std::to_string(kSkyScratchBytes) + " (Reinhart MF:4 over 8760 steps fits, without -A)");
+  if (L.noalloc > kSkyScratchBytes)
+    throw std::runtime_error("gendaymtx: a plan of " + std::to_string(L.noalloc) +
+                             " bytes (device scratch, with -A that of the whole matrix); the allocation-free entry "
+                             "point takes plans of up to " + std::to_string(kSkyScratchBytes) +
+                             " (Reinhart MF:4 over 8760 steps, without -A)");
   std::lock_guard<std::mutex> lock(g_scratch_mu);
   sky_matrix_run(P, out, st, scratch_base(), L);
 }
