@@ -41,6 +41,44 @@ struct alignas(16) BVH4Q {
 };
 static_assert(sizeof(BVH4Q) == 64, "one node, half a cache line");
 
+// Whether and where a ray enters the four rounded boxes of a node: key[k] is
+// the entry distance as an integer with the child's slot k in the low two
+// bits, or kNoEntry.  ot: origin times inverse direction, iv: inverse
+// direction, tlim: boxes entered beyond it are left out.  An axis whose
+// distances are not numbers does not bound a box (fmaxf and fminf drop them).
+constexpr uint32_t kNoEntry = 0xffffffffu;
+RG_HD void walk_keys(const BVH4Q& q, const float ot[3], const float iv[3], float tlim, uint32_t key[4]) {
+  const bool mx = iv[0] < 0.f, my = iv[1] < 0.f, mz = iv[2] < 0.f;
+  const uint32_t nx = mx ? q.hix : q.lox, fx = mx ? q.lox : q.hix;
+  const uint32_t ny = my ? q.hiy : q.loy, fy = my ? q.loy : q.hiy;
+  const uint32_t nz = mz ? q.hiz : q.loz, fz = mz ? q.loz : q.hiz;
+  const float ax = q.scale[0] * iv[0], ay = q.scale[1] * iv[1], az = q.scale[2] * iv[2];
+  const float bx = fmaf(q.org[0], iv[0], -ot[0]), by = fmaf(q.org[1], iv[1], -ot[1]), bz = fmaf(q.org[2], iv[2], -ot[2]);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    auto byte = [&](uint32_t v) { return (float)((v >> (8 * k)) & 255u); };
+    const float tn = fmaxf(fmaxf(fmaxf(fmaf(byte(nx), ax, bx), fmaf(byte(ny), ay, by)), fmaf(byte(nz), az, bz)), 0.f);
+    const float tf = fminf(fminf(fminf(fmaf(byte(fx), ax, bx), fmaf(byte(fy), ay, by)), fmaf(byte(fz), az, bz)), tlim);
+    uint32_t bits;
+    __builtin_memcpy(&bits, &tn, 4);
+    const bool hit = (tn <= tf) & (q.child[k] != INT32_MIN);
+    key[k] = hit ? ((bits & ~3u) | (uint32_t)k) : kNoEntry;
+  }
+}
+
+// The walk's limit on entry distances for a hit at distance t; below every
+// entry when t is not a number.
+RG_HD float walk_limit(double t) {
+  const float f = (float)(t + 2 * FTINY) * 1.000001f;
+  return f == f ? f : -1.f;
+}
+// The same for a ray that starts its walk: no axis of one that is not a
+// number in all three would bound a box, and it would visit the whole tree.
+RG_HD float walk_start(double t, const float ot[3]) {
+  const bool none = (ot[0] != ot[0]) & (ot[1] != ot[1]) & (ot[2] != ot[2]);
+  return none ? -1.f : walk_limit(t);
+}
+
 // A primitive as the walk tests it, in one cache line.  Polygons of three or
 // four vertices: plane, then the vertices in the two coordinates of the
 // inside test (a triangle's last one twice); other shapes hold only their

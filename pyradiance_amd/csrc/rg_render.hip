@@ -1747,7 +1747,6 @@ k_walk4(DevScene Sarg, RunCfg c, const RayGeo* geo, const RaySt* st, RayMap map,
   __shared__ uint64_t stk[WSTACK * BS];         // (entry distance, child)
   constexpr int32_t DONE = INT32_MIN;
   constexpr uint32_t kUnits = kChunk / 64;      // units of 64 rays per chunk
-  constexpr uint32_t kNoHit = 0xffffffffu;
   const int lane = threadIdx.x;
   const uint32_t nunit = map.nchunk * kUnits;
   uint64_t deep[WDEEP];
@@ -1764,7 +1763,6 @@ k_walk4(DevScene Sarg, RunCfg c, const RayGeo* geo, const RaySt* st, RayMap map,
   int sp = 0;
   float ox = 0, oy = 0, oz = 0, ix = 0, iy = 0, iz = 0, tlim = 0;
   uint32_t nvis = 0, nprim = 0;
-  auto limit = [](double t) { return (float)(t + 2 * FTINY) * 1.000001f; };
   // next subtree whose box starts within the current closest hit
   auto pop = [&]() -> int32_t {
     while (sp > 0) {
@@ -1806,7 +1804,6 @@ k_walk4(DevScene Sarg, RunCfg c, const RayGeo* geo, const RaySt* st, RayMap map,
           h = first_hit_of(BATCH || S.nbig > 0, outp, tcur);
           o = v3(g.o[0], g.o[1], g.o[2]);
           d = v3(g.d[0], g.d[1], g.d[2]);
-          tlim = limit(h.t);
           node = 0;
           leaf = -1;
           sp = 0;
@@ -1817,6 +1814,8 @@ k_walk4(DevScene Sarg, RunCfg c, const RayGeo* geo, const RaySt* st, RayMap map,
           };
           ix = inv(d.x); iy = inv(d.y); iz = inv(d.z);
           ox = (float)o.x * ix; oy = (float)o.y * iy; oz = (float)o.z * iz;   // origin x inverse direction
+          const float ot[3] = {ox, oy, oz};
+          tlim = walk_start(h.t, ot);
         }
         rpos += take;
       }
@@ -1833,25 +1832,16 @@ k_walk4(DevScene Sarg, RunCfg c, const RayGeo* geo, const RaySt* st, RayMap map,
       if (nn == 0u || (nn < RG_NODE_LANES && __ballot(leaf >= 0))) break;
       if (node >= 0) {
         const RG_GLOBAL u32x4* np = (const RG_GLOBAL u32x4*)(S.nodes4 + node);
-        const u32x4 w0 = np[0], w1 = np[1], w2 = np[2], w3 = np[3];
-        ++nvis;
-        const float gx = __uint_as_float(w0[0]), gy = __uint_as_float(w0[1]), gz = __uint_as_float(w0[2]);
-        const float sx = __uint_as_float(w0[3]), sy = __uint_as_float(w1[0]), sz = __uint_as_float(w1[1]);
-        const bool mx = ix < 0.f, my = iy < 0.f, mz = iz < 0.f;
-        const uint32_t nx = mx ? w1[3] : w1[2], fx = mx ? w1[2] : w1[3];
-        const uint32_t ny = my ? w2[1] : w2[0], fy = my ? w2[0] : w2[1];
-        const uint32_t nz = mz ? w2[3] : w2[2], fz = mz ? w2[2] : w2[3];
-        const float ax = sx * ix, ay = sy * iy, az = sz * iz;
-        const float bx = fmaf(gx, ix, -ox), by = fmaf(gy, iy, -oy), bz = fmaf(gz, iz, -oz);
-        uint32_t key[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          auto byte = [&](uint32_t v) { return (float)((v >> (8 * k)) & 255u); };
-          const float tn = fmaxf(fmaxf(fmaxf(fmaf(byte(nx), ax, bx), fmaf(byte(ny), ay, by)), fmaf(byte(nz), az, bz)), 0.f);
-          const float tf = fminf(fminf(fminf(fmaf(byte(fx), ax, bx), fmaf(byte(fy), ay, by)), fmaf(byte(fz), az, bz)), tlim);
-          const bool hit = (tn <= tf) & ((int32_t)w3[k] != DONE);
-          key[k] = hit ? ((__float_as_uint(tn) & ~3u) | (uint32_t)k) : kNoHit;
+        BVH4Q q;
+        {
+          const u32x4 w0 = np[0], w1 = np[1], w2 = np[2], w3 = np[3];
+          const u32x4 w[4] = {w0, w1, w2, w3};
+          __builtin_memcpy(&q, w, sizeof w);
         }
+        ++nvis;
+        const float ot[3] = {ox, oy, oz}, iv[3] = {ix, iy, iz};
+        uint32_t key[4];
+        walk_keys(q, ot, iv, tlim, key);
         auto cx = [&](int a, int b) {
           const uint32_t lo = min(key[a], key[b]), hi = max(key[a], key[b]);
           key[a] = lo;
@@ -1859,17 +1849,17 @@ k_walk4(DevScene Sarg, RunCfg c, const RayGeo* geo, const RaySt* st, RayMap map,
         };
         cx(0, 1); cx(2, 3); cx(0, 2); cx(1, 3); cx(1, 2);
         auto child = [&](uint32_t k) -> uint32_t {
-          const uint32_t a = (k & 1u) ? w3[1] : w3[0], b = (k & 1u) ? w3[3] : w3[2];
+          const uint32_t a = (k & 1u) ? q.child[1] : q.child[0], b = (k & 1u) ? q.child[3] : q.child[2];
           return (k & 2u) ? b : a;
         };
-        if (key[0] == kNoHit) {
+        if (key[0] == kNoEntry) {
           node = pop();
         } else {
           node = (int32_t)child(key[0]);
-          if (key[1] != kNoHit) {
+          if (key[1] != kNoEntry) {
             auto entry = [&](uint32_t k) { return ((uint64_t)(k & ~3u) << 32) | child(k); };
             const uint64_t e1 = entry(key[1]), e2 = entry(key[2]), e3 = entry(key[3]);
-            const int h2 = key[2] != kNoHit, h3 = key[3] != kNoHit;
+            const int h2 = key[2] != kNoEntry, h3 = key[3] != kNoEntry;
             if (sp <= WSTACK - 3) {
               // farthest first; a slot that is not used is overwritten
               stk[sp * BS + lane] = e3;
@@ -1908,7 +1898,7 @@ k_walk4(DevScene Sarg, RunCfg c, const RayGeo* geo, const RaySt* st, RayMap map,
       }
       const float ot[3] = {ox, oy, oz}, iv[3] = {ix, iy, iz};
       hit_leaf_ordered(S, L, leaf, o, d, ot, iv, h);
-      tlim = limit(h.t);
+      tlim = walk_limit(h.t);
       ++nprim;
       leaf = -1;
       if ((node < 0) & (node != DONE)) {

@@ -204,3 +204,119 @@ extern "C" int check_order(int n, int nrays, unsigned seed, int grid, long* pair
   }
   return bad;
 }
+
+// A ray's origin and direction as the walk holds them.
+static void walk_ray(const double o[3], const double d[3], float ot[3], float iv[3]) {
+  for (int a = 0; a < 3; ++a) {
+    float f = (float)d[a];
+    if (std::fabs(f) < 1e-20f) f = f < 0 ? -1e-20f : 1e-20f;
+    iv[a] = 1.0f / f;
+    ot[a] = (float)o[a] * iv[a];
+  }
+}
+
+// Boxes within a scene of side `ext` about the origin, widened as a commit
+// widens primitives (1e-5 + 4e-6 ext), four to a rounded node: a ray from up
+// to `far` sides away through a point of an unwidened box enters that box by
+// the walk's own FP32 arithmetic, also with a hit at that point already
+// found.  flat: boxes without thickness in one axis, and rays along axes.
+// Returns the number of rays that miss.
+extern "C" long check_walk_boxes(int n, int nrays, unsigned seed, double ext, double far, int flat) {
+  using namespace rg;
+  std::mt19937 rng(seed);
+  std::uniform_real_distribution<double> U(0.0, 1.0);
+  const double eps = 1e-5 + 4e-6 * ext;
+  long bad = 0;
+  for (int i = 0; i < n; ++i) {
+    BVH4Node N = {};
+    float* lo[3] = {N.lox, N.loy, N.loz};
+    float* hi[3] = {N.hix, N.hiy, N.hiz};
+    double blo[4][3], bhi[4][3];
+    const double e = ext * std::pow(10.0, -4 + 4 * U(rng));
+    for (int k = 0; k < 4; ++k) {
+      N.child[k] = ~k;
+      const int thin = flat ? (int)(rng() % 3) : -1;
+      for (int a = 0; a < 3; ++a) {
+        const double c = (U(rng) - 0.5) * (ext - e), h = a == thin ? 0.0 : 0.5 * e * U(rng);
+        blo[k][a] = c - h;
+        bhi[k][a] = c + h;
+        lo[a][k] = std::nextafter((float)(blo[k][a] - eps), -INFINITY);
+        hi[a][k] = std::nextafter((float)(bhi[k][a] + eps), INFINITY);
+      }
+    }
+    const BVH4Q Q = quantize_node(N);
+    for (int r = 0; r < nrays; ++r) {
+      const int k = (int)(rng() & 3);
+      double p[3], o[3], d[3], t = 0;
+      for (int a = 0; a < 3; ++a) {
+        p[a] = blo[k][a] + (bhi[k][a] - blo[k][a]) * (rng() % 4 ? U(rng) : (double)(rng() & 1));
+        o[a] = (2 * U(rng) - 1) * (0.5 + far) * ext;
+        if (flat && rng() % 3 == 0) o[a] = p[a];
+      }
+      for (int a = 0; a < 3; ++a) t += (p[a] - o[a]) * (p[a] - o[a]);
+      t = std::sqrt(t);
+      if (!(t > 0)) continue;
+      for (int a = 0; a < 3; ++a) d[a] = (p[a] - o[a]) / t;
+      float ot[3], iv[3];
+      walk_ray(o, d, ot, iv);
+      for (const double hit : {FHUGE, t}) {
+        uint32_t key[4];
+        walk_keys(Q, ot, iv, walk_limit(hit), key);
+        if (key[k] == kNoEntry || (int)(key[k] & 3u) != k) ++bad;
+      }
+    }
+  }
+  return bad;
+}
+
+// Rays that are not numbers: with no axis left to bound a box, or behind a
+// hit at a distance that is not a number, the walk enters nothing, as one
+// that compares the slab's own ends does; with one such axis the others
+// decide.  Returns a bit mask.
+extern "C" int check_walk_nan(int n, unsigned seed) {
+  using namespace rg;
+  std::mt19937 rng(seed);
+  std::uniform_real_distribution<float> U(-1.0f, 1.0f);
+  const double bad_number = std::nan("");
+  int bad = 0;
+  for (int i = 0; i < n; ++i) {
+    BVH4Node N = {};
+    float* lo[3] = {N.lox, N.loy, N.loz};
+    float* hi[3] = {N.hix, N.hiy, N.hiz};
+    for (int k = 0; k < 4; ++k) {
+      N.child[k] = ~k;
+      for (int a = 0; a < 3; ++a) { lo[a][k] = U(rng); hi[a][k] = lo[a][k] + std::fabs(U(rng)); }
+    }
+    const BVH4Q Q = quantize_node(N);
+    double o[3] = {U(rng), U(rng), U(rng)}, d[3] = {U(rng), U(rng), U(rng)};
+    float ot[3], iv[3];
+    uint32_t key[4], was[4];
+    auto none = [&](const double* oo, const double* dd, double hit) {
+      walk_ray(oo, dd, ot, iv);
+      walk_keys(Q, ot, iv, walk_start(hit, ot), key);
+      for (uint32_t q : key)
+        if (q != kNoEntry) return false;
+      return true;
+    };
+    const double nan3[3] = {bad_number, bad_number, bad_number};
+    if (!none(o, nan3, FHUGE)) bad |= 1;
+    if (!none(nan3, d, FHUGE)) bad |= 2;
+    if (!none(o, d, bad_number)) bad |= 4;
+    walk_ray(o, d, ot, iv);
+    walk_keys(Q, ot, iv, walk_limit(bad_number), key);
+    for (uint32_t q : key)
+      if (q != kNoEntry) bad |= 8;
+    // one axis: as if every box filled it
+    const int ax = (int)(rng() % 3);
+    double one[3] = {o[0], o[1], o[2]};
+    one[ax] = bad_number;
+    walk_ray(one, d, ot, iv);
+    walk_keys(Q, ot, iv, walk_start(FHUGE, ot), key);
+    for (int k = 0; k < 4; ++k) { lo[ax][k] = -1e6f; hi[ax][k] = 1e6f; }
+    walk_ray(o, d, ot, iv);
+    walk_keys(quantize_node(N), ot, iv, walk_start(FHUGE, ot), was);
+    for (int k = 0; k < 4; ++k)
+      if ((key[k] == kNoEntry) != (was[k] == kNoEntry)) bad |= 16;
+  }
+  return bad;
+}

@@ -721,3 +721,38 @@ def test_tracked_modifiers_belong_to_the_call_and_the_scene(L):
     ctxs[0].set_params(p)
     for got, want in zip(L.contrib_batch(ctxs, sens, mods(names), 1, L.RT_IMM_IRRAD), single):
         assert np.array_equal(got.reshape(want.shape), want)
+
+
+def test_rays_that_are_not_numbers_meet_nothing_in_either_tree(L):
+    """A ray without a direction (or an origin) bounds no box: the four-wide
+    walk leaves it without a hit, as the binary walk does, and its neighbours
+    in the wavefront are not touched.  The scene's rings would take any
+    distance that is not a number for a hit."""
+    _say("rays that are not numbers")
+    text = ("void plastic grey 0 0 5 .5 .5 .5 0 0\nvoid glow lamp 0 0 4 3 2 1 0\nvoid glow sky 0 0 4 1 1 1 0\n"
+            "sky source up 0 0 4 0 0 1 180\n"
+            "grey polygon floor 0 0 12 -5 -5 -1 5 -5 -1 5 5 -1 -5 5 -1\n")
+    for i in range(64):
+        x, y = i % 8 - 3.5, i // 8 - 3.5
+        text += f"{'lamp' if i % 3 else 'grey'} ring r{i} 0 0 8 {x} {y} 1 0 0 -1 0 .3\n"
+    c = _ctx(L, text)
+    c.set_params(_rc_params(L, ambounce=0, seed=1))
+    rng = np.random.default_rng(8)
+    rays = np.hstack([rng.uniform(-4, 4, (300, 2)), np.zeros((300, 1)), rng.normal(size=(300, 3))])
+    got = {}
+    for k in ("good", "direction", "origin"):
+        r = rays.copy()
+        if k != "good":
+            r[::7, 3 if k == "direction" else 0:6 if k == "direction" else 3] = np.nan
+        res = []
+        for wide in (1, 0):
+            c.set_tuning(wide=wide)
+            res.append((c.trace(r, 0), c.last_nrays()))
+        c.set_tuning(wide=1)
+        assert np.array_equal(res[0][0], res[1][0], equal_nan=True) and res[0][1] == res[1][1], k
+        got[k] = res[0][0]
+    rest = np.arange(300) % 7 != 0
+    assert (got["good"] == [3, 2, 1]).all(axis=1).any()
+    for k in ("direction", "origin"):
+        assert np.array_equal(got[k][rest], got["good"][rest])
+        assert not (got[k][~rest] == [3, 2, 1]).all(axis=1).any()      # no ring

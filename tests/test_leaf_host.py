@@ -23,6 +23,9 @@ def leafcheck(tmp_path_factory):
     L.check_quantized.argtypes = [C.c_int, C.c_uint, C.c_int, C.c_double]
     L.check_leaf.argtypes = [C.c_int, C.c_int, C.c_uint, C.c_int, C.c_int, C.POINTER(C.c_long)]
     L.check_leaf.restype = C.c_long
+    L.check_walk_boxes.argtypes = [C.c_int, C.c_int, C.c_uint, C.c_double, C.c_double, C.c_int]
+    L.check_walk_boxes.restype = C.c_long
+    L.check_walk_nan.argtypes = [C.c_int, C.c_uint]
     L.check_order.argtypes = [C.c_int, C.c_int, C.c_uint, C.c_int, C.POINTER(C.c_long)]
     return L
 
@@ -44,3 +47,17 @@ def test_ties_are_ordered_as_a_walk_of_the_unrounded_boxes(leafcheck, n, grid):
     pairs = C.c_long()
     assert leafcheck.check_order(n, 200 if n > 100 else 200000, 23, grid, C.byref(pairs)) == 0
     assert pairs.value > 0
+
+
+@pytest.mark.parametrize("ext", [0.05, 6.0, 2000.0])
+@pytest.mark.parametrize("far,flat", [(0.0, 0), (0.0, 1), (8.0, 0), (8.0, 1)])
+def test_walk_enters_the_boxes_its_ray_meets(leafcheck, ext, far, flat):
+    """In FP32 (u = 2^-24) a plane's distance is off by at most u (4 |plane| +
+    4 |origin| + |plane - origin| + 3 node side + |plane - origin|) measured
+    along its axis: u (12 ext / 2 + 6 (far + 1/2) ext) = 3.4e-6 ext at far = 8,
+    inside the 4e-6 ext + 1e-5 that boxes are widened by."""
+    assert leafcheck.check_walk_boxes(2000, 200, 31, ext, far, flat) == 0
+
+
+def test_walk_enters_nothing_for_rays_that_are_not_numbers(leafcheck):
+    assert leafcheck.check_walk_nan(20000, 37) == 0
