@@ -7,7 +7,6 @@
 #include "rg_bvh.hpp"
 
 #include <algorithm>
-#include <cmath>
 #include <atomic>
 #include <cstdlib>
 #include <cstring>
@@ -288,54 +287,6 @@ int collapse_bvh4(const std::vector<BVHNode>& nodes, int32_t root, std::vector<B
     }
   }
   return dmax;
-}
-
-BVH4Q quantize_node(const BVH4Node& n) {
-  BVH4Q q = {};
-  const float* lo[3] = {n.lox, n.loy, n.loz};
-  const float* hi[3] = {n.hix, n.hiy, n.hiz};
-  uint32_t* ql[3] = {&q.lox, &q.loy, &q.loz};
-  uint32_t* qh[3] = {&q.hix, &q.hiy, &q.hiz};
-  for (int k = 0; k < 4; ++k) q.child[k] = n.child[k];
-  for (int a = 0; a < 3; ++a) {
-    float mn = INFINITY, mx = -INFINITY;
-    for (int k = 0; k < 4; ++k)
-      if (n.child[k] != INT32_MIN) { mn = std::min(mn, lo[a][k]); mx = std::max(mx, hi[a][k]); }
-    if (!(mn <= mx)) mn = mx = 0.f;
-    const double org = mn;
-    float sc = (float)(((double)mx - org) / 255.0);
-    if (!(sc > 1e-20f)) sc = 1e-20f;
-    while (org + 255.0 * (double)sc < (double)mx) sc = std::nextafter(sc, INFINITY);
-    const double s = sc;
-    q.org[a] = mn;
-    q.scale[a] = sc;
-    for (int k = 0; k < 4; ++k) {
-      int l = 255, h = 0;         // an unused slot: no box
-      if (n.child[k] != INT32_MIN) {
-        l = (int)std::min(std::max(std::floor(((double)lo[a][k] - org) / s), 0.0), 255.0);
-        while (l > 0 && org + l * s > (double)lo[a][k]) --l;
-        h = (int)std::min(std::max(std::ceil(((double)hi[a][k] - org) / s), 0.0), 255.0);
-        while (h < 255 && org + h * s < (double)hi[a][k]) ++h;
-      }
-      *ql[a] |= (uint32_t)l << (8 * k);
-      *qh[a] |= (uint32_t)h << (8 * k);
-    }
-  }
-  return q;
-}
-
-void quantize_bvh4(const std::vector<BVH4Node>& in, std::vector<BVH4Q>& out) {
-  out.resize(in.size());
-  const size_t per = 1 << 14;
-  const unsigned nthr = (unsigned)std::min<size_t>({(in.size() + per - 1) / per, 16,
-                                                    std::max(1u, std::thread::hardware_concurrency())});
-  auto part = [&](unsigned t) {
-    for (size_t i = in.size() * t / nthr, e = in.size() * (t + 1) / nthr; i < e; ++i) out[i] = quantize_node(in[i]);
-  };
-  std::vector<std::thread> pool;
-  for (unsigned t = 1; t < nthr; ++t) pool.emplace_back(part, t);
-  if (nthr) part(0);
-  for (auto& th : pool) th.join();
 }
 
 std::vector<int32_t> leaf_positions(const std::vector<BVHNode>& nodes, int32_t root, size_t nprims) {

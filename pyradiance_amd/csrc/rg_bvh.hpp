@@ -28,12 +28,6 @@ int32_t build_sah_bvh(const float* lo, const float* hi, const int32_t* ids, uint
 // four-wide nodes on a path from `root` to a leaf.
 int collapse_bvh4(const std::vector<BVHNode>& nodes, int32_t root, std::vector<BVH4Node>& out);
 
-// The 64-byte form of four-wide nodes: planes rounded outward to steps of
-// 1/255 of the node's extent, evaluated in double so that org + q * scale
-// never lies inside the plane it stands for.
-BVH4Q quantize_node(const BVH4Node& n);
-void quantize_bvh4(const std::vector<BVH4Node>& in, std::vector<BVH4Q>& out);
-
 // Position of every primitive among the leaves of a host SAH tree, left to
 // right (-1: not in it).
 std::vector<int32_t> leaf_positions(const std::vector<BVHNode>& nodes, int32_t root, size_t nprims);

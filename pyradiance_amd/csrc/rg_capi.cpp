@@ -290,7 +290,6 @@ int rg_scene_commit(rg_ctx* c) {
     // three per four-wide node) fit the traversal stack
     std::vector<BVHNode> hn;
     std::vector<BVH4Node> h4;
-    std::vector<BVH4Q> h4q;
     std::vector<int32_t> lpos;
     int root = -1;
     bool wide = false;
@@ -298,12 +297,11 @@ int rg_scene_commit(rg_ctx* c) {
       root = build_sah_bvh(slo_v.data(), shi_v.data(), small_ids.data(), n, hn, kMaxTreeDepth);
       const int d4 = collapse_bvh4(hn, root, h4);
       wide = root == 0 && !h4.empty() && 3 * d4 <= kTraceStackEntries;   // both walks start at node 0
-      if (wide) {
-        quantize_bvh4(h4, h4q);
-        lpos = leaf_positions(hn, root, cs.prims.size());
-      }
+      if (wide) lpos = leaf_positions(hn, root, cs.prims.size());
     }
-    // every table in one device block, sent in one copy
+    // every table in one device block, sent in one copy.  The last part is
+    // the four-wide tree as built: the device rounds its nodes into their
+    // place, then writes the leaf records over it.
     Pack pk;
     const size_t o_prims = pk.add(cs.prims), o_geom = pk.add(cs.geom), o_mats = pk.add(cs.mats),
                  o_srcs = pk.add(cs.srcs), o_scache = pk.add(cs.scache),
@@ -313,9 +311,12 @@ int rg_scene_commit(rg_ctx* c) {
                  o_nodes = pk.add(hn.data(), sizeof(BVHNode) * hn.size(), sizeof(BVHNode) * std::max<uint32_t>(n, 1)),
                  o_leaf = pk.add(sah ? small_ids.data() : nullptr, sah ? sizeof(int32_t) * n : 0,
                                  sizeof(int32_t) * std::max<uint32_t>(n, 1)),
-                 o_nodes4 = wide ? pk.add(h4q) : 0, o_lpos = wide ? pk.add(lpos) : 0, o_blo = sah ? 0 : pk.add(slo_v), o_bhi = sah ? 0 : pk.add(shi_v),
+                 o_lpos = wide ? pk.add(lpos) : 0,
+                 o_blo = sah ? 0 : pk.add(slo_v), o_bhi = sah ? 0 : pk.add(shi_v),
                  o_bids = sah ? 0 : pk.add(small_ids);
-    char* blob = (char*)c->scene_mem.get("blob", pk.total, c->st, false);
+    const size_t o_leafs = wide ? pk.add(h4) : 0,
+                 o_nodes4 = (std::max(pk.total, o_leafs + (wide ? sizeof(LeafRec) * cs.prims.size() : 0)) + 255) & ~(size_t)255;
+    char* blob = (char*)c->scene_mem.get("blob", o_nodes4 + (wide ? sizeof(BVH4Q) * h4.size() : 0), c->st, false);
     pk.send(c, blob);
     S.prims = to_global((const Prim*)(blob + o_prims));
     S.geom = to_global((const double*)(blob + o_geom));
@@ -341,7 +342,8 @@ int rg_scene_commit(rg_ctx* c) {
     S.leaf_prim = to_global(leaf);
     S.leafs = nullptr;
     if (wide) {
-      LeafRec* recs = (LeafRec*)c->scene_mem.get("leafs", sizeof(LeafRec) * cs.prims.size(), c->st, false);
+      LeafRec* recs = (LeafRec*)(blob + o_leafs);
+      round_nodes((const BVH4Node*)recs, (BVH4Q*)(blob + o_nodes4), (uint32_t)h4.size(), c->st);
       leaf_records(S, (const int32_t*)(blob + o_lpos), recs, c->st);
       S.leafs = to_global((const LeafRec*)recs);
     }

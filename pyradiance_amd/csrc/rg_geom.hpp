@@ -41,6 +41,49 @@ struct alignas(16) BVH4Q {
 };
 static_assert(sizeof(BVH4Q) == 64, "one node, half a cache line");
 
+// The 64-byte form of a four-wide node: planes rounded outward to steps of
+// 1/255 of the node's extent, evaluated in double (the products are exact) so
+// that org + q * scale never lies inside the plane it stands for.
+RG_HD BVH4Q quantize_node(const BVH4Node& n) {
+  BVH4Q q = {};
+  const float* lo[3] = {n.lox, n.loy, n.loz};
+  const float* hi[3] = {n.hix, n.hiy, n.hiz};
+  uint32_t ql[3] = {0, 0, 0}, qh[3] = {0, 0, 0};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) q.child[k] = n.child[k];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    float mn = INFINITY, mx = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (n.child[k] != INT32_MIN) { mn = fminf(mn, lo[a][k]); mx = fmaxf(mx, hi[a][k]); }
+    if (!(mn <= mx)) mn = mx = 0.f;
+    const double org = mn;
+    float sc = (float)(((double)mx - org) / 255.0);
+    if (!(sc > 1e-20f)) sc = 1e-20f;
+    while (org + 255.0 * (double)sc < (double)mx) sc = nextafterf(sc, INFINITY);
+    const double s = sc;
+    q.org[a] = mn;
+    q.scale[a] = sc;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      int l = 255, h = 0;         // an unused slot: no box
+      if (n.child[k] != INT32_MIN) {
+        l = (int)fmin(fmax(floor(((double)lo[a][k] - org) / s), 0.0), 255.0);
+        while (l > 0 && org + l * s > (double)lo[a][k]) --l;
+        h = (int)fmin(fmax(ceil(((double)hi[a][k] - org) / s), 0.0), 255.0);
+        while (h < 255 && org + h * s < (double)hi[a][k]) ++h;
+      }
+      ql[a] |= (uint32_t)l << (8 * k);
+      qh[a] |= (uint32_t)h << (8 * k);
+    }
+  }
+  q.lox = ql[0]; q.hix = qh[0];
+  q.loy = ql[1]; q.hiy = qh[1];
+  q.loz = ql[2]; q.hiz = qh[2];
+  return q;
+}
+
 // Whether and where a ray enters the four rounded boxes of a node: key[k] is
 // the entry distance as an integer with the child's slot k in the low two
 // bits, or kNoEntry.  ot: origin times inverse direction, iv: inverse

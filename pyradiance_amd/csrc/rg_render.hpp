@@ -99,8 +99,11 @@ struct Tuning {
 void render(const DevScene& S, RunCfg cfg, const double* d_rays, uint32_t nsens, bool imm_irrad, int max_srcs,
             const Tuning& tn, DevArena& arena, hipStream_t st, RenderStats* stats);
 
-// Leaf records of all primitives of a scene (LeafRec); d_pos: their places
-// among the tree's leaves.
+// The walk's form of a scene on the device: n four-wide nodes rounded to 64
+// bytes, and the leaf records of all primitives (LeafRec; d_pos: their places
+// among the tree's leaves).  The records may overwrite the nodes they were
+// rounded from.
+void round_nodes(const BVH4Node* d_in, BVH4Q* d_out, uint32_t n, hipStream_t st);
 void leaf_records(const DevScene& S, const int32_t* d_pos, LeafRec* d_out, hipStream_t st);
 
 // First intersection of n rays (n x 6 doubles): distance (FHUGE on a miss),

@@ -453,10 +453,16 @@ CompiledScene compile_scene(const SceneDB& db) {
   }
   std::vector<int> obj_prim(nobj, -1);
   std::vector<std::array<double, 6>> dbounds;
-  auto mod_id = [&](const std::string& name) {
-    auto it = cs.mod_index.emplace(name, (int32_t)cs.mod_names.size());
-    if (it.second) cs.mod_names.push_back(name);
-    return it.first->second;
+  std::vector<int32_t> obj_modid(nobj, -1);     // as mod_id(), once per modifier object
+  auto mod_id = [&](int om) {
+    int32_t& id = obj_modid[om];
+    if (id < 0) {
+      const std::string& name = objs[om].name;
+      auto it = cs.mod_index.emplace(name, (int32_t)cs.mod_names.size());
+      if (it.second) cs.mod_names.push_back(name);
+      id = it.first->second;
+    }
+    return id;
   };
   // One surface object -> one primitive (-1 if degenerate).  mo: material
   // object, omod: modifier that ranks coincident hits and names the
@@ -466,7 +472,7 @@ CompiledScene compile_scene(const SceneDB& db) {
     memset(&P, 0, sizeof P);
     P.mat = material_index(mo);
     P.omod = omod;
-    P.mod = mod_id(objs[omod].name);
+    P.mod = mod_id(omod);
     P.srcidx = -1;
     P.goff = (int)cs.geom.size();
     P.nv = 0;
@@ -647,7 +653,7 @@ CompiledScene compile_scene(const SceneDB& db) {
       P.kind = PK_TRIANGLE;
       P.mat = material_index(mo);
       P.omod = mod;
-      P.mod = mod_id(objs[mod].name);
+      P.mod = mod_id(mod);
       P.srcidx = -1;
       P.goff = (int)cs.geom.size();
       P.nv = 3;
@@ -789,7 +795,7 @@ CompiledScene compile_scene(const SceneDB& db) {
     S.prim = -1;
     S.mat = material_index(mo);
     S.objmod = o.omod;
-    S.mod = mod_id(objs[o.omod].name);
+    S.mod = mod_id(o.omod);
     const auto& f = o.fargs;
     auto setflatss = [&]() {
       double u[3];

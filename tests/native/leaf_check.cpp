@@ -31,13 +31,10 @@ extern "C" int check_quantized(int n, unsigned seed, int nused, double far) {
     for (int k = 0; k < 4; ++k) N.child[k] = k < nused ? (int)(rng() & 0xffff) - 0x7fff : INT32_MIN;
     for (int& p : N.pad) p = 0;
   }
-  std::vector<rg::BVH4Q> out;
-  rg::quantize_bvh4(in, out);
-  if (out.size() != in.size()) return 1;
   int bad = 0;
   for (size_t i = 0; i < in.size(); ++i) {
     const rg::BVH4Node& N = in[i];
-    const rg::BVH4Q& Q = out[i];
+    const rg::BVH4Q Q = rg::quantize_node(N);
     const float* lo[3] = {N.lox, N.loy, N.loz};
     const float* hi[3] = {N.hix, N.hiy, N.hiz};
     const uint32_t ql[3] = {Q.lox, Q.loy, Q.loz}, qh[3] = {Q.hix, Q.hiy, Q.hiz};
