@@ -45,10 +45,18 @@ HBM_PEAK_GBS = 8000.0          # MI355X HBM3E
 BF16_PEAK_TFLOPS = 2500.0      # MI355X dense BF16 MFMA
 
 # Algorithmic bytes per ray segment: ray record in + hit out (48 B), one node
-# per BVH node visited (64 B, as the renderer reports), one 128-byte
-# primitive record per primitive tested, one 32-byte path-state
-# read-modify-write.
-B_RAY, B_NODE, B_PRIM, B_STATE = 48.0, 64.0, 128.0, 32.0
+# per BVH node visited (64 B, as the renderer reports), per primitive tested
+# 112 bytes of its leaf record in the four-wide walk and a 48-byte record
+# elsewhere (the binary walks, and the room-sized primitives ahead of the
+# four-wide one), one 32-byte path-state read-modify-write.
+B_RAY, B_NODE, B_LEAF, B_PRIM, B_STATE = 48.0, 64.0, 112.0, 48.0, 32.0
+
+
+def bytes_per_ray(st):
+    """Those bytes for the counts of last_stats() at profiling level 2."""
+    leaf = st["prims"] - st["big_prims"] if st["wide"] else 0.0
+    rest = st["prims"] - leaf
+    return B_RAY + ((st["node_bytes"] or B_NODE) * st["nodes"] + B_LEAF * leaf + B_PRIM * rest) / st["rays"] + B_STATE
 
 
 def log(*a):
@@ -636,7 +644,7 @@ def config5_bench(seed: int = 0):
                         "10-storey office, then DC x sky 20000x2306x8760",
             "primitives": int(info["primitives"]), "sensors": int(len(sens)), "scene_generate_s": t_gen,
             "scene_commit_s": t_commit, "rays": int(rays), "trace_s": t_trace, "Mrays_per_s": rays / t_trace / 1e6,
-            "rays_per_sensor": rays / len(sens), "walk": "wide" if info["primitives"] <= (4 << 20) else "binary",
+            "rays_per_sensor": rays / len(sens), "walk": "wide" if st["wide"] else "binary",
             "dcsky_s": t_dc, "dcsky_output_finite": finite,
             "dc_nonzero_fraction": float((A > 0).mean())}
 
@@ -953,8 +961,7 @@ def main():
     st_c = ctx.last_stats()
     ctx.set_profiling(0)
     nr = st_c["rays"]
-    b_node = st_c.get("node_bytes") or B_NODE
-    per_ray = B_RAY + b_node * st_c["nodes"] / nr + B_PRIM * st_c["prims"] / nr + B_STATE
+    per_ray = bytes_per_ray(st_c)
     avg_launch_ms = st_t["trace_ms"] / max(st_t["launches"], 1)
     bytes_per_launch = per_ray * st_t["rays"] / max(st_t["launches"], 1)
     achieved = bytes_per_launch / (avg_launch_ms * 1e-3) / 1e9
@@ -1019,7 +1026,7 @@ def main():
     bvh_name = args.bvh if args.bvh != "auto" else ("sah" if info["primitives"] <= (4 << 20) else "lbvh")
     if scene_tuned:
         bvh_name = "sah" if scene_tuned["best"]["builder"] == _lib.BVH_SAH else "lbvh"
-    walk = "wide" if bvh_name == "sah" else "binary"
+    walk = "wide" if st_c["wide"] else "binary"
     traffic_ray = committed_traffic(bvh_name, walk)
     # HBM bytes per launch = measured bytes per ray x rays per launch of this run
     traffic = traffic_ray * st_t["rays"] / max(st_t["launches"], 1) if traffic_ray else None
@@ -1059,7 +1066,7 @@ def main():
                      "trace_kernel_ms_per_step": st_t["trace_ms"] / nsteps,
                      "launches_timed": int(st_t["launches"]),
                      "bytes_per_ray": per_ray, "nodes_per_ray": st_c["nodes"] / nr, "walk": walk,
-                     "prims_per_ray": st_c["prims"] / nr},
+                     "prims_per_ray": st_c["prims"] / nr, "big_prims_per_ray": st_c["big_prims"] / nr},
         "dcsky": dcs,
         "dcsky_config5": dc5,
         "config5": c5,

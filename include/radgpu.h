@@ -198,10 +198,12 @@ int rg_set_tuning(rg_ctx *ctx, const char *key, long long value);
 #define RG_BVH_SAH 1
 #define RG_BVH_LBVH 2
 int rg_set_bvh_builder(rg_ctx *ctx, int kind);
-/* out[0..8] = rays, generation launches, threads launched, summed traversal-
+/* out[0..10] = rays, generation launches, threads launched, summed traversal-
  * kernel milliseconds, nodes visited, primitives tested, batches, summed
- * shading-kernel milliseconds, bytes per node visited (64 in
- * either tree) */
+ * shading-kernel milliseconds, bytes per node visited (64 in either tree),
+ * the four-wide tree was walked (1) or the binary one (0; also with no rays),
+ * primitives tested ahead of the four-wide walk (among those of out[5]; the
+ * counts are taken at profiling level 2).  n: entries wanted. */
 int rg_last_stats(rg_ctx *ctx, double *out, int n);
 
 /* DC x sky product, replaces cm_multiply() (util/cmatrix.c:421-474):

@@ -38,7 +38,7 @@ struct rg_ctx {
   Tuning tuning;
   int profile = 0;              // 0 off, 1 time k_bounce launches, 2 also count visits
   RenderStats last_stats;
-  unsigned long long last_visits[2] = {0, 0};
+  unsigned long long last_visits[3] = {0, 0, 0};
   // shadow cache: filled at the first call after a commit (the reference
   // fills a source's cache at its first shadow test in the process); the
   // cast rays of a source count once, in the call that first tests it
@@ -562,7 +562,7 @@ static void run(rg_ctx* c, const double* rays, long long nrays, int accum, int f
   cfg.visits = nullptr;
   unsigned long long* d_vis = nullptr;
   if (c->profile >= 2) {
-    d_vis = (unsigned long long*)c->arena.get("visits", 16, c->st, true);
+    d_vis = (unsigned long long*)c->arena.get("visits", sizeof c->last_visits, c->st, true);
     cfg.visits = d_vis;
   }
   c->last_stats = RenderStats();
@@ -581,8 +581,8 @@ static void run(rg_ctx* c, const double* rays, long long nrays, int accum, int f
     render(Sd, cfg, d_rays, (uint32_t)nrays, (flags & 8) != 0, max_srcs, tn, render_arena(c->device), c->st,
            &c->last_stats);
   }
-  if (d_vis) hipck(hipMemcpyAsync(c->last_visits, d_vis, 16, hipMemcpyDeviceToHost, c->st), "visits");
-  else c->last_visits[0] = c->last_visits[1] = 0;
+  if (d_vis) hipck(hipMemcpyAsync(c->last_visits, d_vis, sizeof c->last_visits, hipMemcpyDeviceToHost, c->st), "visits");
+  else memset(c->last_visits, 0, sizeof c->last_visits);
   if (cfg.fix > 0.0 && outn)
     k_fixed_out<<<(unsigned)((outn + 255) / 256), 256, 0, c->st>>>(d_out, outn, 1.0 / cfg.fix);
   // one read-back of the call block (and of staged records)
@@ -959,10 +959,12 @@ int rg_set_profiling(rg_ctx* c, int level) {
 
 int rg_last_stats(rg_ctx* c, double* out, int n) {
   RG_TRY(c, {
-    double v[9] = {(double)c->last_nrays, (double)c->last_stats.launches, (double)c->last_stats.threads,
+    static_assert(sizeof(BVHNode) == sizeof(BVH4Q), "one size of node");
+    double v[11] = {(double)c->last_nrays, (double)c->last_stats.launches, (double)c->last_stats.threads,
                    c->last_stats.bounce_ms, (double)c->last_visits[0], (double)c->last_visits[1],
-                   (double)c->last_stats.generations, c->last_stats.shade_ms, (double)c->last_stats.node_bytes};
-    for (int i = 0; i < n && i < 9; ++i) out[i] = v[i];
+                   (double)c->last_stats.generations, c->last_stats.shade_ms, (double)sizeof(BVHNode),
+                   c->last_stats.wide ? 1.0 : 0.0, (double)c->last_visits[2]};
+    for (int i = 0; i < n && i < 11; ++i) out[i] = v[i];
   });
 }
 

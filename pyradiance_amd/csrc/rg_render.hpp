@@ -72,7 +72,7 @@ struct RenderStats {
   bool timing = false;       // time every generation's kernels with HIP events
   double bounce_ms = 0;      // summed traversal-kernel (k_trace) durations
   double shade_ms = 0;       // summed shading-kernel (k_shade) durations
-  int node_bytes = 64;       // bytes of one tree node the traversal fetched
+  bool wide = false;         // the four-wide tree was walked, not the binary one
 };
 
 // Per-lane traversal stack entries (LDS and private memory together).

@@ -756,3 +756,28 @@ def test_rays_that_are_not_numbers_meet_nothing_in_either_tree(L):
     for k in ("direction", "origin"):
         assert np.array_equal(got[k][rest], got["good"][rest])
         assert not (got[k][~rest] == [3, 2, 1]).all(axis=1).any()      # no ring
+
+
+def test_stats_tell_the_tree_that_was_walked(L):
+    """last_stats() names the walk that ran, not the one a builder's trees
+    usually take, and counts the room-sized primitives tested ahead of the
+    four-wide walk apart from its leaves; the binary walks test both in one."""
+    _say("the tree of last_stats()")
+    room = scenes.Room()
+    rad = scenes.room_rad(room) + scenes.furniture_rad(np.random.default_rng(2), 2, room) + scenes.sky_rad((1, 1, 1))
+    sens = scenes.config1(0)[1]
+    res = {}
+    for name, builder, shape in [("wide", L.BVH_SAH, {}), ("asked for binary", L.BVH_SAH, dict(wide=0)),
+                                 ("per thread", L.BVH_SAH, dict(trace_kernel=0)), ("lbvh", L.BVH_LBVH, {})]:
+        c = _ctx(L, rad, builder)
+        c.set_params(_rc_params(L, ambounce=0, seed=1))
+        c.set_tuning(**shape)
+        c.set_profiling(2)
+        c.trace(sens, 0)
+        res[name] = c.last_stats()
+        c.trace(sens[:0], 0)
+        assert not c.last_stats()["wide"] and not c.last_stats()["prims"]
+        c.close()
+    for name, st in res.items():
+        assert st["wide"] == (name == "wide") and st["prims"] > 0 and st["node_bytes"] == 64
+        assert 0 < st["big_prims"] < st["prims"] if st["wide"] else st["big_prims"] == 0
