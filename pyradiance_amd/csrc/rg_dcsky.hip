@@ -74,6 +74,14 @@ __global__ void __launch_bounds__(256) k_split(const float* A, const float* B, i
   }
 }
 
+// Between writes of a wavefront's own LDS and reads of it by its other lanes:
+// a wavefront's LDS instructions complete in order, so only the compiler has
+// to keep them so (no instruction).
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 constexpr int DB = 256;        // 4 wavefronts, 2 (m) x 2 (n)
 #ifndef RG_DCSKY_WB
 #define RG_DCSKY_WB 4          // 16-column tiles per wavefront along n
@@ -251,7 +259,7 @@ __global__ void __launch_bounds__(256) k_split_tiled(const float* A, const float
     const int k = i / 48, q = i % 48;
     tl[isb ? (q / 3) * TROW + 3 * k + q % 3 : (i / 96) * TROW + i % 96] = x[j];
   }
-  __builtin_amdgcn_wave_barrier();            // one wavefront's own LDS, in order
+  wave_lds_order();
   const int row = rg * 16 + (lane >> 2), part = lane & 3;
   const float* mine = tl + (lane >> 2) * TROW + part * 24;
   unsigned short* H = isb ? Bh : Ah;
@@ -545,7 +553,7 @@ k_dcsky_short(const unsigned short* Ah, const unsigned short* Al, const unsigned
       t4[0] = make_float4(r[0], g[0], u[0], r[1]);
       t4[1] = make_float4(g[1], u[1], r[2], g[2]);
       t4[2] = make_float4(u[2], r[3], g[3], u[3]);
-      __builtin_amdgcn_wave_barrier();
+      wave_lds_order();
       const int f0 = (ch * SCOLS + 16 * b) * 3;
 #pragma unroll
       for (int i = 0; i < NST; ++i) {
@@ -558,7 +566,7 @@ k_dcsky_short(const unsigned short* Ah, const unsigned short* Al, const unsigned
         if (VEC) *(float4*)dst = *(const float4*)(tw + row * SOUT + f);
         else *dst = tw[row * SOUT + f];
       }
-      __builtin_amdgcn_wave_barrier();
+      wave_lds_order();
     }
     // the next chunk's loads (issued before these stores) done, every LDS
     // read of this one too
