@@ -436,22 +436,29 @@ static int ring_parts(long long tiles, int nk) {
 // 16 rows of A (hi and lo, all K, three channels: 120 registers at K = 160)
 // for the whole launch.  A block of 8 wavefronts owns a slab of 128 rows of A
 // and walks a range of sky columns in chunks of 32: each chunk's B planes
-// (hi/lo, three channels, all K) are loaded straight into LDS, double-
-// buffered (the next chunk's loads are under way during this chunk's MFMAs).  No K loop over global
-// memory, one barrier per chunk.
+// (hi/lo, three channels, all K) are loaded straight into LDS, into the buffer
+// that the chunk before does not use.  No K loop over global memory, one
+// barrier per chunk.
 //
 // Outputs go through LDS: a lane ends up with 12 consecutive floats of a row,
 // and storing those as they are writes 16 bytes every 48, three times as many
 // partial lines as the rows have.  Turned in LDS, a store instruction covers
 // runs of 192 bytes.  2500 x 146 x 8760: 88 us (104 with 48-byte runs and the
 // chunk staged through registers), 3.0 of the 6.9 TB/s that a plain fill
-// reaches; what is left is the wait for a chunk's loads, which complete in
-// order behind the stores of the chunk before, and LDS reads (61 KB per
-// wavefront and chunk).  Four wavefronts of 32 rows halve those and lose
+// reaches; what is left is the wait for the next chunk's loads, which complete
+// in order behind the stores of the chunk before (the compiler does not tell
+// the two buffers apart and waits for them ahead of this chunk's first LDS
+// read, so they overlap nothing), and LDS reads (61 KB per wavefront and
+// chunk).  Four wavefronts of 32 rows halve those and lose
 // more: one wavefront per SIMD, 106 us.
-// Every lane issues the same loads and stores in every chunk (pieces past
-// the chunk load a valid piece again; outputs outside C go to `sink`), so the
-// wait for the next chunk's loads never waits for this chunk's stores.
+// The code's own wait for those loads does not rely on that one.  With 16-byte
+// stores it stands ahead of the chunk's outputs, where nothing has to be
+// counted.  With 4-byte ones it would keep their addresses from being formed
+// beside the MFMAs there (2500 x 146 x 8759: 164 us, 139 behind them), so it
+// stands behind them and takes exactly 2 NST of them to be under way: each is
+// an instruction of its own in the source, and every lane issues all of them
+// in every chunk (pieces past the chunk load a valid piece again; outputs
+// outside C go to `sink`).
 constexpr int SW = 8;                  // wavefronts per block
 constexpr int SROWS = 16 * SW;         // rows of A per block (a slab)
 constexpr int SCOLS = 32;              // sky columns per staged chunk
@@ -543,6 +550,7 @@ k_dcsky_short(const unsigned short* Ah, const unsigned short* Al, const unsigned
             acc[b][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[b][c][p == 1], p == 2 ? al[c][s] : ah[c][s],
                                                                 acc[b][c], 0, 0, 0);
     }
+    if (VEC) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the next chunk's loads done
     // D layout: lane holds D[n = 4 * (lane >> 4) + i][m = lane & 15], 12
     // consecutive floats of row m; turned through this wavefront's own LDS
     const int m0 = slab * SROWS + wave * 16;
@@ -564,13 +572,13 @@ k_dcsky_short(const unsigned short* Ah, const unsigned short* Al, const unsigned
         const bool in = m0 + row < M && f0 + f < 3 * N;
         float* dst = in ? C + (size_t)(m0 + row) * N * 3 + f0 + f : mysink;
         if (VEC) *(float4*)dst = *(const float4*)(tw + row * SOUT + f);
-        else *dst = tw[row * SOUT + f];
+        else asm volatile("global_store_dword %0, %1, off" :: "v"(dst), "v"(tw[row * SOUT + f]) : "memory");
       }
       wave_lds_order();
     }
-    // the next chunk's loads (issued before these stores) done, every LDS
-    // read of this one too
-    ring_wait<2 * NST>();
+    // every LDS read of this chunk done, and the next one's loads (issued
+    // before these stores)
+    ring_wait<VEC ? 63 : 2 * NST>();
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
