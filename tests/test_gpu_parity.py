@@ -613,10 +613,10 @@ def test_path_records_follow_their_rays_through_every_window(L):
 
 
 @pytest.mark.parametrize("m,k,n", [(1, 257, 1), (127, 288, 129), (128, 289, 128), (129, 320, 127), (300, 2306, 4),
-                                   (33, 384, 1157), (2049, 352, 2051), (1500, 578, 1408)])
+                                   (33, 384, 1157), (130, 161, 260), (2049, 352, 2051), (1500, 578, 1408)])
 def test_long_k_product_at_tile_and_split_edges(L, m, k, n):
-    """The ring form of the K > 256 product: tile remainders in both
-    directions, K steps that do and do not fill a group of four, K shared by
+    """The ring form of the K > 160 product (mode 3, whatever the size would
+    choose): tile remainders in both directions, K steps that do and do not fill a group of four, K shared by
     many blocks and by one, sky columns that do and do not allow 16-byte
     stores.  Operands are positive, so every term's relative error bounds the
     sum's: the dropped lo x lo part and the rounding of lo are each at most
@@ -629,7 +629,7 @@ def test_long_k_product_at_tile_and_split_edges(L, m, k, n):
     b = torch.exp(torch.randn((k, n, 3), generator=g, device="cuda"))
     c = torch.full((m, n, 3), float("nan"), device="cuda")
     torch.cuda.synchronize()
-    L.dcsky_device(a.data_ptr(), b.data_ptr(), c.data_ptr(), m, k, n)
+    L.dcsky_device(a.data_ptr(), b.data_ptr(), c.data_ptr(), m, k, n, 3)
     for ch in range(3):
         ref = a[:, :, ch].double().contiguous() @ b[:, :, ch].double().contiguous()
         rel = ((c[:, :, ch].double() - ref) / ref).abs().max().item()
@@ -637,12 +637,16 @@ def test_long_k_product_at_tile_and_split_edges(L, m, k, n):
 
 
 @pytest.mark.parametrize("m,k,n", [(1, 1, 1), (15, 32, 33), (16, 33, 31), (127, 64, 2048), (129, 65, 130), (128, 146, 128),
-                                   (257, 160, 1001), (2500, 146, 97), (40, 161, 36)])
+                                   (257, 160, 1001), (2500, 146, 97), (130, 20, 8192), (130, 64, 8196),
+                                   (257, 96, 6148), (200, 128, 8196), (300, 146, 8196), (2500, 146, 1000),
+                                   (129, 100, 8193), (129, 160, 8191)])
 def test_short_k_product_at_chunk_and_slab_edges(L, m, k, n):
-    """The short-K form: rows that do and do not fill a wavefront's 16 or a
-    slab's 128, sky columns around the 32-column chunks and not a multiple of
-    four, every number of K steps, and the first K that leaves the form.  The
-    bound is the long-K test's."""
+    """The short-K form (mode 4, whatever the size would choose): rows that do
+    and do not fill a wavefront's 16 or a slab's 128, sky columns around the
+    32-column chunks, one and several chunks to a block, and every number of
+    K steps with columns that do and do not allow 16-byte stores (which wait
+    for the next chunk's loads in different places).  The bound is the long-K
+    test's."""
     import torch
     _say(f"short-K product {m} x {k} x {n}")
     g = torch.Generator(device="cuda").manual_seed(m + k + n)
@@ -650,7 +654,7 @@ def test_short_k_product_at_chunk_and_slab_edges(L, m, k, n):
     b = torch.exp(torch.randn((k, n, 3), generator=g, device="cuda"))
     c = torch.full((m + 1, n, 3), -1.0, device="cuda")
     torch.cuda.synchronize()
-    L.dcsky_device(a.data_ptr(), b.data_ptr(), c.data_ptr(), m, k, n)
+    L.dcsky_device(a.data_ptr(), b.data_ptr(), c.data_ptr(), m, k, n, 4)
     assert (c[m] == -1.0).all()                    # nothing past the last row
     for ch in range(3):
         ref = a[:, :, ch].double().contiguous() @ b[:, :, ch].double().contiguous()
@@ -659,13 +663,16 @@ def test_short_k_product_at_chunk_and_slab_edges(L, m, k, n):
 
 
 @pytest.mark.parametrize("m,k,n", [(1, 1, 1), (67, 41, 5), (3, 15, 300), (4, 16, 255), (4, 1024, 1024), (5, 1025, 30),
-                                   (9, 146, 8760), (101, 289, 257), (14000, 578, 1), (63, 513, 256)])
+                                   (9, 146, 8760), (101, 289, 257), (14000, 578, 1), (63, 513, 256),
+                                   (4, 1024, 1025), (128, 257, 255), (129, 257, 255), (3, 1024, 2730),
+                                   (3, 1024, 2731), (4, 1024, 4096), (4, 1024, 4097), (1200, 146, 96)])
 def test_small_product_against_fp64(L, m, k, n):
     """The one-launch form: fewer K than wavefronts, row groups cut short,
-    columns that end inside a block, either side of its lines (K 1024, 256
-    columns, 2^22 and 2^24 multiply-adds).  FP32 sums of positive terms:
-    K 2^-24 relative; the split forms past the line add the long-K test's
-    bound."""
+    columns that end inside a block, either side of its lines (K 1024; 2^22
+    multiply-adds, where rows are grouped; 2^23 with fewer than 256 columns or
+    4 rows; 2^24 with more), past which the product is the split form's bit
+    for bit.  FP32 sums of positive terms: K 2^-24 relative; the split forms
+    add the long-K test's bound."""
     import torch
     _say(f"small product {m} x {k} x {n}")
     g = torch.Generator(device="cuda").manual_seed(m + k + n)
@@ -675,7 +682,11 @@ def test_small_product_against_fp64(L, m, k, n):
     torch.cuda.synchronize()
     L.dcsky_device(a.data_ptr(), b.data_ptr(), c.data_ptr(), m, k, n)
     assert (c[m] == -1.0).all()
-    split = k > 1024
+    split = k > 1024 or m * k * n > (1 << 24 if n >= 256 and m >= 4 else 1 << 23)
+    if m * n >= 100:
+        forced = torch.empty((m, n, 3), device="cuda")
+        L.dcsky_device(a.data_ptr(), b.data_ptr(), forced.data_ptr(), m, k, n, 4 if k <= 160 else 3)
+        assert torch.equal(c[:m], forced) == split
     for ch in range(3):
         ref = a[:, :, ch].double().contiguous() @ b[:, :, ch].double().contiguous()
         rel = ((c[:m, :, ch].double() - ref) / ref).abs().max().item()
@@ -721,6 +732,43 @@ def test_tracked_modifiers_belong_to_the_call_and_the_scene(L):
     ctxs[0].set_params(p)
     for got, want in zip(L.contrib_batch(ctxs, sens, mods(names), 1, L.RT_IMM_IRRAD), single):
         assert np.array_equal(got.reshape(want.shape), want)
+
+
+@pytest.mark.parametrize("shape", [dict(), dict(window=1 << 10), dict(window=1 << 12, inflight=2),
+                                   dict(inflight=2)])
+def test_batch_of_rooms_with_and_without_room_sized_primitives(L, shape):
+    """Rooms whose walls are tested ahead of the walk, one whose walls all lie
+    in its tree and one of a single triangle pair, in one call: every record is
+    that of the room alone, bit for bit, whichever windows its rays share and
+    whether one or two of them are under way."""
+    _say(f"batch of rooms with and without room-sized primitives, {shape}")
+    rng = np.random.default_rng(12)
+    room = scenes.Room()
+    walls = scenes.room_rad(room) + scenes.furniture_rad(rng, 3, room) + scenes.sky_rad((1, 1, 1), ground=(1, 1, 1))
+    bare = ("void plastic grey 0 0 5 .5 .5 .5 0 0\ngrey polygon a 0 0 9 0 0 2 4 0 2 0 4 2\n"
+            "grey polygon b 0 0 9 0 0 1 4 0 1 0 4 1.5\n" + scenes.sky_rad((1, 1, 1), ground=(1, 1, 1)))
+    ctxs, sens = [], []
+    for text, big, n in ((walls, 8, 40), (walls, 0, 33), (bare, 0, 7), (walls, 8, 65)):
+        c = L.Context(0)
+        c.load_text(text)
+        c.set_tuning(max_big=big)
+        c.commit()
+        ctxs.append(c)
+        sens.append(np.hstack([rng.uniform(.5, 3.5, (n, 2)), np.full((n, 1), .8), np.tile([0., 0., 1.], (n, 1))]))
+    p = _rc_params(L, ambounce=3, ambdiv=128, minweight=1e-3, seed=9)
+    single = []
+    for k, (c, s) in enumerate(zip(ctxs, sens)):
+        p.seed = 9 + k
+        c.set_params(p)
+        single.append(c.contrib(s, _sky_mods(L), 1, L.RT_IMM_IRRAD))
+        assert single[-1].any()
+    p.seed = 9
+    ctxs[0].set_params(p)
+    ctxs[0].set_tuning(**shape)
+    got = L.contrib_batch(ctxs, sens, _sky_mods(L), 1, L.RT_IMM_IRRAD)
+    assert ctxs[0].last_stats()["wide"]
+    for k, (a, b) in enumerate(zip(got, single)):
+        assert np.array_equal(a, b), k
 
 
 def test_rays_that_are_not_numbers_meet_nothing_in_either_tree(L):
