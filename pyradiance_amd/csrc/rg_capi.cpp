@@ -84,13 +84,6 @@ static void hipck(hipError_t e, const char* w) {
   if (e != hipSuccess) throw std::runtime_error(std::string(w) + ": " + hipGetErrorString(e));
 }
 
-template <class T>
-static T* upload(DevArena& a, const std::string& name, const std::vector<T>& v, hipStream_t st) {
-  T* p = (T*)a.get(name, sizeof(T) * std::max<size_t>(v.size(), 1), st, false);
-  if (!v.empty()) hipck(hipMemcpyAsync(p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice, st), "upload");
-  return p;
-}
-
 // The context's pinned staging buffer, at least `bytes` long.  Every call
 // ends with its stream synchronised, so no transfer uses it when it grows.
 static char* stage_buf(rg_ctx* c, size_t bytes) {
@@ -961,7 +954,7 @@ int rg_last_stats(rg_ctx* c, double* out, int n) {
   RG_TRY(c, {
     static_assert(sizeof(BVHNode) == sizeof(BVH4Q), "one size of node");
     double v[11] = {(double)c->last_nrays, (double)c->last_stats.launches, (double)c->last_stats.threads,
-                   c->last_stats.bounce_ms, (double)c->last_visits[0], (double)c->last_visits[1],
+                   c->last_stats.bounce_ms, (double)c->last_visits[0], (double)(c->last_visits[1] + c->last_visits[2]),
                    (double)c->last_stats.generations, c->last_stats.shade_ms, (double)sizeof(BVHNode),
                    c->last_stats.wide ? 1.0 : 0.0, (double)c->last_visits[2]};
     for (int i = 0; i < n && i < 11; ++i) out[i] = v[i];

@@ -1699,10 +1699,7 @@ __global__ void __launch_bounds__(TBLOCK) k_big_first(DevScene Sarg, RunCfg c, c
   o.prim = h.prim;
   o.front = h.rod > 0.0;
   outp[blockIdx.x * kChunk + threadIdx.x] = o;
-  if (c.visits) {
-    atomicAdd(c.visits + 1, (unsigned long long)nprim);
-    atomicAdd(c.visits + 2, (unsigned long long)nprim);
-  }
+  if (c.visits) atomicAdd(c.visits + 2, (unsigned long long)nprim);
 }
 
 // Persistent four-wide walk (rays handed out as in k_trace_pf; their first

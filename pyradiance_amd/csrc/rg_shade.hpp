@@ -163,8 +163,8 @@ struct RunCfg {
   double* out;         // [nsensor][ncols]
   double fix;          // > 0: deposits add up as int64 multiples of 1 / fix in `out` (order-independent,
                        // so results repeat bit for bit); 0: FP64 atomics
-  unsigned long long* visits;  // optional: [0] BVH nodes visited, [1] primitives tested, [2] of these ahead of
-                               // the four-wide walk
+  unsigned long long* visits;  // optional: [0] BVH nodes visited, [1] primitives tested, [2] and ahead of the
+                               // four-wide walk
   uint32_t* err;       // error flags
   // adjoint replay (adj != 0): instead of writing `out`, each binned
   // deposit adds d(loss)/d(material parameter) into grad
