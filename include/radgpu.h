@@ -213,11 +213,13 @@ int rg_last_stats(rg_ctx *ctx, double *out, int n);
  * one FP32 launch, larger ones BF16 hi/lo split MFMA (K <= 160: rows of A
  * held in registers, sky columns streamed through LDS; longer K: 128 x 128
  * tiles over a ring of LDS buffers, K shared by several blocks when there are
- * few tiles), 2 / 3 / 4 = the split product forced to per-wavefront loads / the ring of
- * LDS buffers / the short-K form (K <= 160).  The split planes (and a shared
- * K's partial products) live in a buffer kept per device and stream, grown
- * as needed and held until the process ends (2 * 3 * (M + N) * K * 2 bytes,
- * with K rounded up to 32 and, for the ring, M and N to 128). */
+ * few tiles), 2 / 3 / 4 = the split product forced to per-wavefront loads / the
+ * ring of LDS buffers / the short-K form (K <= 160).  The split planes live in
+ * a buffer kept per device and stream, grown as needed and held until the
+ * process ends: 12 * (M + N) * K bytes with K rounded up to 32 and, except in
+ * mode 2, M and N to 128; behind them the partial products of a shared K,
+ * 12 * M * N bytes for each of min(CUs / tiles, K / 128) parts if these are
+ * more than one. */
 int rg_dcsky(const float *A, const float *B, float *C, int M, int K, int N, int mode);
 /* Same with device pointers on the current HIP device. */
 int rg_dcsky_device(const float *A, const float *B, float *C, int M, int K, int N, int mode);
@@ -277,10 +279,10 @@ int rg_sky_matrix_device(rg_sky *s, float *dev_out);
  * graph capture, serving loops, harnesses that forbid hipMalloc).  The
  * step tables, patch tables and luminance plane the kernels use live in a
  * fixed 96 MiB device array that each GPU holds until the process ends
- * (Reinhart MF:4 over 8,760 steps fits, -A over that does not); a larger
- * plan returns -1 with the message in rg_sky_error(s).  Calls on one GPU
- * share the array and are serialised by the library; the result equals
- * rg_sky_matrix_device's. */
+ * (Reinhart MF:4 over 8,760 steps fits; -A over that, counted with the
+ * whole matrix, does not); a larger plan returns -1 with the message in
+ * rg_sky_error(s).  Calls on one GPU share the array and are serialised by the
+ * library; the result equals rg_sky_matrix_device's. */
 int rg_sky_matrix_device_noalloc(rg_sky *s, float *dev_out);
 
 /* ASCII records on the host cores: nrecords records of per_record values,

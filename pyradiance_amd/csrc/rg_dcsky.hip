@@ -203,10 +203,10 @@ __global__ void __launch_bounds__(DB) k_dcsky_mfma(const unsigned short* Ah, con
 // plane is 8 KB in one piece, so a load instruction fetches eight whole cache
 // lines.  (From row-major planes it fetched sixteen half lines, and the
 // texture unit, 61 cycles per instruction, was busy 80 % of the time.)
-// 20000 x 2306 x 8760: 6.9 ms, 1.05 PFLOP/s issued, where 128 x 128 tiles of
-// 32 x 32 per wavefront staged through registers took 10.5 ms; matrix cores
-// busy 54 % of the cycles, at a clock that falls to 1.9 GHz.  The
-// 16-byte parts of a row sit at part ^ ((row >> 1) & 3): the eight lanes that
+// 20000 x 2306 x 8760: 6.5 ms (6.7 to 6.8 with the split), 1.12 PFLOP/s issued,
+// where 128 x 128 tiles of 32 x 32 per wavefront staged through registers took
+// 10.5 ms; matrix cores busy 54 % of the cycles, at a clock that falls to
+// 1.9 GHz.  The 16-byte parts of a row sit at part ^ ((row >> 1) & 3): the eight lanes that
 // read LDS together (same part, consecutive rows of 64 bytes) then cover
 // eight different 16-byte columns of the banks.
 constexpr int LBM = 128, LBN = 128;
@@ -443,7 +443,7 @@ static int ring_parts(long long tiles, int nk) {
 // Outputs go through LDS: a lane ends up with 12 consecutive floats of a row,
 // and storing those as they are writes 16 bytes every 48, three times as many
 // partial lines as the rows have.  Turned in LDS, a store instruction covers
-// runs of 192 bytes.  2500 x 146 x 8760: 88 us (104 with 48-byte runs and the
+// runs of 192 bytes.  2500 x 146 x 8760: 84 to 90 us (104 with 48-byte runs and the
 // chunk staged through registers), 3.0 of the 6.9 TB/s that a plain fill
 // reaches; what is left is the wait for the next chunk's loads, which complete
 // in order behind the stores of the chunk before (the compiler does not tell

@@ -1,8 +1,9 @@
 // Wavefront renderer for the rtrace / rcontrib ray tree on CDNA4 (gfx950).
 //
 // The tree is walked breadth-first in windows.  A window's rays are traced to
-// their closest hits (k_trace_pf) and shaded (k_shade); shading appends the
-// next generation: single rays, already built and admitted by the rules of
+// their closest hits (k_big_first and k_walk4; k_trace_pf where only the
+// binary tree serves) and shaded (k_shade); shading appends the next
+// generation: single rays, already built and admitted by the rules of
 // rayorigin() (rt/raytrace.c:40-135), and hemisphere records, whose children
 // k_hemi_rays builds when their turn comes.  Emission is added into the
 // sensor's output with integer or FP64 atomics.  The walk's stack lives in
@@ -14,8 +15,9 @@
 // wavefront: with one spawn counter k_shade took 14.3 ms for the 1.3 M
 // wavefronts of a 2,500-sensor pass, 14.9 ms of it queueing there.  Rays are
 // therefore appended to kRaySegs segments with a counter each (a block's
-// segment is its index modulo their number), and every other per-wavefront
-// counter is kept in registers or taken in large bites.
+// segment is its index modulo their number), k_window_done adds up the ray
+// counts, and work is taken in large bites.  Hemispheres keep one list: a
+// wavefront that appends any bumps its counter and the sum of children once.
 #include <hip/hip_runtime.h>
 #include "rg_shade.hpp"
 #include "rg_render.hpp"
